@@ -10,7 +10,8 @@
 // computes exactly that product.
 //
 // Shape of the computation (one work group per 256 x 256 tile of y, four
-// waves, each wave a 128 x 128 quarter):
+// waves, each wave a 128 x 128 quarter; calls too small to give the CUs such
+// tiles take smaller ones, fp8_gemm_small below):
 // - Both operands are K-major: xq [M, K] and wq [N, K] as dan stores them
 //   (the weight is never transposed), either as byte rows at a stride or in
 //   the tiled layout of include/dan_fp8.h, where each 256-row panel's 64-byte
@@ -748,6 +749,268 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(1, 1))
   wait_vm<0>();
 }
 
+// ---------------------------------------------------------------------------
+// Small tiles (TM x TN, 32 x 32 to 256 x 128), for calls that 256 x 256 tiles
+// would spread over few of the CUs (77 x 4096 outputs: 16 of 256). The
+// instruction, the k order and the epilogue's arithmetic are
+// fp8_gemm_kernel's, so an output has the same bits whatever its tile.
+//
+// Four waves; the tile's 32 x 32 blocks of y go to them as a GM x GN grid,
+// FM x FN blocks each. A 32 x 32 or 64 x 32 tile has one or two computing
+// waves, and the others only load: with one work group per CU a step is bound
+// by its direct loads (about 30 cycles a KB) and its barrier, not by products.
+//
+// A stage is KS k-steps of the tile: per k-step TN / 16 blocks of w, then for
+// all k-steps the x blocks; each wave issues LW of the w and LX of the x
+// blocks. NST stages make the ring, and a step waits for the next stage with
+// a constant count: past the last k-step the loads read out of range (zeros),
+// so every step issues the same number. What made the step fast, at
+// 200 x 4096 x 14336 on 64 x 64 tiles: fragments read a step ahead (32 -> 24 us),
+// and at 1037 x 4096 x 14336 on 128 x 128: no tests and no resource rebuilt on
+// the loads of stages that lie whole inside K, and the products issued before
+// the loads (94 -> 86 us).
+template <int TM, int TN, int KS, int NST, int GM_>
+struct SmallTile {
+  static constexpr int xBlocks = TM / 16 * KS, wBlocks = TN / 16 * KS;  // 1 KB blocks per stage
+  static constexpr int LX = xBlocks / 4, LW = wBlocks / 4;              // of which each wave loads
+  static constexpr int stage = (xBlocks + wBlocks) * 1024;
+  static constexpr int lds = NST * stage;
+  static constexpr int GM = GM_, GN = TN / 32 < 4 / GM ? TN / 32 : 4 / GM;
+  static constexpr int FM = TM / 32 / GM, FN = TN / 32 / GN;
+  static_assert(xBlocks % 4 == 0 && wBlocks % 4 == 0, "the waves load equal shares");
+  static_assert((NST - 1) * (LX + LW) < 64, "vmcnt is 6 bits");
+  static_assert(lds <= 160 * 1024, "LDS");
+  static_assert(TM % (32 * GM) == 0 && TN % (32 * GN) == 0 && TM <= 256 && TN <= 256, "whole blocks per wave");
+};
+
+template <typename TOut, int TM, int TN, int KS, int NST, int GM>
+__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(SmallTile<TM, TN, KS, NST, GM>::lds <= 80 * 1024 ? 2 : 1)))
+void fp8_gemm_small(Params p) {
+  using S = SmallTile<TM, TN, KS, NST, GM>;
+  constexpr int FM = S::FM, FN = S::FN;
+  extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
+  const int lane = threadIdx.x & 63;
+  const int wave = uniform(threadIdx.x >> 6);
+  const uint32_t lds_base = (uint32_t)(uintptr_t)smem;
+
+  // work group -> tile: XCD-contiguous ranges, then groups of tile rows, so
+  // that the tiles of one w panel run on one XCD and share it in its L2
+  const int tiles = p.tiles_m * p.tiles_n;
+  const int id = blockIdx.x, xcd = id & 7;
+  const int t = xcd * (tiles >> 3) + min(xcd, tiles & 7) + (id >> 3);
+  const int group = max(1, kGroupM * kTile / TM);  // tile rows walked together: the rows of kGroupM large tiles
+  const int per_group = group * p.tiles_n;
+  const int first_m = (t / per_group) * group;
+  const int group_m = min(p.tiles_m - first_m, group);
+  const int in_group = t % per_group;
+  const int m0 = (first_m + in_group % group_m) * TM;
+  const int n0 = (in_group / group_m) * TN;
+
+  // the wave's blocks of the tile, and the epilogue's operands of its lanes
+  // (fetched now: their latency passes under the main loop)
+  const int wm = wave % S::GM, wn = wave / S::GM;
+  const bool computes = wn < S::GN;
+  const int fr = lane & 31, h = lane >> 5;
+  const TOut *bias = static_cast<const TOut *>(p.bias);
+  float xsv[FM];
+  f32x4 wsv[FN][4];
+  typedef TOut o4 __attribute__((ext_vector_type(4)));
+  o4 bv[FN][4];
+  auto col = [&](int a, int g) __attribute__((always_inline)) { return n0 + 32 * (FN * wn + a) + 8 * g + 4 * h; };
+#pragma unroll
+  for (int b = 0; b < FM; ++b) xsv[b] = p.xs[(int64_t)min(m0 + 32 * (FM * wm + b) + fr, p.m - 1) * p.xs_inc];
+#pragma unroll
+  for (int a = 0; a < FN; ++a)
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      const int c = min(col(a, g), p.n - 4);
+      if (p.ws_inc) wsv[a][g] = *(const DAN_GLOBAL f32x4 *)(p.ws + c);
+      else {
+        const float ws = *(const DAN_GLOBAL float *)p.ws;
+        wsv[a][g] = f32x4{ws, ws, ws, ws};
+      }
+      if (bias) bv[a][g] = *(const DAN_GLOBAL o4 *)(bias + c);
+    }
+
+  // Direct loads. Block j of an operand's stage share (j = 0 .. blocks - 1,
+  // k-step major) sits at byte 1024 j of it; the wave takes j = LW wave + i.
+  const int rl = lane >> 2;
+  const int chunk = (lane & 3) ^ swz(rl);
+  const int kt = (p.k + kBK - 1) / kBK;
+  struct Loads {
+    i32x4 rsrc;
+    uint32_t vbase, kstep;  // lane offset; bytes per k-step
+    bool tiled;
+  };
+  auto loads_of = [&](bool w) __attribute__((always_inline)) {
+    const int row0 = w ? n0 : m0, total = w ? p.n : p.m;
+    Loads l;
+    l.tiled = w ? p.w_tiled : p.x_tiled;
+    const uint8_t *ptr = w ? p.w : p.x;
+    if (l.tiled) {  // the tile's panel and, where the tile crosses into it, the next (zeros past the last)
+      const int panel = row0 / kTile, panels = min(2, (total + kTile - 1) / kTile - panel);
+      l.rsrc = resource(ptr + (int64_t)panel * kt * 16384, (uint32_t)(panels * kt) * 16384u);
+      l.vbase = 16 * lane;
+      l.kstep = 16384;
+    } else {
+      const int64_t st = w ? p.w_st : p.x_st;
+      l.rsrc = resource(ptr + (int64_t)row0 * st, (uint32_t)(min(w ? TN : TM, total - row0) * st));
+      l.vbase = (uint32_t)(rl * st + 16 * chunk);
+      l.kstep = kBK;
+    }
+    return l;
+  };
+  const Loads lw = loads_of(true), lx = loads_of(false);
+  constexpr int kLoads = S::LW + S::LX;
+  // Load i of the wave: block j of its operand's share, which lies in k-step
+  // ks of the stage; its lane's offset from the stage's first byte.
+  auto block_of = [&](int i) __attribute__((always_inline)) { return i < S::LW ? wave * S::LW + i : wave * S::LX + i - S::LW; };
+  auto kstep_of = [&](int i) __attribute__((always_inline)) { return block_of(i) / (i < S::LW ? TN / 16 : TM / 16); };
+  uint32_t voff[kLoads];
+#pragma unroll
+  for (int i = 0; i < kLoads; ++i) {
+    const bool w = i < S::LW;
+    const int ks = kstep_of(i), blk = block_of(i) % (w ? TN / 16 : TM / 16);
+    if (w ? lw.tiled : lx.tiled) {
+      const int b = (w ? n0 : m0) % kTile / 16 + blk;  // 16-row block counted from the panel's start
+      voff[i] = (uint32_t)((b / 16 * kt + ks) * 16384 + b % 16 * 1024) + (w ? lw.vbase : lx.vbase);
+    } else {
+      voff[i] = (uint32_t)(16 * blk * (w ? p.w_st : p.x_st)) + (uint32_t)(ks * kBK) + (w ? lw.vbase : lx.vbase);
+    }
+  }
+  // LDS byte (in its stage) of the wave's load i.
+  auto ldst = [&](int i) __attribute__((always_inline)) { return (uint32_t)(i < S::LW ? wave * S::LW + i : S::wBlocks + wave * S::LX + i - S::LW) * 1024; };
+  auto advanced = [](i32x4 r, uint32_t by) __attribute__((always_inline)) {
+    const uint64_t b = ((uint64_t)(uint32_t)r[0] | ((uint64_t)(uint32_t)(r[1] & 0xffff) << 32)) + by;
+    r[0] = (int32_t)(uint32_t)b;
+    r[1] = (int32_t)((uint32_t)(b >> 32) & 0xffff);
+    r[2] = (int32_t)((uint32_t)r[2] - by);
+    return r;
+  };
+  // The direct loads of a stage that lies whole inside K: nothing to test, and
+  // the resources (rw, rx: from the next stage to load on) step along.
+  i32x4 rw = lw.rsrc, rx = lx.rsrc;
+  auto load_full = [&](int i, uint32_t stage) __attribute__((always_inline)) { dma16(i < S::LW ? rw : rx, voff[i], stage + ldst(i)); };
+  auto step_full = [&]() __attribute__((always_inline)) {
+    rw = advanced(rw, KS * lw.kstep);
+    rx = advanced(rx, KS * lx.kstep);
+  };
+  // The same for any stage s: k past K (the rest of a row-major row, the k-steps
+  // past the last) reads out of range, and so does every load past the last stage.
+  auto load_any = [&](int i, int s, uint32_t stage) __attribute__((always_inline)) {
+    const Loads &l = i < S::LW ? lw : lx;
+    const int k0 = (s * KS + kstep_of(i)) * kBK;
+    uint32_t off = voff[i];
+    if (k0 + (l.tiled ? 0 : 16 * chunk) >= p.k) off = kOutOfRange;
+    i32x4 r = l.rsrc;
+    if (s * KS < kt) r = advanced(r, (uint32_t)s * (KS * l.kstep));
+    dma16(r, off, stage + ldst(i));
+  };
+
+  const uint32_t f_lo = fr * kBK + 16 * ((2 * h) ^ swz(fr)), f_hi = fr * kBK + 16 * ((2 * h + 1) ^ swz(fr));
+  auto read_frag = [&](uint32_t blk) __attribute__((always_inline)) {
+    const u32x4 lo = *(const DAN_LDS u32x4 *)(uintptr_t)(blk + f_lo);
+    const u32x4 hi = *(const DAN_LDS u32x4 *)(uintptr_t)(blk + f_hi);
+    return __builtin_bit_cast(i32x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+  };
+
+  f32x16 acc[FN][FM];
+#pragma unroll
+  for (int a = 0; a < FN; ++a)
+#pragma unroll
+    for (int b = 0; b < FM; ++b) acc[a][b] = (f32x16){};
+
+  // One step: the products of stage s on `cur`, whose reads were issued a step
+  // ago; between them the fragment reads of stage s + 1 (into `nxt`) and the
+  // direct loads of stage s + NST (into the buffer of stage s): a wave issues
+  // in order, and a load queued at the CU's address unit holds back whatever
+  // follows it, so the products go first.
+  struct F {
+    i32x8 w[KS][FN], x[KS][FM];
+  };
+  constexpr int kProducts = KS * FN * FM, kReads = KS * (FN + FM);
+  auto read_one = [&](F &f, uint32_t stage, int i) __attribute__((always_inline)) {
+    const uint32_t wr = stage + (uint32_t)(FN * wn) * 2048, xr = stage + (uint32_t)S::wBlocks * 1024 + (uint32_t)(FM * wm) * 2048;
+    const int ks = i / (FN + FM), j = i % (FN + FM);
+    if (j < FN) f.w[ks][j] = read_frag(wr + (uint32_t)(ks * (TN / 16) + 2 * j) * 1024);
+    else f.x[ks][j - FN] = read_frag(xr + (uint32_t)(ks * (TM / 16) + 2 * (j - FN)) * 1024);
+  };
+  uint32_t here = lds_base, next = lds_base + S::stage;  // the buffers of stages s and s + 1
+  auto step = [&](auto full, int s, F &cur, F &nxt) __attribute__((always_inline)) {
+    constexpr bool kFull = decltype(full)::value;
+    wait_vm<(NST - 2) * kLoads>();  // stage s + 1 landed; the NST - 2 after it may be in flight
+    barrier_lds();                  // for every wave, and every wave has read stage s: its buffer is free
+    auto ld = [&](int i) __attribute__((always_inline)) {
+      if (kFull) load_full(i, here);
+      else load_any(i, s + NST, here);
+    };
+    if (computes) {  // (past the last stage the reads give zeros that nothing uses)
+#pragma unroll
+      for (int i = 0; i < kProducts; ++i) {
+        const int ks = i / (FN * FM), a = i / FM % FN, b = i % FM;
+        acc[a][b] = mfma(cur.w[ks][a], cur.x[ks][b], acc[a][b]);
+#pragma unroll
+        for (int r = i * kReads / kProducts; r < (i + 1) * kReads / kProducts; ++r) read_one(nxt, next, r);
+#pragma unroll
+        for (int l = i * kLoads / kProducts; l < (i + 1) * kLoads / kProducts; ++l) ld(l);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    } else {
+#pragma unroll
+      for (int l = 0; l < kLoads; ++l) ld(l);
+    }
+    if (kFull) step_full();
+    here = next;
+    next = next + S::stage == lds_base + S::lds ? lds_base : next + S::stage;
+  };
+  const int steps = (kt + KS - 1) / KS, whole = p.k / (KS * kBK);  // stages; of which inside K
+#pragma unroll
+  for (int s = 0; s < NST; ++s)
+#pragma unroll
+    for (int l = 0; l < kLoads; ++l) load_any(l, s, lds_base + s * S::stage);
+  wait_vm<(NST - 1) * kLoads>();
+  barrier_lds();
+  F f0, f1;
+  if (computes) {
+#pragma unroll
+    for (int r = 0; r < kReads; ++r) read_one(f0, lds_base, r);
+  }
+  const std::integral_constant<bool, true> full;
+  const std::integral_constant<bool, false> any;
+  int s = 0;
+  if (NST + 1 < whole) {
+    rw = advanced(rw, (uint32_t)NST * (KS * lw.kstep));
+    rx = advanced(rx, (uint32_t)NST * (KS * lx.kstep));
+    for (; s + NST + 1 < whole; s += 2) {
+      step(full, s, f0, f1);
+      step(full, s + 1, f1, f0);
+    }
+  }
+  for (; s + 1 < steps; s += 2) {
+    step(any, s, f0, f1);
+    step(any, s + 1, f1, f0);
+  }
+  if (s < steps) step(any, s, f0, f1);
+  wait_vm<0>();  // no direct load may land after the work group's LDS is given back
+
+  if (!computes) return;
+  TOut *y = static_cast<TOut *>(p.y);
+#pragma unroll
+  for (int b = 0; b < FM; ++b) {
+    const int row = m0 + 32 * (FM * wm + b) + fr;
+#pragma unroll
+    for (int a = 0; a < FN; ++a)
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        const int c = col(a, g);
+        f32x4 v;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[i] = __builtin_fmaf(acc[a][b][4 * g + i] * xsv[b], wsv[a][g][i], bias ? (float)bv[a][g][i] : 0.0f);
+        if (row < p.m && c < p.n) Out<TOut>::store4(y + (int64_t)row * p.y_st + c, v);
+      }
+  }
+}
+
 template <typename TOut, bool kTail>
 hipError_t launch(const Params &p, hipStream_t s) {
   auto kernel = fp8_gemm_kernel<TOut, kTail>;
@@ -780,9 +1043,43 @@ int num_cus() {  // of the current device, cached per device
   return cached[dev];
 }
 
+template <typename TOut, int TM, int TN, int KS, int NST, int GM>
+hipError_t launch_small(Params p, hipStream_t s) {
+  p.tiles_m = (p.m + TM - 1) / TM;
+  p.tiles_n = (p.n + TN - 1) / TN;
+  auto kernel = fp8_gemm_small<TOut, TM, TN, KS, NST, GM>;
+  constexpr int lds = SmallTile<TM, TN, KS, NST, GM>::lds;
+  static const hipError_t attr =
+      hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+  if (attr != hipSuccess) return attr;
+  hipLaunchKernelGGL(kernel, dim3(p.tiles_m * p.tiles_n), dim3(kThreads), lds, s, p);
+  return hipGetLastError();
+}
+
 template <typename TOut>
 hipError_t launch(const Params &p, hipStream_t s) {
   const int kt = (p.k + kBK - 1) / kBK, tiles = p.tiles_m * p.tiles_n, cus = num_cus();
+  // The smallest of these tiles that gives every CU at most one; 256 x 256
+  // tiles where even 256 x 128 ones are more than the CUs. A CU's time grows
+  // with its tile, and a second round doubles it. Over 190 sizes (m 1 to 8192;
+  // n x k 4096 x 4096, 6144 x 4096, 4096 x 14336, 28672 x 4096, 2048 x 2048,
+  // 1040 x 6000, 8192 x 8192; tiled operands) this choice is on average 0.6 %
+  // and at most 13 % behind the best tile of each size. us, 256 x 256 tiles -> this choice:
+  //   n 4096 k 4096   m 77: 38.6 -> 9.0    m 512: 38.9 -> 15   m 1037: 39 -> 25   m 2048: 42 -> 38
+  //   n 4096 k 14336  m 77: 112 -> 20      m 512: 113 -> 39    m 1037: 114 -> 64  m 2048: 125 -> 100
+  //   n 28672 k 4096  m 1: 48 -> 24        m 77: 48 -> 31      m 200: 50 -> 41    m 512: 256 x 256
+  // (Two panels of a tiled operand must span less than 2 GiB: kOutOfRange lies past them.)
+  auto one_each = [&](int tm, int tn) { return (int64_t)((p.m + tm - 1) / tm) * ((p.n + tn - 1) / tn) <= cus; };
+  if ((int64_t)2 * kt * 16384 < ((int64_t)1 << 31)) {
+    if (one_each(32, 32)) return launch_small<TOut, 32, 32, 4, 4, 1>(p, s);
+    if (one_each(64, 32)) return launch_small<TOut, 64, 32, 4, 3, 2>(p, s);
+    if (one_each(64, 64)) return launch_small<TOut, 64, 64, 2, 4, 2>(p, s);
+    if (one_each(64, 128)) return launch_small<TOut, 64, 128, 2, 3, 1>(p, s);
+    if (one_each(128, 128)) return launch_small<TOut, 128, 128, 2, 4, 2>(p, s);
+    if (one_each(160, 128)) return launch_small<TOut, 160, 128, 2, 4, 1>(p, s);
+    if (one_each(192, 128)) return launch_small<TOut, 192, 128, 2, 4, 2>(p, s);
+    if (one_each(256, 128)) return launch_small<TOut, 256, 128, 2, 3, 1>(p, s);
+  }
   // The persistent form: 16-bit outputs, an even number of k-steps >= 6, and
   // 256 output rows spanning less than 2 GiB (its stores use a buffer resource).
   if constexpr (sizeof(TOut) == 2) {
