@@ -134,7 +134,7 @@ class DanFp8GemmArgs(ctypes.Structure):
                 ("w_scale", _vp), ("bias", _vp), ("y", _vp), ("y_stride", _i64)]
 
 
-GDN_ABI_VERSION = 4
+GDN_ABI_VERSION = 5
 GDN_FORM_TOKEN, GDN_FORM_CHUNK = 0, 1
 GDN_CHUNK = 64
 
@@ -160,11 +160,17 @@ class DanGdnConvArgs(ctypes.Structure):
                 ("beta", _vp), ("g", _vp)]
 
 
+class DanGdnNormArgs(ctypes.Structure):
+    _fields_ = [("abi_version", _i32), ("dtype", _i32), ("num_tokens", _i32), ("num_v_heads", _i32), ("v_dim", _i32),
+                ("eps", _f32), ("x", _vp), ("x_stride", _i64), ("gate", _vp), ("gate_stride", _i64), ("weight", _vp),
+                ("out", _vp), ("out_stride", _i64)]
+
+
 EXPORTS = ("dan_tree_attn_fwd", "dan_tree_attn_fwd_noalloc", "dan_tree_attn_stage_f16", "dan_tree_attn_tile_q", "dan_tree_attn_head_groups", "dan_tree_attn_workspace_size",
            "dan_tree_attn_last_error", "dan_tree_attn_abi_version", "dan_qkv_front", "dan_qkv_front_abi_version",
            "dan_tree_attn_plan", "dan_tree_attn_plan_slots", "dan_tree_attn_plan_abi_version",
            "dan_fp8_quantize", "dan_fp8_gemm", "dan_fp8_tiled_bytes", "dan_fp8_abi_version", "dan_gdn_fwd", "dan_gdn_workspace_size", "dan_gdn_abi_version",
-           "dan_gdn_conv")
+           "dan_gdn_conv", "dan_gdn_gated_norm")
 
 _lock = threading.Lock()
 _lib = None
@@ -222,6 +228,8 @@ def load(path=LIB_PATH):
         lib.dan_gdn_workspace_size.restype = _i64
         lib.dan_gdn_conv.argtypes = [ctypes.POINTER(DanGdnConvArgs), _vp]
         lib.dan_gdn_conv.restype = ctypes.c_int
+        lib.dan_gdn_gated_norm.argtypes = [ctypes.POINTER(DanGdnNormArgs), _vp]
+        lib.dan_gdn_gated_norm.restype = ctypes.c_int
         lib.dan_gdn_abi_version.argtypes = []
         lib.dan_gdn_abi_version.restype = ctypes.c_int
         got = (lib.dan_tree_attn_abi_version(), lib.dan_qkv_front_abi_version(), lib.dan_tree_attn_plan_abi_version(),
@@ -336,3 +344,11 @@ def gdn_conv(args, stream, lib=None):
     rc = lib.dan_gdn_conv(ctypes.byref(args), _vp(stream))
     if rc != OK:
         raise RuntimeError(f"dan_gdn_conv failed ({rc}): {last_error(lib)}")
+
+
+def gdn_gated_norm(args, stream, lib=None):
+    """Launch the gated RMS norm of a DeltaNet layer; raises RuntimeError with the library's message on failure."""
+    lib = lib or load()
+    rc = lib.dan_gdn_gated_norm(ctypes.byref(args), _vp(stream))
+    if rc != OK:
+        raise RuntimeError(f"dan_gdn_gated_norm failed ({rc}): {last_error(lib)}")

@@ -129,6 +129,29 @@ def gated_rms_norm(x, gate, weight, eps):
     return (y * torch.nn.functional.silu(gate.float())).to(x.dtype)
 
 
+def _gated_norm(out, z, weight, eps):
+    """``gated_rms_norm`` of every (token, head) row of out [N, Hv, Dv] with
+    the gate z [N, Hv * Dv], as [N, Hv * Dv]: one ``dan_gdn_gated_norm``
+    launch where its layout and types allow and no gradient is wanted, else
+    the eager ops (both round at the same places)."""
+    n, hv, dv = out.shape
+    grad = torch.is_grad_enabled() and any(t.requires_grad for t in (out, z, weight))
+    if (grad or torch.compiler.is_compiling() or dv not in (32, 64, 128, 256) or out.dtype not in (torch.bfloat16, torch.float16)
+            or not (z.dtype == weight.dtype == out.dtype) or not out.is_contiguous() or z.stride(1) != 1
+            or z.stride(0) % 8 or z.stride(0) < hv * dv or not weight.is_contiguous()
+            or any(t.data_ptr() % 16 for t in (out, z, weight)) or not 0 <= eps < float("inf")):
+        return gated_rms_norm(out.reshape(-1, dv), z.reshape(-1, dv), weight, eps).reshape(n, hv * dv)
+    y = torch.empty((n, hv * dv), dtype=out.dtype, device=out.device)
+    a = _native.DanGdnNormArgs()
+    a.abi_version = _native.GDN_ABI_VERSION
+    a.dtype = _DTYPES[out.dtype]
+    a.num_tokens, a.num_v_heads, a.v_dim, a.eps = n, hv, dv, eps
+    a.x, a.x_stride, a.gate, a.gate_stride = out.data_ptr(), hv * dv, z.data_ptr(), z.stride(0)
+    a.weight, a.out, a.out_stride = weight.data_ptr(), y.data_ptr(), hv * dv
+    _native.gdn_gated_norm(a, torch.cuda.current_stream(out.device).cuda_stream)
+    return y
+
+
 @dataclass
 class Phase:
     """One batch of runs (dan/models/qwen3_5.py:230-236). Index lists are
@@ -325,8 +348,7 @@ class DeltaNet(nn.Module):
             segments[i].saved[self.index] = (_virtual_rows(qkv, hist, tail), final[i].clone())
         if lay.branches is not None:
             self._phase(lay.branches, qkv, hist, b, a, final_end, out, lay.branch_segment)
-        y = gated_rms_norm(out.reshape(-1, self.dv), z.reshape(-1, self.dv), self.norm.weight, self.eps)
-        return self.out_proj(y.reshape(n, -1))
+        return self.out_proj(_gated_norm(out, z, self.norm.weight, self.eps))
 
     def _phase(self, ph, qkv, hist, b, a, states, out, state_index=None):
         conv, beta, g = conv_phase(qkv, hist, ph, self.conv1d.weight, b, a, self.A_log, self.dt_bias)

@@ -29,7 +29,7 @@
 extern "C" {
 #endif
 
-#define DAN_GDN_ABI_VERSION 4
+#define DAN_GDN_ABI_VERSION 5
 
 /* Tokens per chunk of the chunked form. */
 #define DAN_GDN_CHUNK 64
@@ -137,6 +137,27 @@ typedef struct {
  * concatenation), :216-218 (index_select, conv1d, silu, index_select) and
  * the gathers of g and beta at :223, with dan/fused.py:80-82. */
 int dan_gdn_conv(const DanGdnConvArgs *args, void *stream);
+
+/* The gated RMS norm after the recurrence, dan/fused.py:52-56, per (token,
+ * value head) row of v_dim values:
+ *   out = rnd(weight * rnd(x * rsqrt(mean(x^2) + eps))) * silu(gate)
+ * rnd() rounding to dtype; sums, silu and the last product in fp32, rounded
+ * to dtype at the store. (GDN ABI 5) */
+typedef struct {
+  int32_t abi_version;  /* DAN_GDN_ABI_VERSION */
+  int32_t dtype;        /* DanDtype of x, gate, weight and out: bf16 or f16 */
+  int32_t num_tokens;   /* N */
+  int32_t num_v_heads;  /* Hv */
+  int32_t v_dim;        /* Dv: 32, 64, 128 or 256 */
+  float eps;
+  const void *x; int64_t x_stride;        /* [N, Hv * Dv], token strides in elements: multiples of 8, 16-byte aligned rows */
+  const void *gate; int64_t gate_stride;  /* [N, Hv * Dv] */
+  const void *weight;                     /* [Dv] */
+  void *out; int64_t out_stride;          /* [N, Hv * Dv] */
+} DanGdnNormArgs;
+
+/* Replaces dan/fused.py:52-56 as dan/models/qwen3_5.py:226 calls it. */
+int dan_gdn_gated_norm(const DanGdnNormArgs *args, void *stream);
 
 int dan_gdn_abi_version(void);
 
