@@ -134,7 +134,7 @@ class DanFp8GemmArgs(ctypes.Structure):
                 ("w_scale", _vp), ("bias", _vp), ("y", _vp), ("y_stride", _i64)]
 
 
-GDN_ABI_VERSION = 5
+GDN_ABI_VERSION = 6
 GDN_FORM_TOKEN, GDN_FORM_CHUNK = 0, 1
 GDN_CHUNK = 64
 
@@ -148,14 +148,14 @@ class DanGdnArgs(ctypes.Structure):
                 ("g", _vp), ("beta", _vp), ("states_in", _vp), ("states_out", _vp),
                 ("out", _vp), ("o_stride_tok", _i64), ("o_stride_head", _i64),
                 ("workspace", _vp), ("workspace_bytes", _i64), ("form", _i32), ("reserved", _i32),
-                ("state_index", _vp), ("num_states_in", _i32), ("reserved2", _i32)]
+                ("state_index", _vp), ("num_states_in", _i32), ("num_out_rows", _i32), ("out_start", _vp)]
 
 
 class DanGdnConvArgs(ctypes.Structure):
     _fields_ = [("abi_version", _i32), ("dtype", _i32), ("channels", _i32), ("kernel", _i32), ("num_rows", _i32),
                 ("num_hist_rows", _i32), ("num_ext", _i32), ("num_out", _i32),
                 ("src", _vp), ("src_stride", _i64), ("hist", _vp), ("ext", _vp), ("take", _vp), ("weight", _vp),
-                ("out", _vp), ("out_stride", _i64), ("num_heads", _i32), ("reserved", _i32), ("rows", _vp),
+                ("out", _vp), ("out_stride", _i64), ("num_heads", _i32), ("gate_dtype", _i32), ("rows", _vp),
                 ("b", _vp), ("b_stride", _i64), ("a", _vp), ("a_stride", _i64), ("a_log", _vp), ("dt_bias", _vp),
                 ("beta", _vp), ("g", _vp)]
 

@@ -92,7 +92,8 @@ struct Params {
   void *o;
   float *norms;  // [N][Hk][2]: 1 / sqrt(sum q^2 + eps), 1 / sqrt(sum k^2 + eps)
   const int32_t *sidx;  // NULL or [R]: run r's entry of s_in (clamped to [0, nsin))
-  int32_t N, Hk, Hv, Dv, R, cblocks, nsin;
+  const int32_t *ostart;  // NULL or [R]: run r's first row of o (o holds orows rows)
+  int32_t N, Hk, Hv, Dv, R, cblocks, nsin, orows;
 };
 
 // One wave per (token, key head): lanes 0-31 hold 4 values of q, 32-63 of k.
@@ -184,6 +185,8 @@ __global__ __launch_bounds__(64 * kWavesPerGroup) void gdn_kernel(const Params p
     gv[2] = nr[0];
     gv[3] = nr[1];
   };
+  int out0 = row0;  // the row of o that the run's first token writes
+  if (p.ostart) out0 = max(0, min(__builtin_amdgcn_readfirstlane(*(const DAN_GLOBAL int32_t *)(p.ostart + r)), p.orows - len));
   T *oh = static_cast<T *>(p.o) + (int64_t)h * p.o_sh + c;
   const float qscale = 0.08838834764831845f;  // Dk^-1/2 (dan/models/qwen3_5.py:110)
 
@@ -225,7 +228,7 @@ __global__ __launch_bounds__(64 * kWavesPerGroup) void gdn_kernel(const Params p
       o1 = fmaf(qv[i + 1], s[i + 1], o1);
     }
     const float o = sum_column(o0 + o1) * (rq * qscale);
-    if (re == 0) *(DAN_GLOBAL T *)(oh + (int64_t)(row0 + t) * p.o_st) = (T)o;
+    if (re == 0) *(DAN_GLOBAL T *)(oh + (int64_t)(out0 + t) * p.o_st) = (T)o;
   };
 
   // Every load below is unconditional, with its token clamped to the run:
@@ -321,6 +324,8 @@ int dan_gdn_fwd(const DanGdnArgs *a, void *stream) {
   if (a->form != DAN_GDN_FORM_TOKEN && a->form != DAN_GDN_FORM_CHUNK) return fail(DAN_ERR_INVALID_ARGUMENT, "form %d", a->form);
   if (a->state_index && a->num_states_in <= 0)
     return fail(DAN_ERR_INVALID_ARGUMENT, "state_index needs num_states_in > 0, got %d", a->num_states_in);
+  if (a->out_start && a->num_out_rows < a->num_tokens)
+    return fail(DAN_ERR_INVALID_ARGUMENT, "out_start needs num_out_rows >= num_tokens, got %d for %d", a->num_out_rows, a->num_tokens);
   if (a->form == DAN_GDN_FORM_CHUNK && a->v_dim % 32)
     return fail(DAN_ERR_UNSUPPORTED, "v_dim %d: the chunked form takes a multiple of 32", a->v_dim);
   const int64_t need =
@@ -350,6 +355,7 @@ int dan_gdn_fwd(const DanGdnArgs *a, void *stream) {
   p.Hk = a->num_k_heads; p.Hv = a->num_v_heads; p.Dv = a->v_dim; p.R = a->num_runs;
   p.cblocks = a->v_dim / dan_gdn::kCols; p.N = a->num_tokens; p.norms = norms;
   p.sidx = a->state_index; p.nsin = a->num_states_in;
+  p.ostart = a->out_start; p.orows = a->num_out_rows;
   hipError_t err = dan_gdn::launch_norms(a, norms, s);
   if (err == hipSuccess) {
     const dim3 block(64 * dan_gdn::kWavesPerGroup);

@@ -86,8 +86,16 @@ struct Params {
   float *s_out, *rec;
   void *o;
   const int32_t *sidx;  // NULL or [R]: run r's entry of s_in (clamped to [0, nsin))
-  int32_t Hk, Hv, Dv, R, ncb, units, nsin;
+  const int32_t *ostart;  // NULL or [R]: run r's first row of o (o holds orows rows)
+  int32_t Hk, Hv, Dv, R, ncb, units, nsin, orows;
 };
+
+// Rows of o minus rows of the inputs for run r of rows [row0, end) (wave-uniform).
+__device__ inline int out_shift(const Params &p, int r, int row0, int end) {
+  if (!p.ostart) return 0;
+  const int first = __builtin_amdgcn_readfirstlane(*(const __attribute__((address_space(1))) int32_t *)(p.ostart + r));
+  return max(0, min(first, p.orows - (end - row0))) - row0;
+}
 
 // Run r's entry of s_in (wave-uniform).
 __device__ inline int state_in_of(const Params &p, int r) {
@@ -463,7 +471,7 @@ __global__ __launch_bounds__(64 * W) void chunk_scan_kernel(const Params p) {
   const T *qh = static_cast<const T *>(p.q) + (int64_t)hk * p.q_sh;
   const T *kh = static_cast<const T *>(p.k) + (int64_t)hk * p.k_sh;
   const T *vh = static_cast<const T *>(p.v) + (int64_t)h * p.v_sh + col0;
-  T *oh = static_cast<T *>(p.o) + (int64_t)h * p.o_sh + col0;
+  T *oh = static_cast<T *>(p.o) + (int64_t)h * p.o_sh + col0 + (int64_t)out_shift(p, r, row0, end) * p.o_st;
   const int ri = 16 * rb + l16;   // the A-operand row of the 64-row products
   const int ro = 16 * rb + 4 * q4;  // the first of the lane's accumulator rows
 
@@ -746,7 +754,7 @@ void chunk_scan_bf16_kernel(const Params p) {
   const __bf16 *qh = static_cast<const __bf16 *>(p.q) + (int64_t)hk * p.q_sh;
   const __bf16 *kh = static_cast<const __bf16 *>(p.k) + (int64_t)hk * p.k_sh;
   const __bf16 *vh = static_cast<const __bf16 *>(p.v) + (int64_t)h * p.v_sh + col0;
-  __bf16 *oh = static_cast<__bf16 *>(p.o) + (int64_t)h * p.o_sh + col0;
+  __bf16 *oh = static_cast<__bf16 *>(p.o) + (int64_t)h * p.o_sh + col0 + (int64_t)out_shift(p, r, row0, end) * p.o_st;
   const int ri = 16 * rb + l16;     // the A-operand row of the 64-row products
   const int ro = 16 * rb + 4 * g4;  // the first of the lane's accumulator rows
 
@@ -949,6 +957,7 @@ hipError_t dan_gdn_fwd_chunked(const DanGdnArgs *a, float *records, hipStream_t 
   p.Hk = a->num_k_heads; p.Hv = a->num_v_heads; p.Dv = a->v_dim; p.R = a->num_runs;
   p.units = a->num_runs * a->num_v_heads;
   p.sidx = a->state_index; p.nsin = a->num_states_in;
+  p.ostart = a->out_start; p.orows = a->num_out_rows;
   const int64_t prep = dan_gdnc::slots(a->num_tokens, a->num_runs) * a->num_v_heads;
   // Runs of DAN_GDN_SHORT_RUN tokens or fewer on average: the short-run scan;
   // longer: the long-run scan.

@@ -68,11 +68,12 @@ __device__ inline u32x4 pack8(f32x8 x) {
 struct Params {
   const void *src, *hist, *weight, *b, *a;
   const int32_t *ext, *take, *rows;
-  const float *a_log, *dt_bias;
+  const void *a_log, *dt_bias;
   void *out;
   float *beta, *g;
   int64_t src_stride, out_stride, b_stride, a_stride;
   int32_t C, N, hist_rows, num_ext, T, Hv, groups;  // groups = C / 8
+  int32_t gate_lp;               // a_log and dt_bias in the I/O type, else fp32
   int32_t cblocks, gate_blocks;  // ceil(groups / 64) waves per strip; work groups of gates
 };
 
@@ -90,12 +91,14 @@ __device__ inline void gates(const Params &p, int64_t gid) {
   const int r = p.rows[i];
   float beta = 0.0f, g = 0.0f;
   if (r >= 0 && r < p.N) {
+    const float al = p.gate_lp ? (float)static_cast<const T *>(p.a_log)[h] : static_cast<const float *>(p.a_log)[h];
+    const float dt = p.gate_lp ? (float)static_cast<const T *>(p.dt_bias)[h] : static_cast<const float *>(p.dt_bias)[h];
     const float bb = (float)static_cast<const T *>(p.b)[(int64_t)r * p.b_stride + h];
     const float aa = (float)static_cast<const T *>(p.a)[(int64_t)r * p.a_stride + h];
     beta = (float)(T)(1.0f / (1.0f + expf(-bb)));
-    const float z = aa + p.dt_bias[h];
+    const float z = aa + dt;
     const float sp = z > 20.0f ? z : log1pf(expf(z));  // softplus, threshold 20
-    g = -expf(p.a_log[h]) * sp;
+    g = -expf(al) * sp;
   }
   p.beta[gid] = beta;
   p.g[gid] = g;
@@ -249,12 +252,14 @@ extern "C" int dan_gdn_conv(const DanGdnConvArgs *a, void *stream) {
   if ((uintptr_t)a->weight & 15) return fail(DAN_ERR_INVALID_ARGUMENT, "weight must be 16-byte aligned");
   if (a->num_heads && (!a->rows || !a->b || !a->a || !a->a_log || !a->dt_bias || !a->beta || !a->g))
     return fail(DAN_ERR_INVALID_ARGUMENT, "NULL gate pointer");
+  if (a->gate_dtype != 0 && a->gate_dtype != 1) return fail(DAN_ERR_INVALID_ARGUMENT, "gate_dtype %d: 0 (fp32) or 1 (dtype)", a->gate_dtype);
   dan_conv::Params p;
   p.src = a->src; p.hist = a->hist; p.weight = a->weight; p.b = a->b; p.a = a->a;
   p.ext = a->ext; p.take = a->take; p.rows = a->rows; p.a_log = a->a_log; p.dt_bias = a->dt_bias;
   p.out = a->out; p.beta = a->beta; p.g = a->g;
   p.src_stride = a->src_stride; p.out_stride = a->out_stride; p.b_stride = a->b_stride; p.a_stride = a->a_stride;
   p.C = a->channels; p.N = a->num_rows; p.hist_rows = a->num_hist_rows; p.num_ext = a->num_ext; p.T = a->num_out;
+  p.gate_lp = a->gate_dtype;
   p.Hv = a->num_heads; p.groups = a->channels / 8;
   p.cblocks = (p.groups + 63) / 64;
   const int64_t waves = (int64_t)(a->num_out + dan_conv::kStrip - 1) / dan_conv::kStrip * p.cblocks;

@@ -51,6 +51,14 @@ def delta_rule(q, k, v, g, beta, lengths, states, cu=None, form=None, state_inde
     32), or None to take "chunk" when the longest run has at least
     CHUNK_MIN_RUN tokens and Dv allows it. Both forms compute the same
     recurrence in fp32."""
+    return _delta_rule(q, k, v, g, beta, lengths, states, cu, form, state_index)
+
+
+def _delta_rule(q, k, v, g, beta, lengths, states, cu=None, form=None, state_index=None, out=None, out_start=None, finals=None):
+    """``delta_rule``; with ``out`` [M, Hv, Dv] and ``out_start`` ([R] int32 on
+    the device) run r's outputs go to rows ``out_start[r]`` .. of ``out``, and
+    ``finals`` [R, Hv, 128, Dv] (contiguous fp32, not overlapping ``states``)
+    takes the final states."""
     if not q.is_cuda:
         raise RuntimeError("dan_amd.deltanet.delta_rule runs on a gfx950 GPU only; got tensors on "
                            f"{q.device} (the CPU forms are the test oracle, not a backend)")
@@ -91,8 +99,12 @@ def delta_rule(q, k, v, g, beta, lengths, states, cu=None, form=None, state_inde
         cu_d = cu_d.pin_memory().to(dev, non_blocking=True)
     else:
         cu_d = cu[0].to(torch.int32)
-    out = torch.empty((n, hv, dv), dtype=q.dtype, device=dev)
-    finals = torch.empty((r, hv, dk, dv), dtype=torch.float32, device=dev)
+    if out is None:
+        out = torch.empty((n, hv, dv), dtype=q.dtype, device=dev)
+    elif out.dtype != q.dtype or out.device != dev or tuple(out.shape[1:]) != (hv, dv):
+        raise ValueError(f"out {tuple(out.shape)} {out.dtype} on {out.device}: want [M, {hv}, {dv}] {q.dtype} on {dev}")
+    if finals is None:
+        finals = torch.empty((r, hv, dk, dv), dtype=torch.float32, device=dev)
     a = _native.DanGdnArgs()
     a.abi_version = _native.GDN_ABI_VERSION
     a.dtype = _DTYPES[q.dtype]
@@ -109,6 +121,8 @@ def delta_rule(q, k, v, g, beta, lengths, states, cu=None, form=None, state_inde
     a.workspace, a.workspace_bytes, a.form = ws.data_ptr(), nbytes, code
     if state_index is not None:
         a.state_index, a.num_states_in = state_index.data_ptr(), s_in.shape[0]
+    if out_start is not None:
+        a.out_start, a.num_out_rows = out_start.data_ptr(), out.shape[0]
     _native.gdn(a, torch.cuda.current_stream(dev).cuda_stream)
     return out, finals
 
@@ -164,7 +178,7 @@ class Phase:
     rows: torch.Tensor
     lens: list
     cu: tuple  # (device int32 cumulative lengths, host list)
-    rows_long: torch.Tensor = None  # ``rows`` as int64, for index_copy_
+    starts: torch.Tensor = None  # packed row of each run's first token (its tokens are consecutive packed rows)
 
 
 @dataclass
@@ -186,6 +200,10 @@ class RecurrentLayout:
     branch_segment: torch.Tensor | None  # segment of each branch
     past_segments: list  # segments with a cached conv history, in history order
     saves: list  # (segment, the k1 virtual rows of its conv tail at the save boundary)
+    # Where a run's initial state is: segment i's in [zeros; the past segments'
+    # states], a branch's in [every trunk 1's finals; every trunk 2's].
+    init_state: torch.Tensor | None = None
+    branch_state: torch.Tensor | None = None
 
     @classmethod
     def build(cls, segments, k1, n_rows, device):
@@ -221,9 +239,13 @@ class RecurrentLayout:
             take = np.concatenate([st + np.arange(len(t)) for st, (_, t) in zip(starts, runs)])
             rows = np.concatenate([t for _, t in runs])
             cu = np.concatenate([[0], np.cumsum(lens)])
-            parts.append((add(ext), add(take), add(rows), add(cu), lens))
+            first = [toks[0] if len(toks) else 0 for _, toks in runs]
+            parts.append((add(ext), add(take), add(rows), add(cu), lens, add(first)))
+        at = {i: len(segments) + j for j, i in enumerate(split)}  # a split segment's end state follows the trunk 1 finals
+        entry = {i: 1 + p for p, i in enumerate(past_segments)}
         extra = [add(split)] if split else []
-        extra += [add(br_seg)] if br_seg else []
+        extra += [add(br_seg), add([at.get(i, i) for i in br_seg])] if br_seg else []
+        extra += [add([entry.get(i, 0) for i in range(len(segments))])]
         sizes = [len(x) for x in lists]
         host = torch.from_numpy(np.concatenate(lists) if lists else np.zeros(0, np.int32))
         blob = (host.pin_memory().to(device, non_blocking=True) if torch.device(device).type == "cuda"
@@ -234,13 +256,14 @@ class RecurrentLayout:
         def phase(part):
             if part is None:
                 return None
-            e, t, r, c, lens = part
-            return Phase(piece[e], piece[t], piece[r], lens, (piece[c], lists[c].tolist()), piece[r].long())
+            e, t, r, c, lens, f = part
+            return Phase(piece[e], piece[t], piece[r], lens, (piece[c], lists[c].tolist()), piece[f])
 
-        j = len(lists) - len(extra)
-        split_d = piece[j].long() if split else None
-        br_d = piece[j + (1 if split else 0)].long() if br_seg else None
-        return cls(n_rows, phase(parts[0]), phase(parts[1]), phase(parts[2]), split_d, br_d, past_segments, saves)
+        tail = [piece[j] for j in extra]
+        split_d = tail.pop(0) if split else None
+        br_d, br_state = (tail.pop(0), tail.pop(0)) if br_seg else (None, None)
+        return cls(n_rows, phase(parts[0]), phase(parts[1]), phase(parts[2]), split_d, br_d, past_segments, saves,
+                   tail[0], br_state)
 
 
 def conv_phase(qkv, hist, ph, weight, b, a, a_log, dt_bias):
@@ -275,7 +298,9 @@ def conv_phase_args(qkv, hist, ph, weight, b, a, a_log, dt_bias):
     hist = None if hist is None else hist.to(qkv.dtype).contiguous()
     b = b if b.stride(1) == 1 else b.contiguous()
     a = a if a.stride(1) == 1 else a.contiguous()
-    al, dtb = a_log.float().contiguous(), dt_bias.float().contiguous()
+    lp = a_log.dtype == dt_bias.dtype == qkv.dtype  # the kernel reads these as they are, or as fp32
+    al, dtb = ((a_log, dt_bias) if lp else (a_log.float(), dt_bias.float()))
+    al, dtb = al.contiguous(), dtb.contiguous()
     out = torch.empty((t, c), dtype=qkv.dtype, device=dev)
     beta = torch.empty((t, hv), dtype=torch.float32, device=dev)
     g = torch.empty((t, hv), dtype=torch.float32, device=dev)
@@ -289,7 +314,7 @@ def conv_phase_args(qkv, hist, ph, weight, b, a, a_log, dt_bias):
     x.hist = 0 if hist is None else hist.data_ptr()
     x.ext, x.take, x.weight = ph.ext.data_ptr(), ph.take.data_ptr(), w.data_ptr()
     x.out, x.out_stride = out.data_ptr(), out.stride(0)
-    x.num_heads, x.rows = hv, ph.rows.data_ptr()
+    x.num_heads, x.gate_dtype, x.rows = hv, int(lp), ph.rows.data_ptr()
     x.b, x.b_stride, x.a, x.a_stride = b.data_ptr(), b.stride(0), a.data_ptr(), a.stride(0)
     x.a_log, x.dt_bias, x.beta, x.g = al.data_ptr(), dtb.data_ptr(), beta.data_ptr(), g.data_ptr()
     return x, (out, beta, g), (qkv, w, hist, b, a, al, dtb, ph)
@@ -335,30 +360,29 @@ class DeltaNet(nn.Module):
                 segments.recurrent = lay
         hist = (torch.cat([segments[i].past[self.index][0] for i in lay.past_segments])
                 if lay.past_segments else None)
-        zeros = torch.zeros(self.hv, self.dk, self.dv, device=x.device, dtype=torch.float32)
-        init = torch.stack([s.past[self.index][1].float() if s.past else zeros for s in segments])
+        states = torch.zeros(1, self.hv, self.dk, self.dv, device=x.device, dtype=torch.float32)
+        if lay.past_segments:
+            states = torch.cat([states] + [segments[i].past[self.index][1].float()[None] for i in lay.past_segments])
         out = torch.empty(n, self.hv, self.dv, device=x.device, dtype=x.dtype)
-        final = self._phase(lay.trunk1, qkv, hist, b, a, init, out)
-        if lay.trunk2 is not None:
-            f2 = self._phase(lay.trunk2, qkv, hist, b, a, final, out, lay.split_segments)
-            final_end = final.index_copy(0, lay.split_segments, f2)
-        else:
-            final_end = final
+        # the trunks' final states: part 1's, then part 2's
+        r, split = len(segments), 0 if lay.trunk2 is None else len(lay.trunk2.lens)
+        final = torch.empty(r + split, self.hv, self.dk, self.dv, device=x.device, dtype=torch.float32)
+        self._phase(lay.trunk1, qkv, hist, b, a, states, lay.init_state, out, final[:r])
+        if split:
+            self._phase(lay.trunk2, qkv, hist, b, a, final[:r], lay.split_segments, out, final[r:])
         for i, tail in lay.saves:  # prefix-cache entries at each save boundary
             segments[i].saved[self.index] = (_virtual_rows(qkv, hist, tail), final[i].clone())
         if lay.branches is not None:
-            self._phase(lay.branches, qkv, hist, b, a, final_end, out, lay.branch_segment)
+            self._phase(lay.branches, qkv, hist, b, a, final, lay.branch_state, out)
         return self.out_proj(_gated_norm(out, z, self.norm.weight, self.eps))
 
-    def _phase(self, ph, qkv, hist, b, a, states, out, state_index=None):
+    def _phase(self, ph, qkv, hist, b, a, states, state_index, out, finals=None):
         conv, beta, g = conv_phase(qkv, hist, ph, self.conv1d.weight, b, a, self.A_log, self.dt_bias)
         t, kd = conv.shape[0], self.hk * self.dk
         q = conv[:, :kd].view(t, self.hk, self.dk)
         k = conv[:, kd:2 * kd].view(t, self.hk, self.dk)
         v = conv[:, 2 * kd:].view(t, self.hv, self.dv)
-        o, f = delta_rule(q, k, v, g, beta, ph.lens, states, ph.cu, state_index=state_index)
-        out.index_copy_(0, ph.rows_long, o)
-        return f
+        _delta_rule(q, k, v, g, beta, ph.lens, states, ph.cu, state_index=state_index, out=out, out_start=ph.starts, finals=finals)
 
 
 def _virtual_rows(qkv, hist, idx):

@@ -29,7 +29,7 @@
 extern "C" {
 #endif
 
-#define DAN_GDN_ABI_VERSION 5
+#define DAN_GDN_ABI_VERSION 6
 
 /* Tokens per chunk of the chunked form. */
 #define DAN_GDN_CHUNK 64
@@ -78,7 +78,12 @@ typedef struct {
    * and :211 done in the state load; states_out must not overlap states_in. */
   const int32_t *state_index;
   int32_t num_states_in;
-  int32_t reserved2; /* 0 */
+  int32_t num_out_rows; /* rows of out, with out_start; at least num_tokens */
+  /* (GDN ABI 6) NULL (row t of the inputs writes row t of out), or [R] int32
+   * on the device: run r's outputs go to rows out_start[r] .. of out (clamped
+   * so that the run lies inside out), the packed rows the run's tokens came
+   * from (dan/models/qwen3_5.py:224, out.index_copy_). */
+  const int32_t *out_start;
 } DanGdnArgs;
 
 /* The gated delta rule over every run, from states_in to states_out.
@@ -122,12 +127,12 @@ typedef struct {
   const void *weight;                   /* [C, K] (nn.Conv1d's [C, 1, K]), 16-byte aligned */
   void *out; int64_t out_stride;        /* [T, C] */
   int32_t num_heads;                    /* Hv; 0 skips the gates */
-  int32_t reserved;
+  int32_t gate_dtype;                   /* (GDN ABI 6) 0: a_log and dt_bias are fp32; 1: they are of dtype */
   const int32_t *rows;                  /* [T] packed row of output row i */
   const void *b; int64_t b_stride;      /* [N, Hv] */
   const void *a; int64_t a_stride;      /* [N, Hv] */
-  const float *a_log;                   /* [Hv] */
-  const float *dt_bias;                 /* [Hv] */
+  const void *a_log;                    /* [Hv] */
+  const void *dt_bias;                  /* [Hv] */
   float *beta;                          /* [T, Hv] */
   float *g;                             /* [T, Hv] */
 } DanGdnConvArgs;
