@@ -20,7 +20,7 @@ LIB_DIR = os.path.join(HERE, "_lib")
 LIB_NAME = "libdan_tree_attn.so"
 LIB_PATH = os.path.join(LIB_DIR, LIB_NAME)
 
-ABI_VERSION = 8
+ABI_VERSION = 9
 KEY_TILE = 64
 SCRATCH_BYTES = 32 << 20  # DAN_TREE_ATTN_SCRATCH_BYTES: dan_tree_attn_fwd_noalloc's V^T scratch per GPU
 
@@ -72,7 +72,11 @@ class DanTreeAttnArgs(ctypes.Structure):
                 ("tile_q", _i32), ("vt_cols", _i32),
                 ("col_seg", _vp),
                 ("workspace", _vp), ("workspace_bytes", _i64), ("phases", _i32),
-                ("units", _vp), ("sched_off", _vp), ("num_slots", _i32), ("counts", _vp)]
+                ("units", _vp), ("sched_off", _vp), ("num_slots", _i32), ("counts", _vp),
+                ("pasts_host", _vp)]
+
+
+INLINE_PASTS = 8  # DAN_TREE_ATTN_INLINE_PASTS
 
 
 STAGE_PARTIALS = 1024  # DAN_TREE_ATTN_STAGE_PARTIALS
@@ -83,7 +87,7 @@ class DanStageF16Args(ctypes.Structure):
                 ("stride0", _i64), ("stride1", _i64), ("out", _vp), ("scale", _vp), ("partial", _vp)]
 
 
-FRONT_ABI_VERSION = 1
+FRONT_ABI_VERSION = 2
 FRONT_NORM_NONE, FRONT_NORM_RMS, FRONT_NORM_RMS_ZERO_CENTERED = 0, 1, 2
 
 
@@ -101,7 +105,10 @@ class DanQkvFrontArgs(ctypes.Structure):
                 ("q_norm_weight", _vp), ("k_norm_weight", _vp),
                 ("q_out", _vp), ("qo_stride_tok", _i64), ("qo_stride_head", _i64),
                 ("k_out", _vp), ("ko_stride_tok", _i64), ("ko_stride_head", _i64),
-                ("save_of", _vp), ("saves", _vp), ("num_saves", _i32)]
+                ("save_of", _vp), ("saves", _vp), ("num_saves", _i32), ("saves_host", _vp)]
+
+
+FRONT_INLINE_SAVES = 16  # DAN_QKV_FRONT_INLINE_SAVES
 
 
 PLAN_ABI_VERSION = 2

@@ -254,16 +254,20 @@ def _stage_f16(x):
     return out, scale
 
 
-def _past_table(plan, layer, hkv, d, dtype, device):
-    """Device table of DanPastDesc for ``layer`` (cached on the plan). An
-    e4m3 entry is (k, v, k_scale, v_scale)."""
-    hit = plan.past_tables.get(layer)
-    if hit is not None:
-        return hit
-    raw, refs = _past_descs(plan.past_dicts, plan.segs, layer, hkv, d, dtype, device)
-    table = raw.pin_memory().to(device, non_blocking=True) if device.type == "cuda" else raw
-    plan.past_tables[layer] = (table, refs)
-    return plan.past_tables[layer]
+def _past_table(plan, layer, hkv, d, dtype, device, upload=True):
+    """Device table of DanPastDesc for ``layer`` and the tensors it points at
+    (cached on the plan). An e4m3 entry is (k, v, k_scale, v_scale). Without
+    ``upload`` a table of at most INLINE_PASTS entries is left to the launch,
+    which takes its bytes (``plan.past_hosts[layer]``) by value and fills it."""
+    if layer not in plan.past_tables:
+        raw, refs = _past_descs(plan.past_dicts, plan.segs, layer, hkv, d, dtype, device)
+        plan.past_hosts[layer] = raw if len(plan.past_dicts) <= _native.INLINE_PASTS else None
+        plan.past_tables[layer] = (torch.empty(raw.numel(), dtype=torch.uint8, device=device), (refs, raw))
+    table, (refs, raw) = plan.past_tables[layer]
+    if (upload or plan.past_hosts[layer] is None) and layer not in plan.past_uploaded:
+        table.copy_(raw.pin_memory() if device.type == "cuda" else raw, non_blocking=True)
+        plan.past_uploaded.add(layer)
+    return table, refs
 
 
 def _past_descs(past_dicts, segs, layer, hkv, d, dtype, device, capacity=None):
@@ -328,17 +332,15 @@ def _attend_fused(q, k, v, segments, layer, scale, fp8_scales=None, phases=_nati
         raise ValueError("noalloc calls run both phases (PHASES_ALL); a split call needs a workspace")
     if phases != _native.PHASES_ALL and workspace is None:
         raise ValueError("a split call (PHASE_PACK / PHASE_ATTEND) needs the workspace the two phases share")
-    return _call_op(*_op_args(q, k, v, segments, layer, scale, fp8_scales, phases, noalloc), workspace)
-
-
-def _call_op(*args):
-    """``torch.ops.dan_amd.tree_attn`` under ``torch.compile``; in eager mode
-    the launch itself, without the operator dispatch (the autograd and
-    in-place wrappers cost about as much host time per call as the launch:
-    the call is forward-only and its workspace is the call's own)."""
+    # Eager calls launch without the operator dispatch (its autograd and in-place
+    # wrappers cost about as much host time as the launch: the call is
+    # forward-only and its workspace is the call's own).
     if torch.compiler.is_compiling():
-        return torch.ops.dan_amd.tree_attn(*args)
-    return _launch_tree_attn(*args)
+        return torch.ops.dan_amd.tree_attn(*_op_args(q, k, v, segments, layer, scale, fp8_scales, phases, noalloc), workspace)
+    # an attention-only launch has no copy before it that would fill the prefix table
+    args, pasts_host = _call_args(q, k, v, segments, layer, scale, fp8_scales, phases, noalloc,
+                                  upload=phases == _native.PHASE_ATTEND)
+    return _launch_tree_attn(*args, workspace, pasts_host)
 
 
 def workspace_bytes(q, k, segments):
@@ -356,6 +358,12 @@ def workspace_bytes(q, k, segments):
 def _op_args(q, k, v, segments, layer, scale, fp8_scales=None, phases=_native.PHASES_ALL, noalloc=False):
     """Checks the inputs, builds (or finds) the batch's plan and the layer's
     prefix-cache table, and returns the arguments of ``tree_attn``."""
+    return _call_args(q, k, v, segments, layer, scale, fp8_scales, phases, noalloc)[0]
+
+
+def _call_args(q, k, v, segments, layer, scale, fp8_scales, phases, noalloc, upload=True):
+    """``_op_args``, and the host bytes of the prefix-cache table that the
+    launch fills it from (None: the table is uploaded, or empty)."""
     if not q.is_cuda:
         raise RuntimeError("dan_amd.attend runs on a gfx950 GPU only; got tensors on "
                            f"{q.device} (the masked CPU path is the test oracle, not a backend)")
@@ -372,7 +380,7 @@ def _op_args(q, k, v, segments, layer, scale, fp8_scales=None, phases=_native.PH
         raise ValueError(f"unsupported head layout H={h}, Hkv={hkv}")
     groups = _native.head_groups(h, hkv, lib)
     plan = get_plan(segments, n, tile_q, q.device, groups=groups, num_cus=_num_cus(q.device))
-    table, _refs = _past_table(plan, layer, hkv, d, q.dtype, q.device)
+    table, _refs = _past_table(plan, layer, hkv, d, q.dtype, q.device, upload)
     if q.dtype == E4M3:
         q_scale, k_scale, v_scale = (_check_scale(t, nm, q.device) for t, nm in zip(fp8_scales, ("q_scale", "k_scale", "v_scale")))
     scales = [q_scale, k_scale, v_scale] if q.dtype == E4M3 else []
@@ -386,7 +394,8 @@ def _op_args(q, k, v, segments, layer, scale, fp8_scales=None, phases=_native.PH
         tables += [units, sched_off]
     meta = [len(plan.segs), len(plan.past_dicts), plan.num_work, tile_q, plan.vt_cols, slots, phases, int(noalloc)]
     softmax_scale = (1.0 / math.sqrt(d)) if scale is None else float(scale)
-    return q, k, v, tables, scales, meta, softmax_scale
+    pasts_host = None if upload or not plan.past_dicts or layer in plan.past_uploaded else plan.past_hosts[layer]
+    return (q, k, v, tables, scales, meta, softmax_scale), pasts_host
 
 
 def _out_dtype(q, v):
@@ -418,8 +427,9 @@ def tree_attn(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, tables: List[to
     return _launch_tree_attn(q, k, v, tables, scales, meta, scale, workspace)
 
 
-def _launch_tree_attn(q, k, v, tables, scales, meta, scale, workspace):
-    """The body of ``tree_attn``."""
+def _launch_tree_attn(q, k, v, tables, scales, meta, scale, workspace, pasts_host=None):
+    """The body of ``tree_attn``; ``pasts_host`` (uint8, on the host): the
+    prefix-cache table's entries, which the launch writes to the table."""
     lib = _native.load()
     h, n, d = q.shape
     hkv = k.shape[0]
@@ -447,6 +457,8 @@ def _launch_tree_attn(q, k, v, tables, scales, meta, scale, workspace):
         a.out, a.o_stride_tok, a.o_stride_head = out.data_ptr(), out.stride(0), out.stride(1)
         a.segments, a.num_segments = segs_d.data_ptr(), num_segments
         a.pasts, a.num_pasts = past_table.data_ptr(), num_pasts
+        if pasts_host is not None:
+            a.pasts_host = pasts_host.data_ptr()
         a.work, a.num_work = work_d.data_ptr(), num_work
         a.key_lo = key_lo_d.data_ptr()
         a.tile_q = tile_q
@@ -635,4 +647,6 @@ class BudgetPlan:
         meta = [self.max_segments, self.max_segments, self.max_work, self.tile_q, self.max_cols * _native.KEY_TILE,
                 self.slots, _native.PHASES_ALL, 0]
         softmax_scale = (1.0 / math.sqrt(self.d)) if scale is None else float(scale)
-        return _call_op(q, k, v, tables, scales, meta, softmax_scale, None)
+        if torch.compiler.is_compiling():
+            return torch.ops.dan_amd.tree_attn(q, k, v, tables, scales, meta, softmax_scale, None)
+        return _launch_tree_attn(q, k, v, tables, scales, meta, softmax_scale, None)

@@ -110,10 +110,24 @@ struct Params {
   void *qo, *ko;
   int64_t q_st, q_sh, k_st, k_sh, v_st, v_sh, cs_st, qo_st, qo_sh, ko_st, ko_sh;
   const int32_t *save_of;
-  const DanFrontSave *saves;
+  const DanFrontSave *saves;  // NULL: the entries are `inl`
   int32_t N, H, Hkv, R, norm;
   float eps;
+  DanFrontSave inl[DAN_QKV_FRONT_INLINE_SAVES];
 };
+
+// Entry si of the saves. The inline ones are read from the kernel's argument
+// segment (Params is its first argument) by their index in memory: indexing
+// the argument itself would copy it to scratch.
+__device__ inline DanFrontSave save_at(const Params &p, int si) {
+  typedef const __attribute__((address_space(4))) uint8_t *ArgPtr;
+  typedef const __attribute__((address_space(4))) DanFrontSave *SavePtr;
+  if (p.saves) return p.saves[si];
+  const SavePtr e = (SavePtr)((ArgPtr)__builtin_amdgcn_kernarg_segment_ptr() + __builtin_offsetof(Params, inl)) + si;
+  DanFrontSave sv;
+  sv.start = e->start; sv.len = e->len; sv.k_dst = e->k_dst; sv.v_dst = e->v_dst;
+  return sv;
+}
 
 // Head vectors per lane (qkv_front_kernel).
 constexpr int kVecs = 2;
@@ -215,7 +229,7 @@ __global__ __launch_bounds__(256) void qkv_front_kernel(const Params p) {
     if (!isq && p.save_of) {
       const int si = p.save_of[t];
       if (si >= 0) {
-        const DanFrontSave sv = p.saves[si];
+        const DanFrontSave sv = save_at(p, si);
         const int64_t row = (int64_t)head * sv.len + (t - sv.start);
         store16(static_cast<T *>(sv.k_dst) + row * D + 8 * j, out);
         const T *vs = static_cast<const T *>(p.v) + t * p.v_st + head * p.v_sh;
@@ -261,8 +275,10 @@ int dan_qkv_front(const DanQkvFrontArgs *a, void *stream) {
     return fail(DAN_ERR_INVALID_ARGUMENT, "norm %d is not a DanFrontNorm", a->norm);
   if (a->norm != DAN_FRONT_NORM_NONE && (!a->q_norm_weight || !a->k_norm_weight || !dan::finite_nonnegative(a->eps)))
     return fail(DAN_ERR_INVALID_ARGUMENT, "a norm needs q_norm_weight, k_norm_weight and a finite eps >= 0");
-  if (a->num_saves < 0 || (a->num_saves > 0 && (!a->save_of || !a->saves || !a->v)))
+  if (a->num_saves < 0 || (a->num_saves > 0 && (!a->save_of || !(a->saves || a->saves_host) || !a->v)))
     return fail(DAN_ERR_INVALID_ARGUMENT, "saves need save_of, saves and v");
+  if (a->saves_host && a->num_saves > DAN_QKV_FRONT_INLINE_SAVES)
+    return fail(DAN_ERR_INVALID_ARGUMENT, "saves_host holds at most %d entries, got %d", DAN_QKV_FRONT_INLINE_SAVES, a->num_saves);
   if (N == 0) return DAN_OK;
   if (!a->q || !a->k || !a->q_out || !a->k_out || (R > 0 && (!a->cos || !a->sin)))
     return fail(DAN_ERR_INVALID_ARGUMENT, "NULL tensor pointer");
@@ -285,7 +301,8 @@ int dan_qkv_front(const DanQkvFrontArgs *a, void *stream) {
   p.v_st = a->v_stride_tok; p.v_sh = a->v_stride_head; p.cs_st = a->cs_stride_tok;
   p.qo_st = a->qo_stride_tok; p.qo_sh = a->qo_stride_head; p.ko_st = a->ko_stride_tok; p.ko_sh = a->ko_stride_head;
   p.save_of = a->num_saves > 0 ? a->save_of : nullptr;
-  p.saves = a->saves;
+  p.saves = a->saves_host ? nullptr : a->saves;
+  for (int i = 0; a->saves_host && i < a->num_saves; ++i) p.inl[i] = a->saves_host[i];
   p.N = N; p.H = H; p.Hkv = Hkv; p.R = R; p.norm = a->norm; p.eps = a->eps;
 
   hipStream_t s = static_cast<hipStream_t>(stream);

@@ -162,6 +162,13 @@ struct PackParams {
   int32_t num_kv_heads, vt_cols;
   const float *v_scale;  // e4m3 only: per-tensor scale of v (prefix-cache entries carry their own)
   const int32_t *counts; // budget mode: device {S, B, W, C}; column blocks from C on are skipped
+  // Prefix entries given by value (num_inline > 0): read here, and written by
+  // the first work group to `pasts_out` (then the same memory as `pasts`) for
+  // the attention launch. An uploaded table cost each layer's first call a
+  // pinned allocation and a copy (about 20 us of host and 2.8 us of GPU time).
+  DanPastDesc *pasts_out;
+  int32_t num_inline;
+  DanPastDesc inl[DAN_TREE_ATTN_INLINE_PASTS];
 };
 
 // ---------------------------------------------------------------- element I/O
@@ -600,6 +607,15 @@ __global__ __launch_bounds__(256) void vt_pack_kernel(const PackParams p) {
   __shared__ __attribute__((aligned(16))) uint32_t tile[D * 32];
   __shared__ float wave_max[4];
   const int kvh = blockIdx.x % p.num_kv_heads, cb = blockIdx.x / p.num_kv_heads;
+  const DanPastDesc *pasts = p.pasts;
+  if (p.num_inline > 0) {  // in the argument segment (p is the first argument), indexed in memory
+    const __attribute__((address_space(4))) uint8_t *args = (const __attribute__((address_space(4))) uint8_t *)__builtin_amdgcn_kernarg_segment_ptr();
+    pasts = (const DanPastDesc *)(args + __builtin_offsetof(PackParams, inl));
+    constexpr int kWords = (int)sizeof(DanPastDesc) / 4;
+    if (blockIdx.x == 0 && (int)threadIdx.x < p.num_inline * kWords)
+      *gbl_mut(reinterpret_cast<uint32_t *>(p.pasts_out) + threadIdx.x) = reinterpret_cast<const uint32_t *>(pasts)[threadIdx.x];
+    static_assert(DAN_TREE_ATTN_INLINE_PASTS * kWords <= 256, "one word per thread");
+  }
   if (p.counts && cb >= load_scalar(p.counts + 3)) return;  // past this batch's columns (the grid covers the capacity)
   const DanSegmentDesc sg = load_scalar(p.segs + load_scalar(p.col_seg + cb));
   const int key0 = cb * kKeyTile - sg.vt_col;
@@ -610,7 +626,7 @@ __global__ __launch_bounds__(256) void vt_pack_kernel(const PackParams p) {
   float vs = 1.f, pvs = 1.f;
   if (kF8) vs = load_scalar(p.v_scale);
   if (P > 0) {
-    const DanPastDesc pd = load_scalar(p.pasts + sg.past_idx);
+    const DanPastDesc pd = load_scalar(pasts + sg.past_idx);
     pvp = static_cast<const TV *>(pd.v) + (int64_t)kvh * pd.v_stride_head;
     pv_st = pd.v_stride_tok;
     if (kF8) pvs = load_scalar(pd.v_scale);
@@ -1635,6 +1651,8 @@ int dan_tree_attn_fwd(const DanTreeAttnArgs *a, void *stream) {
   if (!a->q || !a->k || !a->v || !a->out || !a->segments || !a->work || !a->key_lo || !a->col_seg)
     return fail(DAN_ERR_INVALID_ARGUMENT, "NULL tensor or table pointer");
   if (a->num_pasts > 0 && !a->pasts) return fail(DAN_ERR_INVALID_ARGUMENT, "num_pasts > 0 with NULL pasts");
+  if (a->pasts_host && a->num_pasts > DAN_TREE_ATTN_INLINE_PASTS)
+    return fail(DAN_ERR_INVALID_ARGUMENT, "pasts_host holds at most %d entries, got %d", DAN_TREE_ATTN_INLINE_PASTS, a->num_pasts);
   if (f8 && (!a->q_scale || !a->k_scale || !a->v_scale))
     return fail(DAN_ERR_INVALID_ARGUMENT, "e4m3 inputs need q_scale, k_scale and v_scale");
   if (!f8 && (!a->q_scale != !a->k_scale || (a->q_scale && !f32)))
@@ -1680,6 +1698,9 @@ int dan_tree_attn_fwd(const DanTreeAttnArgs *a, void *stream) {
   pp.num_kv_heads = Hkv; pp.vt_cols = a->vt_cols;
   pp.v_scale = a->v_scale;
   pp.counts = a->counts;
+  pp.pasts_out = const_cast<DanPastDesc *>(a->pasts);
+  pp.num_inline = a->pasts_host ? a->num_pasts : 0;
+  for (int i = 0; i < pp.num_inline; ++i) pp.inl[i] = a->pasts_host[i];
 
   KParams kp;
   kp.q = a->q; kp.k = a->k; kp.o = a->out; kp.vt = pp.vt; kp.vexp = pp.vexp;

@@ -15,6 +15,8 @@ Numerics are the eager ops': fp32 arithmetic with each op's result rounded to
 the model dtype; only the summation order of the norm's sum of squares
 differs from torch.
 """
+import ctypes
+
 import numpy as np
 import torch
 
@@ -142,10 +144,14 @@ def qkv_front(q, k, v, cos, sin, *, q_norm_weight=None, k_norm_weight=None, eps=
         table = (_native.DanFrontSave * len(order))()
         for i, (s, (kd, vd)) in enumerate(zip(order, dst)):
             table[i].start, table[i].len, table[i].k_dst, table[i].v_dst = s.start, s.save, kd.data_ptr(), vd.data_ptr()
-        raw = torch.frombuffer(bytearray(table), dtype=torch.uint8)
-        table_d = raw.pin_memory().to(dev, non_blocking=True)
-        a.save_of, a.saves, a.num_saves = save_of.data_ptr(), table_d.data_ptr(), len(order)
-        keep = [table_d]
+        a.save_of, a.num_saves = save_of.data_ptr(), len(order)
+        if len(order) <= _native.FRONT_INLINE_SAVES:  # in the launch's arguments
+            a.saves_host = ctypes.addressof(table)
+        else:
+            raw = torch.frombuffer(bytearray(table), dtype=torch.uint8)
+            table_d = raw.pin_memory().to(dev, non_blocking=True)
+            a.saves = table_d.data_ptr()
+            keep = [table_d]
         for s, kv in zip(order, dst):
             s.saved[layer] = kv
     _native.front(a, torch.cuda.current_stream(dev).cuda_stream, lib)

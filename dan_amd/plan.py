@@ -247,6 +247,8 @@ class TilePlan:
     key_lo_d: object = None
     col_seg_d: object = None
     past_tables: dict = field(default_factory=dict)  # layer -> (device bytes, keep-alive refs)
+    past_hosts: dict = field(default_factory=dict)  # layer -> the table's host bytes (None: too long to ride in a launch)
+    past_uploaded: set = field(default_factory=set)  # the layers whose device table was filled by an upload
     schedules: dict = field(default_factory=dict)  # (groups, CUs) -> (units_d, sched_off_d, slots)
 
     @classmethod

@@ -36,7 +36,7 @@
 extern "C" {
 #endif
 
-#define DAN_QKV_FRONT_ABI_VERSION 1
+#define DAN_QKV_FRONT_ABI_VERSION 2
 
 typedef enum {
   DAN_FRONT_NORM_NONE = 0,
@@ -80,7 +80,13 @@ typedef struct {
   const int32_t *save_of;
   const DanFrontSave *saves;
   int32_t num_saves;
+  /* (ABI 2) NULL, or a host copy of the num_saves entries, at most
+   * DAN_QKV_FRONT_INLINE_SAVES, which travels in the kernel's arguments: no
+   * table is uploaded and `saves` is not read. Read during the call only. */
+  const DanFrontSave *saves_host;
 } DanQkvFrontArgs;
+
+#define DAN_QKV_FRONT_INLINE_SAVES 16
 
 /* q_out, k_out (and the saves) from q, k, v in one launch. Replaces the GPU
  * leg of dan/models/llama.py:78-86 and dan/models/qwen3_5.py:318-326 up to

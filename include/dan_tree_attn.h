@@ -42,7 +42,7 @@
 extern "C" {
 #endif
 
-#define DAN_TREE_ATTN_ABI_VERSION 8
+#define DAN_TREE_ATTN_ABI_VERSION 9
 
 /* Keys per key tile; the work list's key-tile indices count in these. */
 #define DAN_TREE_ATTN_KEY_TILE 64
@@ -199,7 +199,16 @@ typedef struct {
    * slots past this batch's are empty. The same launches, captured once,
    * serve every batch within the capacities. */
   const int32_t *counts;
+  /* (ABI 9) NULL, or a host copy of the num_pasts entries of `pasts`, at most
+   * DAN_TREE_ATTN_INLINE_PASTS: the entries travel in the V^T copy's kernel
+   * arguments, and the copy writes them to `pasts` (device memory for
+   * num_pasts entries, whatever it held) for the attention launch, so the
+   * caller uploads no table. Read during the call only; unused by
+   * DAN_TREE_ATTN_PHASE_ATTEND, which reads the table the copy wrote. */
+  const DanPastDesc *pasts_host;
 } DanTreeAttnArgs;
+
+#define DAN_TREE_ATTN_INLINE_PASTS 8
 
 #define DAN_TREE_ATTN_PHASES_ALL 0
 #define DAN_TREE_ATTN_PHASE_PACK 1
