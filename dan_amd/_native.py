@@ -73,7 +73,7 @@ class DanTreeAttnArgs(ctypes.Structure):
                 ("col_seg", _vp),
                 ("workspace", _vp), ("workspace_bytes", _i64), ("phases", _i32),
                 ("units", _vp), ("sched_off", _vp), ("num_slots", _i32), ("counts", _vp),
-                ("pasts_host", _vp)]
+                ("pasts_host", _vp), ("key_halves", _i32)]
 
 
 INLINE_PASTS = 8  # DAN_TREE_ATTN_INLINE_PASTS

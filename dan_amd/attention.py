@@ -232,6 +232,13 @@ def get_plan(segments, num_tokens, tile_q, device, groups=None, num_cus=None, pl
     return plan
 
 
+# Half tiles (``_tile_q``) where the whole ones, this many times over, fit the
+# CUs. Attention launch on 256 CUs, whole / half time: 1.0 to 1.5 at up to 128
+# units (834 tokens on 32/8 heads 1.35), 0.92 to 1.36 at 192, 0.84 to 1.22 at 256
+# (more than one request: 0.84 to 1.0), 0.82 to 0.97 from 352 on.
+HALF_TILE_UNITS = 2
+
+
 def _qk_dtype(dtype):
     """Matrix-core type of q and k: fp32 callers' are staged as fp16 (``_stage_f16``)."""
     return torch.float16 if dtype == torch.float32 else dtype
@@ -343,16 +350,33 @@ def _attend_fused(q, k, v, segments, layer, scale, fp8_scales=None, phases=_nati
     return _launch_tree_attn(*args, workspace, pasts_host)
 
 
+@functools.lru_cache(maxsize=None)
+def _layout(h, hkv, d):
+    """(queries per whole work item, head groups) of a head layout; zeros if unsupported."""
+    lib = _native.load()
+    return _native.tile_q(h, hkv, d, lib=lib), _native.head_groups(h, hkv, lib)
+
+
+def _tile_q(h, hkv, d, n, device):
+    """Queries per work item of a batch of ``n`` packed tokens: the kernel's
+    tile, or half of it where whole tiles would leave at least half of the
+    CUs without one (the kernel then splits each key tile between its waves).
+    It depends on the packed length alone, so a BudgetPlan and a batch's own
+    plan agree. 0: unsupported head layout."""
+    tile_q, groups = _layout(h, hkv, d)
+    if tile_q > 0 and d <= 128 and -(-n // tile_q) * groups * HALF_TILE_UNITS <= _num_cus(device):
+        return tile_q // 2
+    return tile_q
+
+
 def workspace_bytes(q, k, segments):
     """Bytes of the V^T workspace of a split ``_attend_fused`` call on this
     batch (the plan is built or found as for the call itself)."""
     h, n, d = q.shape
     hkv = k.shape[0]
-    lib = _native.load()
-    tile_q = _native.tile_q(h, hkv, d, lib=lib)
-    groups = _native.head_groups(h, hkv, lib)
+    tile_q, groups = _tile_q(h, hkv, d, n, q.device), _layout(h, hkv, d)[1]
     plan = get_plan(segments, n, tile_q, q.device, groups=groups, num_cus=_num_cus(q.device))
-    return _native.workspace_size(hkv, d, plan.vt_cols, lib)
+    return _native.workspace_size(hkv, d, plan.vt_cols)
 
 
 def _op_args(q, k, v, segments, layer, scale, fp8_scales=None, phases=_native.PHASES_ALL, noalloc=False):
@@ -372,13 +396,12 @@ def _call_args(q, k, v, segments, layer, scale, fp8_scales, phases, noalloc, upl
     _check_inputs(q, k, v)
     if scale is not None and not (float(scale) > 0 and math.isfinite(float(scale))):
         raise ValueError(f"scale {scale}: the kernel needs a finite positive softmax scale")
-    lib = _native.load()
     h, n, d = q.shape
     hkv = k.shape[0]
-    tile_q = _native.tile_q(h, hkv, d, lib=lib)
+    tile_q = _tile_q(h, hkv, d, n, q.device)
     if tile_q <= 0:
         raise ValueError(f"unsupported head layout H={h}, Hkv={hkv}")
-    groups = _native.head_groups(h, hkv, lib)
+    groups = _layout(h, hkv, d)[1]
     plan = get_plan(segments, n, tile_q, q.device, groups=groups, num_cus=_num_cus(q.device))
     table, _refs = _past_table(plan, layer, hkv, d, q.dtype, q.device, upload)
     if q.dtype == E4M3:
@@ -461,7 +484,7 @@ def _launch_tree_attn(q, k, v, tables, scales, meta, scale, workspace, pasts_hos
             a.pasts_host = pasts_host.data_ptr()
         a.work, a.num_work = work_d.data_ptr(), num_work
         a.key_lo = key_lo_d.data_ptr()
-        a.tile_q = tile_q
+        a.tile_q, a.key_halves = tile_q, _layout(h, hkv, d)[0] // tile_q
         a.vt_cols = vt_cols
         a.col_seg = col_seg_d.data_ptr()
         if ws is not None:
@@ -518,8 +541,8 @@ class BudgetPlan:
             raise RuntimeError("BudgetPlan runs on a gfx950 GPU only")
         lib = _native.load()
         self.n, self.h, self.hkv, self.d, self.dtype, self.device = num_tokens, num_heads, num_kv_heads, head_dim, dtype, device
-        self.tile_q = _native.tile_q(num_heads, num_kv_heads, head_dim, lib=lib)
-        self.groups = _native.head_groups(num_heads, num_kv_heads, lib)
+        self.tile_q = _tile_q(num_heads, num_kv_heads, head_dim, num_tokens, device)
+        self.groups = _layout(num_heads, num_kv_heads, head_dim)[1]
         if self.tile_q <= 0 or head_dim not in (64, 128, 256) or dtype not in _DTYPES:
             raise ValueError(f"unsupported layout {num_heads}/{num_kv_heads} x {head_dim}, {dtype}")
         self.max_segments, self.max_branches = max_segments, max_branches

@@ -536,6 +536,18 @@ struct Lds {
   static_assert(buf % (32 * kRowBytes) == 0, "buffer alignment");
 };
 
+// LDS of the key halves' merge, past the ring and the votes: per wave pair the
+// statistics (3 x 64 floats) and `blocks` d blocks of O (4 KB each) a round.
+template <int D, int KB>
+struct Merge {
+  static constexpr int stat = Lds<D, KB>::total + kVoteBytes;
+  static constexpr int part = stat + 4 * 768;
+  static constexpr int room = (160 * 1024 - part) / (4 * 4096);
+  static constexpr int blocks = room >= D / 32 ? D / 32 : room >= 2 ? 2 : 1;
+  static constexpr int total = part + 4 * 4096 * blocks;
+  static_assert(D == 256 || total <= 160 * 1024, "LDS");
+};
+
 // Slot of chunk c of K row m (see Lds).
 template <int D, int KB>
 __host__ __device__ constexpr int kswz(int m) {
@@ -696,7 +708,18 @@ __global__ __launch_bounds__(256) void vt_pack_kernel(const PackParams p) {
 // TQK: matrix-core type of S = K Q^T (q, k and the pasts' k): bf16, fp16 or
 // e4m3. P V always runs in fp16: P keeps 11 significant bits instead of
 // bf16's 8 (or e4m3's 4), and the V^T copy is fp16.
-template <typename TQK, typename TOut, int D>
+// KH: key halves. With 2, waves 0-3 and 4-7 take the same queries (half as
+// many per work item) and keys 0-31 and 32-63 of every tile, each with its
+// own running max, row sum and O, merged through LDS at the unit's end. For
+// batches of at most half as many units as CUs, where the longest unit's
+// serial steps set the time: the units double, and a step has half the
+// products, exponentials and operand reads (2.2 -> 1.3 us; its direct loads
+// are the same). Attention launch, one request on 32/8 heads x 128, whole tiles
+// -> halves: 834 tokens 29.4 -> 21.7 us, 834 behind a 1024-token prefix 50.8 ->
+// 36.0; 8/2 heads x 64, 2048 tokens 39.9 -> 26.8. With more units than that the
+// doubled loads lose (2776 tokens in 4 requests, 352 units: 29.8 -> 34.5). All
+// eight waves issuing the loads: 5 to 12 % slower than waves 0-3.
+template <typename TQK, typename TOut, int D, int KH>
 __global__ __attribute__((amdgpu_flat_work_group_size(Shape<D>::threads, Shape<D>::threads),
                           amdgpu_waves_per_eu(Shape<D>::waves_per_simd, Shape<D>::waves_per_simd)))
 void tree_attn_kernel(const KParams args) {
@@ -707,6 +730,8 @@ void tree_attn_kernel(const KParams args) {
   // loads.
   constexpr bool kTwoStage = NB == 2;
   static_assert(NB == 4 || (NB == 2 && D == 256), "ring of 4, or 2 at head_dim 256");
+  static_assert(KH == 1 || (KH == 2 && !kTwoStage), "key halves: ring of 4 only");
+  constexpr int NMB = 2 / KH;  // 32-key blocks of a tile per wave
   constexpr int WQ = Shape<D>::wave_q;  // queries per wave
   constexpr int kIssuers = Issuers<D>::n;  // waves that issue the stage loads
   constexpr bool kF8 = std::is_same<TQK, E4M3>::value;
@@ -724,6 +749,8 @@ void tree_attn_kernel(const KParams args) {
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lane = tid & 63, hl = lane >> 5, lq = lane & 31;
+  // The wave among those that share a key half, and its half.
+  const int cwave = KH == 2 ? wave & 3 : wave, khalf = KH == 2 ? wave >> 2 : 0;
   // The lane's query within the wave, and which part of a k-step of S it
   // holds (32x32 products: two halves; 16x16: four quarters).
   const int lqq = WQ == 16 ? (lane & 15) : lq, kpart = WQ == 16 ? (lane >> 4) : hl;
@@ -731,8 +758,9 @@ void tree_attn_kernel(const KParams args) {
   // 32-row block with its chunk swizzle and half-step folded in; the chunk
   // of each k-step is XOR'd in per read (it only touches the low bits).
   // V^T: the lane's 16 bytes of each operand fragment block.
-  const uint32_t k_lane = (uint32_t)(lq * RB + kswz<D, (int)sizeof(TQK)>(lq) * 16) ^ (uint32_t)(hl * CH * 16);
-  const uint32_t v_lane = (uint32_t)(L::kBytes + lane * 16);
+  const uint32_t k_lane = ((uint32_t)(lq * RB + kswz<D, (int)sizeof(TQK)>(lq) * 16) ^ (uint32_t)(hl * CH * 16)) +
+                          (uint32_t)(khalf * 32 * RB);
+  const uint32_t v_lane = (uint32_t)(L::kBytes + khalf * 2 * ND * 1024 + lane * 16);
 
   // units holds num_units records: clamping the range keeps a malformed
   // offset table from reading past it.
@@ -879,8 +907,8 @@ void tree_attn_kernel(const KParams args) {
   bool q_ready = false;
   auto load_q = [&](const KParams &p, const DanUnit &un) __attribute__((always_inline)) {
     const int g = un.group, kvh = g % p.num_kv_heads, chunk = g / p.num_kv_heads;
-    const int hig = chunk * p.hpw + (wave % p.hpw), head = kvh * p.rep + hig;
-    const int qw0 = un.item.t0 + (wave / p.hpw) * WQ, qend = un.item.t0 + un.item.tq;
+    const int hig = chunk * p.hpw + (cwave % p.hpw), head = kvh * p.rep + hig;
+    const int qw0 = un.item.t0 + (cwave / p.hpw) * WQ, qend = un.item.t0 + un.item.tq;
     const int ql = qw0 + lqq;
     const bool qvalid = hig < p.rep && qw0 < qend && ql < qend;
     const int qrow = un.start + min(ql, qend - 1);
@@ -931,9 +959,9 @@ void tree_attn_kernel(const KParams args) {
     };
     auto issued_cat = [&](int i) __attribute__((always_inline)) { return i < ntile + nn; };
 
-    const int hig = chunk * p.hpw + (wave % p.hpw);
+    const int hig = chunk * p.hpw + (cwave % p.hpw);
     const int head = kvh * p.rep + hig;
-    const int qw0 = w.t0 + (wave / p.hpw) * WQ;  // wave's first query (segment-local)
+    const int qw0 = w.t0 + (cwave / p.hpw) * WQ;  // wave's first query (segment-local)
     const int qend = w.t0 + w.tq;
     const bool wave_work = hig < p.rep && qw0 < qend;
 
@@ -961,29 +989,30 @@ void tree_attn_kernel(const KParams args) {
     // O holds O_true * 2^-vE: the exponent of the V^T blocks it was last
     // accumulated from (0 unless a block of this unit needed one).
     int vE = 0;
-    u32x4 pf[4];  // P^T B operands (fp16), one per 16 keys of the tile
+    u32x4 pf[2 * NMB];  // P^T B operands (fp16), one per 16 keys of the wave's part of the tile
 
-    // S^T = K Q^T for the 64 keys of stage buffer b x this wave's 32 queries.
-    auto qk_phase = [&](int b, f32x16(&s)[2], auto &&after_kstep) {
+    // S^T = K Q^T for the 64 keys (or the wave's half) of stage buffer b x this
+    // wave's 32 queries.
+    auto qk_phase = [&](int b, f32x16(&s)[NMB], auto &&after_kstep) {
       // LDS address of this lane's row in buffer b. The dynamic LDS block is
       // the kernel's only LDS object and starts at address 0, and buffer
       // offsets are multiples of 32 rows, so XOR-ing a chunk into the address
       // only changes the lane's row offset: one v_xor per k-step.
       const uint32_t kbase = (uint32_t)(uintptr_t)(DAN_LDS uint8_t *)(smem + b * L::buf) + k_lane;
-      s[0] = f32x16{};
-      s[1] = f32x16{};
+#pragma unroll
+      for (int mb = 0; mb < NMB; ++mb) s[mb] = f32x16{};
 #pragma unroll
       for (int kk = 0; kk < NK; ++kk) {
-        Frag<TQK> a[2];
+        Frag<TQK> a[NMB];
 #pragma unroll
         for (int i = 0; i < CH; ++i) {
           const uint32_t off = kbase ^ (uint32_t)((2 * kk * CH + i) * 16);
 #pragma unroll
-          for (int mb = 0; mb < 2; ++mb)
+          for (int mb = 0; mb < NMB; ++mb)
             a[mb].c[i] = *reinterpret_cast<const DAN_LDS u32x4 *>((uintptr_t)(off + mb * 32 * RB));
         }
 #pragma unroll
-        for (int mb = 0; mb < 2; ++mb) s[mb] = mfma_qk<TQK>(a[mb], qf[kk], s[mb]);
+        for (int mb = 0; mb < NMB; ++mb) s[mb] = mfma_qk<TQK>(a[mb], qf[kk], s[mb]);
         after_kstep(kk);
       }
     };
@@ -991,14 +1020,15 @@ void tree_attn_kernel(const KParams args) {
     // start: 32*mb + 16*(r/8) + 8*hl + r%8. The causal limit and the
     // sibling-branch gap are per-lane bounds on it; the gap test runs only on
     // tiles meeting [PT, lo_max).
-    auto mask_phase = [&](int j, f32x16(&s)[2]) {
+    auto mask_phase = [&](int j, f32x16(&s)[NMB]) {
       if (j < w.jfull) return;
       const int kb = j * kKeyTile;
-      const int lim = qk - kb - 8 * hl;  // visible: rel <= lim
+      const int kw = kb + 32 * khalf;  // the wave's first key of the tile
+      const int lim = qk - kw - 8 * hl;  // visible: rel <= lim
       if (kb + kKeyTile > PT && kb < w.lo_max) {
-        const int g0 = PT - kb - 8 * hl, g1 = qlo - kb - 8 * hl;  // hidden: g0 <= rel < g1
+        const int g0 = PT - kw - 8 * hl, g1 = qlo - kw - 8 * hl;  // hidden: g0 <= rel < g1
 #pragma unroll
-        for (int mb = 0; mb < 2; ++mb)
+        for (int mb = 0; mb < NMB; ++mb)
 #pragma unroll
           for (int r = 0; r < 16; ++r) {
             const int rel = 32 * mb + 16 * (r >> 3) + (r & 7);
@@ -1007,7 +1037,7 @@ void tree_attn_kernel(const KParams args) {
           }
       } else {
 #pragma unroll
-        for (int mb = 0; mb < 2; ++mb)
+        for (int mb = 0; mb < NMB; ++mb)
 #pragma unroll
           for (int r = 0; r < 16; ++r) {
             const int rel = 32 * mb + 16 * (r >> 3) + (r & 7);
@@ -1019,13 +1049,13 @@ void tree_attn_kernel(const KParams args) {
     // tile that holds both prefix-cache and new keys: the prefix keys' scores
     // are brought to the new keys' k scale, and the tile then uses c_new.
     auto tile_c = [&](int j) __attribute__((always_inline)) { return j * kKeyTile + kKeyTile <= P ? c_past : c_new; };
-    auto fix_straddle = [&](int j, f32x16(&s)[2]) __attribute__((always_inline)) {
+    auto fix_straddle = [&](int j, f32x16(&s)[NMB]) __attribute__((always_inline)) {
       const int kb = j * kKeyTile;
       if (c_past == c_new || !(kb < P && kb + kKeyTile > P)) return;
       const float ratio = c_past / c_new;
-      const int lim = P - kb - 8 * hl;  // prefix key: rel < lim
+      const int lim = P - kb - 32 * khalf - 8 * hl;  // prefix key: rel < lim
 #pragma unroll
-      for (int mb = 0; mb < 2; ++mb)
+      for (int mb = 0; mb < NMB; ++mb)
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
           const int rel = 32 * mb + 16 * (r >> 3) + (r & 7);
@@ -1047,9 +1077,14 @@ void tree_attn_kernel(const KParams args) {
     // both keep the same m.
     // max S over the lane's 32 keys: a tree of three-input maxima (v_max3_f32,
     // two values per instruction): 32 -> 12 -> 4 -> 1 in 16 instructions.
-    auto lane_max = [&](const f32x16(&s)[2]) __attribute__((always_inline)) {
+    auto lane_max = [&](const f32x16(&s)[NMB]) __attribute__((always_inline)) {
       auto e = [&](int i) __attribute__((always_inline)) { return s[i >> 4][i & 15]; };
       auto max3 = [](float a, float b, float c) __attribute__((always_inline)) { return fmaxf(fmaxf(a, b), c); };
+      if constexpr (NMB == 1) {
+        const float a0 = max3(e(0), e(1), e(2)), a1 = max3(e(3), e(4), e(5)), a2 = max3(e(6), e(7), e(8));
+        const float a3 = max3(e(9), e(10), e(11)), a4 = max3(e(12), e(13), e(14));
+        return fmaxf(max3(a0, a1, a2), max3(a3, a4, e(15)));
+      } else {
       float m12[12];
 #pragma unroll
       for (int i = 0; i < 10; ++i) m12[i] = max3(e(3 * i), e(3 * i + 1), e(3 * i + 2));
@@ -1059,14 +1094,15 @@ void tree_attn_kernel(const KParams args) {
 #pragma unroll
       for (int i = 0; i < 4; ++i) m4[i] = max3(m12[3 * i], m12[3 * i + 1], m12[3 * i + 2]);
       return fmaxf(max3(m4[0], m4[1], m4[2]), m4[3]);
+      }
     };
-    auto s_max = [&](const f32x16(&s)[2]) __attribute__((always_inline)) {  // max S over the query's keys
+    auto s_max = [&](const f32x16(&s)[NMB]) __attribute__((always_inline)) {  // max S over the query's keys
       const LanePair mp = lane_pair(lane_max(s));
       return fmaxf(mp.self, mp.other);
     };
-    auto exp_phase = [&](const f32x16(&s)[2], float c) __attribute__((always_inline)) {
+    auto exp_phase = [&](const f32x16(&s)[NMB], float c) __attribute__((always_inline)) {
 #pragma unroll
-      for (int mb = 0; mb < 2; ++mb) {
+      for (int mb = 0; mb < NMB; ++mb) {
         f32x8 x0, x1;
 #pragma unroll
         for (int r = 0; r < 8; ++r) {
@@ -1076,16 +1112,17 @@ void tree_attn_kernel(const KParams args) {
         pf[2 * mb] = pack8<_Float16>(x0);
         pf[2 * mb + 1] = pack8<_Float16>(x1);
       }
-      float acc[4];
+      float acc[2 * NMB];
 #pragma unroll
-      for (int kj = 0; kj < 4; ++kj) {  // four short chains instead of one long one
+      for (int kj = 0; kj < 2 * NMB; ++kj) {  // short chains instead of one long one
         const f16x8 h = __builtin_bit_cast(f16x8, pf[kj]);
         acc[kj] = __builtin_amdgcn_fdot2(__builtin_shufflevector(h, h, 0, 1), kOnes2, 0.f, false);
         acc[kj] = __builtin_amdgcn_fdot2(__builtin_shufflevector(h, h, 2, 3), kOnes2, acc[kj], false);
         acc[kj] = __builtin_amdgcn_fdot2(__builtin_shufflevector(h, h, 4, 5), kOnes2, acc[kj], false);
         acc[kj] = __builtin_amdgcn_fdot2(__builtin_shufflevector(h, h, 6, 7), kOnes2, acc[kj], false);
       }
-      return (acc[0] + acc[1]) + (acc[2] + acc[3]);
+      if constexpr (NMB == 1) return acc[0] + acc[1];
+      else return (acc[0] + acc[1]) + (acc[2] + acc[3]);
     };
     // Before a tile's softmax: raise m to the tile's max if some score would
     // put p above 2^kLog2Limit, and bring O to the scale of the tile's V^T
@@ -1094,7 +1131,7 @@ void tree_attn_kernel(const KParams args) {
     // Without the check (kCheck false) no score raises m: a p that overflows
     // fp16 becomes inf, which the row sum carries to the unit's end, where
     // the work group then runs the unit again with the check (see the vote).
-    auto begin_tile = [&](bool chk, const f32x16(&s)[2], float c, int ve) __attribute__((always_inline)) {
+    auto begin_tile = [&](bool chk, const f32x16(&s)[NMB], float c, int ve) __attribute__((always_inline)) {
       bool raise = false;
       if (chk) raise = __any(!(fmaf(lane_max(s), c, mneg) <= kLog2Limit));
       if (raise || ve != vE) {
@@ -1117,7 +1154,7 @@ void tree_attn_kernel(const KParams args) {
     auto pv_phase = [&](int b) __attribute__((always_inline)) {
       const uint8_t *vbuf = smem + b * L::buf + v_lane;
 #pragma unroll
-      for (int kj = 0; kj < 4; ++kj) {
+      for (int kj = 0; kj < 2 * NMB; ++kj) {
 #pragma unroll
         for (int db = 0; db < ND; ++db) {
           const u32x4 a = *reinterpret_cast<const u32x4 *>(vbuf + (kj * ND + db) * 1024);
@@ -1349,7 +1386,7 @@ void tree_attn_kernel(const KParams args) {
       // Every wave has read the previous pass's vote: its word is the next
       // pass's, cleared now.
       if (tid == 0) vote_word(pass + 1) = 0u;
-      f32x16 sc[2];  // S of the current tile
+      f32x16 sc[NMB];  // S of the current tile
       // The running max m starts at the largest visible score of the first
       // tile (exact, so that tile's largest p is 1). A query that sees no key
       // of the first tile (only when the segment has neither past nor trunk)
@@ -1372,7 +1409,7 @@ void tree_attn_kernel(const KParams args) {
       // unit's first tiles) is issued into the buffer that tile it-1 used:
       // every wave has finished tile it-1 before the barrier.
       int it = 0;
-      auto step = [&](auto last, f32x16(&s)[2]) {
+      auto step = [&](auto last, f32x16(&s)[NMB]) {
         constexpr bool kLast = decltype(last)::value;
         if (!kLast && wave < kIssuers) {
           if (issued_cat(it + 2)) wait_vmem<SLOTS>();  // tile it+1 landed; it+2 may be in flight
@@ -1436,8 +1473,54 @@ void tree_attn_kernel(const KParams args) {
       // r4 of block db holds d = 32 db + 8 r4 + 4 hl + (0..3); lanes l and
       // l ^ 32 (the same query) trade halves so that each stores 8 contiguous
       // d: lane hl = 0 the even groups, hl = 1 the odd ones.
-      const float l = lsum + __shfl_xor(lsum, 32);
-      const float linv = l > 0.f ? exp2i(vE) / l : 0.f;
+      float l = lsum + __shfl_xor(lsum, 32);
+      if constexpr (KH == 2) {
+        // Merge the halves: the waves of keys 32-63 hand m, l, the V scale and
+        // O (kRound d blocks at a time) to their partners over LDS, past the
+        // ring, whose buffers may hold the next unit's tiles already.
+        constexpr int kRound = Merge<D, (int)sizeof(TQK)>::blocks;
+        const uint32_t stat = smem_lds + (uint32_t)Merge<D, (int)sizeof(TQK)>::stat + (uint32_t)((wave & 3) * 768 + lane * 4);
+        const uint32_t part = smem_lds + (uint32_t)Merge<D, (int)sizeof(TQK)>::part + (uint32_t)((wave & 3) * kRound * 4096 + lane * 16);
+        auto word = [&](uint32_t at) __attribute__((always_inline)) -> DAN_LDS float & { return *(DAN_LDS float *)(uintptr_t)at; };
+        if (khalf == 1) {
+          word(stat) = -mneg;
+          word(stat + 256) = l;
+          word(stat + 512) = exp2i(vE);
+        }
+        float f0 = 0.f, f1 = 0.f;
+#pragma unroll
+        for (int d0 = 0; d0 < ND; d0 += kRound) {
+          if (khalf == 1) {
+#pragma unroll
+            for (int b = 0; b < kRound; ++b)
+#pragma unroll
+              for (int i = 0; i < 4; ++i) {
+                const f32x16 &x = o[d0 + b];
+                *(DAN_LDS f32x4 *)(uintptr_t)(part + (uint32_t)(b * 4096 + i * 1024)) = f32x4{x[4 * i], x[4 * i + 1], x[4 * i + 2], x[4 * i + 3]};
+              }
+          }
+          barrier_lds();
+          if (khalf == 0) {
+            if (d0 == 0) {
+              const float m0 = -mneg, m1 = word(stat), m = fmaxf(m0, m1);
+              const float e0 = __builtin_amdgcn_exp2f(m0 - m), e1 = __builtin_amdgcn_exp2f(m1 - m);
+              const float lm = l * e0 + word(stat + 256) * e1, inv = lm > 0.f ? 1.0f / lm : 0.f;
+              f0 = e0 * exp2i(vE) * inv;
+              f1 = e1 * word(stat + 512) * inv;
+            }
+#pragma unroll
+            for (int b = 0; b < kRound; ++b)
+#pragma unroll
+              for (int i = 0; i < 4; ++i) {
+                const f32x4 y = *(const DAN_LDS f32x4 *)(uintptr_t)(part + (uint32_t)(b * 4096 + i * 1024));
+#pragma unroll
+                for (int e = 0; e < 4; ++e) o[d0 + b][4 * i + e] = o[d0 + b][4 * i + e] * f0 + y[e] * f1;
+              }
+          }
+          if (d0 + kRound < ND) barrier_lds();  // the last round's reads end before the next unit's first barrier
+        }
+      }
+      const float linv = KH == 2 ? 1.0f : l > 0.f ? exp2i(vE) / l : 0.f;
       TOut *orow = static_cast<TOut *>(p.o) + (int64_t)(cur.start + ql) * p.o_st + (int64_t)head * p.o_sh;
   #pragma unroll
       for (int db = 0; db < ND; ++db)
@@ -1453,7 +1536,7 @@ void tree_attn_kernel(const KParams args) {
             first.w[w4] = sw[0];
             second.w[w4] = sw[1];
           }
-          if (qvalid) store8<TOut>(orow + 32 * db + 8 * (2 * jp + hl), first, second);
+          if (qvalid && khalf == 0) store8<TOut>(orow + 32 * db + 8 * (2 * jp + hl), first, second);
         }
     }
     gbase += ntile;
@@ -1589,15 +1672,22 @@ hipError_t launch_pack(const PackParams &pp, int blocks, hipStream_t stream) {
   return hipGetLastError();
 }
 
-template <typename TQK, typename TOut, int D>
-hipError_t launch_attn(const KParams &kp, int grid, hipStream_t stream) {
-  auto kernel = tree_attn_kernel<TQK, TOut, D>;
-  constexpr int lds = Lds<D, (int)sizeof(TQK)>::total + kVoteBytes;
+template <typename TQK, typename TOut, int D, int KH>
+hipError_t launch_attn_halves(const KParams &kp, int grid, hipStream_t stream) {
+  auto kernel = tree_attn_kernel<TQK, TOut, D, KH>;
+  constexpr int lds = KH == 2 ? Merge<D, (int)sizeof(TQK)>::total : Lds<D, (int)sizeof(TQK)>::total + kVoteBytes;
   static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void *>(kernel),
                                                      hipFuncAttributeMaxDynamicSharedMemorySize, lds);
   if (attr != hipSuccess) return attr;
   hipLaunchKernelGGL(kernel, dim3(grid), dim3(Shape<D>::threads), lds, stream, kp);
   return hipGetLastError();
+}
+
+template <typename TQK, typename TOut, int D>
+hipError_t launch_attn(const KParams &kp, int grid, bool halves, hipStream_t stream) {
+  if constexpr (D <= 128)
+    if (halves) return launch_attn_halves<TQK, TOut, D, 2>(kp, grid, stream);
+  return launch_attn_halves<TQK, TOut, D, 1>(kp, grid, stream);
 }
 
 }  // namespace dan
@@ -1637,7 +1727,11 @@ int dan_tree_attn_fwd(const DanTreeAttnArgs *a, void *stream) {
   if (D != 64 && D != 128 && D != 256) return fail(DAN_ERR_UNSUPPORTED, "head_dim %d: only 64, 128 and 256 are built", D);
   const int rep = H / Hkv;
   const int tq = dan_tree_attn_tile_q(H, Hkv, D);
-  if (a->tile_q != tq) return fail(DAN_ERR_INVALID_ARGUMENT, "tile_q %d, the kernel needs %d", a->tile_q, tq);
+  if (a->key_halves < 0 || a->key_halves > 2 || (a->key_halves == 2 && D > 128))
+    return fail(DAN_ERR_INVALID_ARGUMENT, "key_halves %d: 0 or 1, or 2 up to head_dim 128", a->key_halves);
+  const bool halves = a->key_halves == 2;
+  if (a->tile_q != (halves ? tq / 2 : tq))
+    return fail(DAN_ERR_INVALID_ARGUMENT, "tile_q %d, the kernel needs %d", a->tile_q, halves ? tq / 2 : tq);
   const int in = a->in_dtype, vd = a->v_dtype, out = a->out_dtype;
   const bool bf16 = in == DAN_DTYPE_BF16 && vd == DAN_DTYPE_BF16 && out == DAN_DTYPE_BF16;
   const bool f16 = in == DAN_DTYPE_F16 && vd == DAN_DTYPE_F16 && out == DAN_DTYPE_F16;
@@ -1720,9 +1814,9 @@ int dan_tree_attn_fwd(const DanTreeAttnArgs *a, void *stream) {
 #define DAN_PACK(TV) by_d([&] { return launch_pack<TV, 64>(pp, (int)pack_grid, s); }, \
                           [&] { return launch_pack<TV, 128>(pp, (int)pack_grid, s); }, \
                           [&] { return launch_pack<TV, 256>(pp, (int)pack_grid, s); })
-#define DAN_ATTN(TQK, TO) by_d([&] { return launch_attn<TQK, TO, 64>(kp, grid, s); }, \
-                               [&] { return launch_attn<TQK, TO, 128>(kp, grid, s); }, \
-                               [&] { return launch_attn<TQK, TO, 256>(kp, grid, s); })
+#define DAN_ATTN(TQK, TO) by_d([&] { return launch_attn<TQK, TO, 64>(kp, grid, halves, s); }, \
+                               [&] { return launch_attn<TQK, TO, 128>(kp, grid, halves, s); }, \
+                               [&] { return launch_attn<TQK, TO, 256>(kp, grid, halves, s); })
   hipError_t err = hipSuccess;
   if (a->phases != DAN_TREE_ATTN_PHASE_ATTEND) {
     if (bf16) err = DAN_PACK(__bf16);

@@ -162,7 +162,7 @@ typedef struct {
    * its branch); 0 for trunk tokens. Key kc is visible to query qc iff
    *   kc <= qc  and  (kc < P + trunk  or  kc >= key_lo[query]). */
   const int32_t *key_lo;
-  int32_t tile_q; /* queries per work item; must equal dan_tree_attn_tile_q() */
+  int32_t tile_q; /* queries per work item: dan_tree_attn_tile_q(), half of it with key_halves = 2 */
   int32_t vt_cols; /* columns of the V^T copy: sum over segments of roundup(past_len + n) */
   /* [vt_cols / DAN_TREE_ATTN_KEY_TILE]: the segment owning each column block */
   const int32_t *col_seg;
@@ -206,6 +206,10 @@ typedef struct {
    * caller uploads no table. Read during the call only; unused by
    * DAN_TREE_ATTN_PHASE_ATTEND, which reads the table the copy wrote. */
   const DanPastDesc *pasts_host;
+  /* (ABI 9) 0 or 1; or 2 (head_dim <= 128): work items of half as many
+   * queries, whose key tiles the two halves of a work group's waves split --
+   * the faster form for a batch of at most half as many units as CUs. */
+  int32_t key_halves;
 } DanTreeAttnArgs;
 
 #define DAN_TREE_ATTN_INLINE_PASTS 8
