@@ -173,7 +173,7 @@ class DanGdnNormArgs(ctypes.Structure):
                 ("out", _vp), ("out_stride", _i64)]
 
 
-EXPORTS = ("dan_tree_attn_fwd", "dan_tree_attn_fwd_noalloc", "dan_tree_attn_stage_f16", "dan_tree_attn_tile_q", "dan_tree_attn_head_groups", "dan_tree_attn_workspace_size",
+EXPORTS = ("dan_tree_attn_fwd", "dan_tree_attn_fwd_noalloc", "dan_tree_attn_stage_f16", "dan_tree_attn_stage_f16_pair", "dan_tree_attn_tile_q", "dan_tree_attn_head_groups", "dan_tree_attn_workspace_size",
            "dan_tree_attn_last_error", "dan_tree_attn_abi_version", "dan_qkv_front", "dan_qkv_front_abi_version",
            "dan_tree_attn_plan", "dan_tree_attn_plan_slots", "dan_tree_attn_plan_abi_version",
            "dan_fp8_quantize", "dan_fp8_gemm", "dan_fp8_tiled_bytes", "dan_fp8_abi_version", "dan_gdn_fwd", "dan_gdn_workspace_size", "dan_gdn_abi_version",
@@ -201,6 +201,8 @@ def load(path=LIB_PATH):
         lib.dan_tree_attn_fwd_noalloc.restype = ctypes.c_int
         lib.dan_tree_attn_stage_f16.argtypes = [ctypes.POINTER(DanStageF16Args), _vp]
         lib.dan_tree_attn_stage_f16.restype = ctypes.c_int
+        lib.dan_tree_attn_stage_f16_pair.argtypes = [ctypes.POINTER(DanStageF16Args), ctypes.POINTER(DanStageF16Args), _vp]
+        lib.dan_tree_attn_stage_f16_pair.restype = ctypes.c_int
         lib.dan_tree_attn_tile_q.argtypes = [_i32, _i32, _i32]
         lib.dan_tree_attn_tile_q.restype = ctypes.c_int
         lib.dan_tree_attn_head_groups.argtypes = [_i32, _i32]
@@ -276,6 +278,14 @@ def stage_f16(args, stream, lib=None):
     rc = lib.dan_tree_attn_stage_f16(ctypes.byref(args), _vp(stream))
     if rc != OK:
         raise RuntimeError(f"dan_tree_attn_stage_f16 failed (status {rc}): {last_error(lib)}")
+
+
+def stage_f16_pair(first, second, stream, lib=None):
+    """Launch the fp32 -> fp16 staging of two tensors; raises RuntimeError on failure."""
+    lib = lib or load()
+    rc = lib.dan_tree_attn_stage_f16_pair(ctypes.byref(first), ctypes.byref(second), _vp(stream))
+    if rc != OK:
+        raise RuntimeError(f"dan_tree_attn_stage_f16_pair failed (status {rc}): {last_error(lib)}")
 
 
 def forward(args, stream, lib=None):

@@ -244,21 +244,34 @@ def _qk_dtype(dtype):
     return torch.float16 if dtype == torch.float32 else dtype
 
 
-def _stage_f16(x):
-    """fp32 [d0, d1, d2] -> (fp16 copy, scale) with x = copy * scale, scale a
-    power of 2 that keeps the copy within fp16's range
-    (``dan_tree_attn_stage_f16``, two launches on the current stream)."""
+def _stage_args(x):
+    """``DanStageF16Args`` of fp32 x [d0, d1, d2], its fp16 copy, its scale and
+    the tensors the arguments point at."""
     x = _kernel_view(x)
     out = torch.empty(x.shape, dtype=torch.float16, device=x.device)
     scratch = torch.empty(1 + _native.STAGE_PARTIALS, dtype=torch.float32, device=x.device)  # scale, then the partials
-    scale, partial = scratch[:1], scratch[1:]
     a = _native.DanStageF16Args()
     a.abi_version = _native.ABI_VERSION
     a.d0, a.d1, a.d2 = x.shape
     a.x, a.stride0, a.stride1 = x.data_ptr(), x.stride(0), x.stride(1)
-    a.out, a.scale, a.partial = out.data_ptr(), scale.data_ptr(), partial.data_ptr()
-    _native.stage_f16(a, torch.cuda.current_stream(x.device).cuda_stream)
+    a.out, a.scale, a.partial = out.data_ptr(), scratch.data_ptr(), scratch.data_ptr() + 4
+    return a, out, scratch[:1], x
+
+
+def _stage_f16(x):
+    """fp32 [d0, d1, d2] -> (fp16 copy, scale) with x = copy * scale, scale a
+    power of 2 that keeps the copy within fp16's range
+    (``dan_tree_attn_stage_f16``, two launches on the current stream)."""
+    a, out, scale, _x = _stage_args(x)
+    _native.stage_f16(a, torch.cuda.current_stream(out.device).cuda_stream)
     return out, scale
+
+
+def _stage_f16_pair(q, k):
+    """``_stage_f16`` of q and of k through one pair of launches."""
+    (a, qo, qs, _q), (b, ko, ks, _k) = _stage_args(q), _stage_args(k)
+    _native.stage_f16_pair(a, b, torch.cuda.current_stream(qo.device).cuda_stream)
+    return (qo, qs), (ko, ks)
 
 
 def _past_table(plan, layer, hkv, d, dtype, device, upload=True):
@@ -408,7 +421,7 @@ def _call_args(q, k, v, segments, layer, scale, fp8_scales, phases, noalloc, upl
         q_scale, k_scale, v_scale = (_check_scale(t, nm, q.device) for t, nm in zip(fp8_scales, ("q_scale", "k_scale", "v_scale")))
     scales = [q_scale, k_scale, v_scale] if q.dtype == E4M3 else []
     if q.dtype == torch.float32:  # fp16 for the matrix core, with power-of-2 scales
-        (q, q_scale), (k, k_scale) = _stage_f16(q), _stage_f16(k)
+        (q, q_scale), (k, k_scale) = _stage_f16_pair(q, k)
         scales = [q_scale, k_scale]
     q, k, v = _kernel_view(q), _kernel_view(k), _kernel_view(v)
     units, sched_off, slots = plan.schedule(groups, _num_cus(q.device)) if plan.num_work else (None, None, 0)
@@ -662,7 +675,7 @@ class BudgetPlan:
             scales = [_check_scale(t, nm, q.device) for t, nm in
                       zip((q_scale, k_scale, v_scale), ("q_scale", "k_scale", "v_scale"))]
         if q.dtype == torch.float32:
-            (q, qs), (k, ks) = _stage_f16(q), _stage_f16(k)
+            (q, qs), (k, ks) = _stage_f16_pair(q, k)
             scales = [qs, ks]
         q, k, v = _kernel_view(q), _kernel_view(k), _kernel_view(v)
         tables = [self.segs_d, self.work, self.key_lo, self.col_seg, self._table(layer), self.units, self.sched_off,

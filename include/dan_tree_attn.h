@@ -247,6 +247,10 @@ typedef struct {
 
 int dan_tree_attn_stage_f16(const DanStageF16Args *args, void *stream);
 
+/* Two tensors (q and k), each with its own arguments and scale, through one
+ * pair of launches; the same results. (ABI 9) */
+int dan_tree_attn_stage_f16_pair(const DanStageF16Args *first, const DanStageF16Args *second, void *stream);
+
 /* Capacity in bytes of the library's own V^T scratch (one per GPU). */
 #define DAN_TREE_ATTN_SCRATCH_BYTES (32LL << 20)
 
