@@ -24,11 +24,12 @@
 //                      to the chunk records of the workspace, T and A staged
 //                      in LDS for 16-byte stores.
 //   chunk_scan_bf16_kernel  (bf16 inputs) one work group per (run, value
-//                      head, 32 state columns), the state slice in LDS; the
-//                      run's chunks in order, each the five products above on
-//                      v_mfma_f32_16x16x32_bf16, fp32 operands as bf16 pairs
-//                      (hi + lo, ~16 significant bits) against an fp32 master
-//                      copy of the state; q, k and v read in place.
+//                      head, 32 or 16 state columns), the state slice in the
+//                      waves' registers; the run's chunks in order, each the
+//                      five products above on v_mfma_f32_16x16x32_bf16, fp32
+//                      operands as bf16 pairs (hi + lo, ~16 significant bits)
+//                      against an fp32 master copy of the state; q, k and v
+//                      read in place.
 //   chunk_scan_kernel  (fp16 inputs) the same on v_mfma_f32_16x16x4_f32 (fp32
 //                      operands), 16 state columns per work group for long
 //                      runs, 32 for many short ones.
@@ -50,15 +51,18 @@ namespace dan_gdnc {
 constexpr int kC = DAN_GDN_CHUNK;  // tokens per chunk
 constexpr int kDk = 128;
 constexpr int kThreads = 256;
-// State columns per scan work group (a template argument of the scan: 32 or
-// 16) for phases of long and of short runs.
+// State columns per work group of the fp32 scan (a template argument of it: 32
+// or 16) for phases of long and of short runs.
 constexpr int kLongCols = 16, kShortCols = 32;
 // Chunk record per (slot, value head), two layouts:
 // - fp16 inputs (the fp32 scan): T [64][64] and A [64][64] in fp32, then the
 //   five rows of 64 floats below, at float kVecF32;
 // - bf16 inputs (the bf16 scan): T and A as bf16 pairs (hi = bf16(x), lo =
-//   bf16(x - hi): x to ~16 significant bits), each [64][64] row-major, then
-//   K^T [128][64] bf16 (exact), then the five rows at float kVecBf.
+//   bf16(x - hi): x to ~16 significant bits), 64 x 64 each, then K^T 128 x 64
+//   bf16 (exact), then the five rows at float kVecBf. The matrices lie as the
+//   scan's operand fragments, 16 rows x 32 columns in 1 KB each: lane
+//   l16 + 16 g4's 16 bytes hold row l16, columns 8 g4 .. + 7, so an operand load
+//   is 1 KB of contiguous memory (frag_at).
 // The five rows: beta gamma r_k, beta, r_q Dk^-1/2 gamma, exp(G_63 - G) r_k,
 // {gamma_63, 0, ..}.
 constexpr int kVecF32 = 2 * kC * kC;
@@ -67,6 +71,9 @@ constexpr int kRec = kVecBf + 5 * kC;  // floats; the fp32 layout uses the first
 // bf16 layout: byte offsets of T hi / lo, A hi / lo and K^T.
 constexpr int kThiB = 0, kTloB = kC * kC * 2, kAhiB = 2 * kC * kC * 2, kAloB = 3 * kC * kC * 2, kKtB = 4 * kC * kC * 2;
 constexpr float kQs = 0.08838834764831845f;  // Dk^-1/2
+
+// Byte of the 16-byte piece (row, columns 8 c8 .. + 7) of a 64-column bf16 matrix in fragment order.
+__device__ inline int frag_at(int row, int c8) { return ((row >> 4) * 2 + (c8 >> 2)) * 1024 + ((c8 & 3) * 16 + (row & 15)) * 16; }
 
 #define DAN_GLOBAL __attribute__((address_space(1)))
 
@@ -77,6 +84,14 @@ typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
+
+// The bf16 scan takes 16 state columns per work group while that makes at most
+// one group per CU, else 32. A chunk's step of 16 columns is the shorter, but
+// two groups on a CU take longer than one of twice the columns. The whole rule
+// (16 value heads of 128 columns, microseconds at 16 / 32 columns): 4 runs of
+// 1000 tokens 82.9 / 71.0, 8 of 800 128.8 / 96.4, 45 branches of 16-96 108.9 /
+// 80.7, 150 of 1-200 499 / 356; with one group per CU 2 runs of 1000 take 53.1 / 61.7.
+constexpr int kScan16Groups = 256;
 
 struct Params {
   const int32_t *cu;
@@ -290,11 +305,11 @@ __global__ __launch_bounds__(kThreads) void chunk_prep_kernel(const Params p) {
     QK = mfma_in<T>(aq, bb, QK);
   }
   if constexpr (kBf) {
-    // K^T [Dk][kC] for the bf16 scan: thread t writes d rows 2 dp and 2 dp + 1,
+    // K^T for the bf16 scan: thread t writes d rows 2 dp and 2 dp + 1,
     // tokens 8 oc .. 8 oc + 7, from 8 dwords (d 2 dp, 2 dp + 1) of 8 tile rows.
 #pragma unroll
     for (int n = 0; n < 2; ++n) {
-      const int dp = (tid >> 3) + 32 * n, oc = tid & 7;
+      const int dp = tid & 63, oc = (tid >> 6) + 4 * n;
       uint32_t w[8];
 #pragma unroll
       for (int e = 0; e < 8; ++e) w[e] = *reinterpret_cast<const uint32_t *>(sKt + (8 * oc + e) * kTileRow + 4 * dp);
@@ -304,8 +319,8 @@ __global__ __launch_bounds__(kThreads) void chunk_prep_kernel(const Params p) {
         lo[e] = (w[2 * e] & 0xffffu) | (w[2 * e + 1] << 16);
         hi[e] = (w[2 * e] >> 16) | (w[2 * e + 1] & 0xffff0000u);
       }
-      *(DAN_GLOBAL u32x4 *)(recb + kKtB + 2 * ((2 * dp) * kC + 8 * oc)) = lo;
-      *(DAN_GLOBAL u32x4 *)(recb + kKtB + 2 * ((2 * dp + 1) * kC + 8 * oc)) = hi;
+      *(DAN_GLOBAL u32x4 *)(recb + kKtB + frag_at(2 * dp, oc)) = lo;
+      *(DAN_GLOBAL u32x4 *)(recb + kKtB + frag_at(2 * dp + 1, oc)) = hi;
     }
   }
   barrier_lds();  // sG, the row factors; every read of the tiles is done
@@ -337,10 +352,17 @@ __global__ __launch_bounds__(kThreads) void chunk_prep_kernel(const Params p) {
   //    L[i][m] = 0 for m >= i, so whole groups of four are summed.
   constexpr int kBlockBytes = kC * kC * 4;  // the T block, then the A block, of the record
   static_assert(kAhiB == kBlockBytes && kThiB == 0, "record layout");
+  // The stage's byte that goes to byte `off` of the record's block: for bf16
+  // the hi and lo planes (row-major in the stage) in fragment order.
+  auto staged = [](int off) __attribute__((always_inline)) {
+    if (!kBf) return off;
+    const int f = off % (kC * kC * 2), lane = f / 16 % 64, fb = f / 1024;  // fragment fb: rows 16 (fb / 2), columns 32 (fb % 2)
+    return off - f + 2 * ((16 * (fb >> 1) + (lane & 15)) * kC + 32 * (fb & 1) + 8 * (lane >> 4));
+  };
 #pragma unroll
   for (int m = 0; m < kBlockBytes / (16 * kThreads); ++m) {
     const int off = 16 * (kThreads * m + tid);
-    *(DAN_GLOBAL u32x4 *)(recb + kBlockBytes + off) = *reinterpret_cast<const u32x4 *>(sKt + off);
+    *(DAN_GLOBAL u32x4 *)(recb + kBlockBytes + off) = *reinterpret_cast<const u32x4 *>(sKt + staged(off));
   }
   const int j = 16 * wave + (lane >> 2), part = lane & 3;
   float xm[kC / 4];  // x_{4 k + part}
@@ -368,7 +390,7 @@ __global__ __launch_bounds__(kThreads) void chunk_prep_kernel(const Params p) {
 #pragma unroll
   for (int m = 0; m < kBlockBytes / (16 * kThreads); ++m) {
     const int off = 16 * (kThreads * m + tid);
-    *(DAN_GLOBAL u32x4 *)(recb + off) = *reinterpret_cast<const u32x4 *>(sKt + off);
+    *(DAN_GLOBAL u32x4 *)(recb + off) = *reinterpret_cast<const u32x4 *>(sKt + staged(off));
   }
 }
 
@@ -650,55 +672,56 @@ __global__ __launch_bounds__(64 * W) void chunk_scan_kernel(const Params p) {
 // x lo term, ~2^-17 relative, is dropped). Sums stay fp32, and the state's
 // fp32 master copy carries the decay and the updates; the bf16 pairs of S are
 // rewritten from it every chunk.
-// LDS (bytes): the state's fp32 master [128][COLS + 2]; the state as bf16
-// planes (hi, lo) of [COLS][128 + 8] (one state column per row, so the B
-// operand's 8 consecutive state rows are 16 contiguous bytes); Y, D and
-// diag(exp(G_63 - G) r_k) D as planes of [COLS][64 + 8]. The 8-element pads
-// spread a B-operand read's 16 columns over the banks.
+// LDS (bytes): the state as bf16 planes (hi, lo) of [COLS][128 + 8] (one state
+// column per row, so the B operand's 8 consecutive state rows are 16
+// contiguous bytes); Y, D and diag(exp(G_63 - G) r_k) D as planes of
+// [COLS][64 + 8]; each wave's 16 rows of v. The 8-element pads spread a
+// B-operand read's 16 columns over the banks. The state's fp32 master stays in
+// registers: the lane that updates a state element is the one that reads it.
 template <int COLS>
 struct BfLds {
-  static constexpr int kSS = COLS + 2, kPS = kDk + 8, kPC = kC + 8;
-  static constexpr int sHi = kDk * kSS * 4, sLo = sHi + COLS * kPS * 2;
+  static constexpr int kPS = kDk + 8, kPC = kC + 8;
+  static constexpr int sHi = 0, sLo = sHi + COLS * kPS * 2;
   static constexpr int yHi = sLo + COLS * kPS * 2, yLo = yHi + COLS * kPC * 2;
   static constexpr int dHi = yLo + COLS * kPC * 2, dLo = dHi + COLS * kPC * 2;
   static constexpr int eHi = dLo + COLS * kPC * 2, eLo = eHi + COLS * kPC * 2;
-  static constexpr int bytes = eLo + COLS * kPC * 2;
+  static constexpr int vRows = eLo + COLS * kPC * 2, vWave = 16 * COLS * 2;
+  static constexpr int bytes = vRows + 4 * vWave;
   static_assert(sHi % 16 == 0 && (kPS * 2) % 16 == 0 && (kPC * 2) % 16 == 0, "16-byte operand reads");
 };
-
-// State columns per work group of the bf16 scan, long and short runs alike:
-// its per-chunk operands (q, k, T, A, K^T) are loaded by every column group
-// of a (run, head), and with 16 columns the CUs' address units were the
-// limit (trunk phase of 5 runs of 286 to 1843 tokens: 0.209 ms on 16
-// columns, 0.164 on 32, 0.226 on 64 with one group per CU).
-constexpr int kBfCols = 32;
 
 __device__ inline f32x4 mma_bf(u32x4 a, u32x4 b, f32x4 c) {
   return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
 }
-// x as a bf16 pair, the hi and lo halves' bits.
-__device__ inline void split_bf(float x, uint32_t &hi, uint32_t &lo) {
-  const __bf16 h = (__bf16)x;
-  const __bf16 l = (__bf16)(x - (float)h);
-  hi = __builtin_bit_cast(uint16_t, h);
-  lo = __builtin_bit_cast(uint16_t, l);
+// Two values as bf16 pairs: the packed hi halves and the packed lo halves.
+__device__ inline void split2_bf(float x0, float x1, uint32_t &hi, uint32_t &lo) {
+  typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+  typedef float f32x2 __attribute__((ext_vector_type(2)));
+  hi = __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2{x0, x1}), bf16x2));
+  const float h0 = __builtin_bit_cast(float, hi << 16), h1 = __builtin_bit_cast(float, hi & 0xffff0000u);
+  lo = __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2{x0 - h0, x1 - h1}), bf16x2));
 }
 // Four consecutive rows of one plane column (8 bytes, hi and lo planes).
 __device__ inline void put4_bf(uint8_t *hi_plane, uint8_t *lo_plane, int off, const f32x4 &x) {
-  uint32_t h[4], l[4];
-#pragma unroll
-  for (int i = 0; i < 4; ++i) split_bf(x[i], h[i], l[i]);
-  *reinterpret_cast<u32x2 *>(hi_plane + off) = u32x2{h[0] | (h[1] << 16), h[2] | (h[3] << 16)};
-  *reinterpret_cast<u32x2 *>(lo_plane + off) = u32x2{l[0] | (l[1] << 16), l[2] | (l[3] << 16)};
+  u32x2 h, l;
+  uint32_t a, b;
+  split2_bf(x[0], x[1], a, b);
+  h[0] = a; l[0] = b;
+  split2_bf(x[2], x[3], a, b);
+  h[1] = a; l[1] = b;
+  *reinterpret_cast<u32x2 *>(hi_plane + off) = h;
+  *reinterpret_cast<u32x2 *>(lo_plane + off) = l;
 }
 
 // One wave's operands of one chunk, loaded a chunk ahead (each group right
 // after its last use in the chunk before).
-template <int NC>
+template <int COLS>
 struct OpsBf {
-  u32x4 ka[4], qa[4];   // k, q row 16 rb + l16, d 32 j + 8 g4 .. + 7 (A operands of K S, Q S)
-  f32x4 va, vb, vq, vs; // the row factors of rows 16 rb + 4 g4 .. + 3
-  float vv[NC][4];      // v of those rows, the wave's columns
+  u32x4 ka[4], qa[4];   // k, q row 16 rb + l16, d 32 j + 8 g4 .. + 7
+  f32x4 va, vb, vs;     // the row factors of rows 16 rb + 4 g4 .. + 3
+  float vq;             // r_q Dk^-1/2 gamma of row 16 rb + l16
+  uint32_t v[COLS / 8]; // row 16 rb + lane / 4 of v, columns COLS / 4 (lane % 4) .. (kVec)
+  float vv[COLS / 16][4];  // v of rows 16 rb + 4 g4 .. + 3, columns 16 n + l16 (not kVec)
   u32x4 th[2], tl[2];   // T row 16 rb + l16, chunk rows 32 j + 8 g4 .. + 7 (hi, lo)
   u32x4 ah[2], al[2];   // A, the same
   u32x4 kt[2][2];       // K^T row 32 rb + 16 mb + l16, chunk rows 32 j + 8 g4 .. + 7
@@ -715,14 +738,28 @@ struct OpsBf {
 //            into the master and the S planes                           barrier
 // Padding rows (past the run) come out as zeros in Y, D and Ds (their row
 // factors are zero), so every wave runs every phase.
-template <int COLS>
+// The two output products are taken transposed (the planes as the A operand),
+// so that a lane holds four consecutive columns of one row: one 8-byte store
+// for four 2-byte ones. v comes as one load per lane of whole row pieces and is
+// turned through the wave's own LDS rows by transposing reads (lane 4 c + p of
+// 16 receives element p of the pieces that lanes c, c + 4, c + 8 and c + 12
+// address). kVec: v's and out's rows allow these accesses; else one element at
+// a time, as any alignment does.
+// A chain of chunk steps, bound by each step's issue and its three barriers,
+// not by memory. The step before had 32 more LDS accesses (the fp32 master lay
+// there), read the record in 16-byte pieces of different rows, stored 2 bytes
+// at a time and split one value at a time. The whole rule with its preparation
+// (16 value heads of 128 columns), before and now, microseconds: 1 run of 1462
+// tokens 98.1, 64.5; 5 of 286-1843 165.7, 130.8; 45 branches of 16-96 105.3,
+// 80.7. The state's products on four waves and the output's on four others: 73.0,
+// 125.0, 103.8, not taken.
+template <int COLS, bool kVec>
 __global__ __attribute__((amdgpu_flat_work_group_size(256, 256), amdgpu_waves_per_eu(2)))
 void chunk_scan_bf16_kernel(const Params p) {
   constexpr int NC = COLS / 16;
   using LB = BfLds<COLS>;
-  constexpr int kSS = LB::kSS, kPS = LB::kPS, kPC = LB::kPC;
+  constexpr int kPS = LB::kPS, kPC = LB::kPC;
   __shared__ __attribute__((aligned(16))) uint8_t lds[LB::bytes];
-  float *sS = reinterpret_cast<float *>(lds);
   const int b = blockIdx.x;
   const int u = (b / (8 * p.ncb)) * 8 + (b & 7), cb = (b >> 3) % p.ncb;
   if (u >= p.units) return;  // the whole group, before any barrier
@@ -732,37 +769,31 @@ void chunk_scan_bf16_kernel(const Params p) {
   const int col0 = COLS * cb;
   const int64_t sbase = ((int64_t)r * p.Hv + h) * kDk * p.Dv + col0;
   const int64_t sbase_in = ((int64_t)state_in_of(p, r) * p.Hv + h) * kDk * p.Dv + col0;
-  {  // the state slice: every load in flight before the first LDS write
-    constexpr int kSt = kDk * COLS / 256;
-    float sv[kSt];
+  // The state's fp32 master: rows 32 rb + 16 mb + 4 g4 + rr, column 16 n + l16.
+  f32x4 st[2][NC];
+  auto srow = [&](int mb) __attribute__((always_inline)) { return 32 * rb + 16 * mb + 4 * g4; };
 #pragma unroll
-    for (int m = 0; m < kSt; ++m) {
-      const int x = tid + 256 * m;
-      sv[m] = *(const DAN_GLOBAL float *)(p.s_in + sbase_in + (int64_t)(x / COLS) * p.Dv + x % COLS);
-    }
+  for (int mb = 0; mb < 2; ++mb)
 #pragma unroll
-    for (int m = 0; m < kSt; ++m) {
-      const int x = tid + 256 * m, row = x / COLS, c = x % COLS;
-      sS[row * kSS + c] = sv[m];
-      uint32_t hi, lo;
-      split_bf(sv[m], hi, lo);
-      *reinterpret_cast<uint16_t *>(lds + LB::sHi + 2 * (c * kPS + row)) = (uint16_t)hi;
-      *reinterpret_cast<uint16_t *>(lds + LB::sLo + 2 * (c * kPS + row)) = (uint16_t)lo;
-    }
-  }
+    for (int n = 0; n < NC; ++n)
+#pragma unroll
+      for (int rr = 0; rr < 4; ++rr) st[mb][n][rr] = *(const DAN_GLOBAL float *)(p.s_in + sbase_in + (int64_t)(srow(mb) + rr) * p.Dv + 16 * n + l16);
   const int row0 = *(const DAN_GLOBAL int32_t *)(p.cu + r), end = *(const DAN_GLOBAL int32_t *)(p.cu + r + 1);
   const __bf16 *qh = static_cast<const __bf16 *>(p.q) + (int64_t)hk * p.q_sh;
   const __bf16 *kh = static_cast<const __bf16 *>(p.k) + (int64_t)hk * p.k_sh;
   const __bf16 *vh = static_cast<const __bf16 *>(p.v) + (int64_t)h * p.v_sh + col0;
   __bf16 *oh = static_cast<__bf16 *>(p.o) + (int64_t)h * p.o_sh + col0 + (int64_t)out_shift(p, r, row0, end) * p.o_st;
-  const int ri = 16 * rb + l16;     // the A-operand row of the 64-row products
-  const int ro = 16 * rb + 4 * g4;  // the first of the lane's accumulator rows
+  const int ri = 16 * rb + l16;     // the row of the lane's 64-row operands and of its outputs
+  const int ro = 16 * rb + 4 * g4;  // the first of the lane's accumulator rows (Y, D)
 
   auto recb = [&](int s) __attribute__((always_inline)) {
     return reinterpret_cast<const uint8_t *>(p.rec + ((int64_t)s * p.Hv + h) * kRec);
   };
-  auto ld16 = [&](const uint8_t *q) __attribute__((always_inline)) { return *(const DAN_GLOBAL u32x4 *)q; };
-  auto load0 = [&](OpsBf<NC> &o, int t0, int s) __attribute__((always_inline)) {
+  // fragment f (16 rows x 32 columns) of the record's matrix at byte `at`
+  auto ldf = [&](const uint8_t *rc, int at, int f) __attribute__((always_inline)) {
+    return *(const DAN_GLOBAL u32x4 *)(rc + at + f * 1024 + lane * 16);
+  };
+  auto load0 = [&](OpsBf<COLS> &o, int t0, int s) __attribute__((always_inline)) {
     const int L = min(kC, end - t0);
     const int64_t tr = t0 + min(ri, L - 1);
     const float *vec = reinterpret_cast<const float *>(recb(s)) + kVecBf;
@@ -772,34 +803,41 @@ void chunk_scan_bf16_kernel(const Params p) {
     for (int j = 0; j < 4; ++j) o.qa[j] = *(const DAN_GLOBAL u32x4 *)(qh + tr * p.q_st + 32 * j + 8 * g4);
     o.va = *(const DAN_GLOBAL f32x4 *)(vec + 0 * kC + ro);
     o.vb = *(const DAN_GLOBAL f32x4 *)(vec + 1 * kC + ro);
+    if constexpr (kVec) {
+      typedef uint32_t piece __attribute__((ext_vector_type(COLS / 8)));
+      const piece x = *(const DAN_GLOBAL piece *)(vh + (int64_t)(t0 + min(16 * rb + (lane >> 2), L - 1)) * p.v_st + COLS / 4 * (lane & 3));
 #pragma unroll
-    for (int n = 0; n < NC; ++n)
+      for (int i = 0; i < COLS / 8; ++i) o.v[i] = x[i];
+    } else {
 #pragma unroll
-      for (int rr = 0; rr < 4; ++rr)
-        o.vv[n][rr] = (float)*(const DAN_GLOBAL __bf16 *)(vh + (int64_t)(t0 + min(ro + rr, L - 1)) * p.v_st + 16 * n + l16);
+      for (int n = 0; n < NC; ++n)
+#pragma unroll
+        for (int rr = 0; rr < 4; ++rr)
+          o.vv[n][rr] = (float)*(const DAN_GLOBAL __bf16 *)(vh + (int64_t)(t0 + min(ro + rr, L - 1)) * p.v_st + 16 * n + l16);
+    }
   };
-  auto load1 = [&](OpsBf<NC> &o, int s) __attribute__((always_inline)) {
+  auto load1 = [&](OpsBf<COLS> &o, int s) __attribute__((always_inline)) {
     const uint8_t *rc = recb(s);
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
-      o.th[j] = ld16(rc + kThiB + 2 * (ri * kC + 32 * j + 8 * g4));
-      o.tl[j] = ld16(rc + kTloB + 2 * (ri * kC + 32 * j + 8 * g4));
+      o.th[j] = ldf(rc, kThiB, 2 * rb + j);
+      o.tl[j] = ldf(rc, kTloB, 2 * rb + j);
     }
     o.vs = *(const DAN_GLOBAL f32x4 *)(reinterpret_cast<const float *>(rc) + kVecBf + 3 * kC + ro);
   };
-  auto load2 = [&](OpsBf<NC> &o, int s) __attribute__((always_inline)) {
+  auto load2 = [&](OpsBf<COLS> &o, int s) __attribute__((always_inline)) {
     const uint8_t *rc = recb(s);
     const float *vec = reinterpret_cast<const float *>(rc) + kVecBf;
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
-      o.ah[j] = ld16(rc + kAhiB + 2 * (ri * kC + 32 * j + 8 * g4));
-      o.al[j] = ld16(rc + kAloB + 2 * (ri * kC + 32 * j + 8 * g4));
+      o.ah[j] = ldf(rc, kAhiB, 2 * rb + j);
+      o.al[j] = ldf(rc, kAloB, 2 * rb + j);
     }
 #pragma unroll
     for (int mb = 0; mb < 2; ++mb)
 #pragma unroll
-      for (int j = 0; j < 2; ++j) o.kt[mb][j] = ld16(rc + kKtB + 2 * ((32 * rb + 16 * mb + l16) * kC + 32 * j + 8 * g4));
-    o.vq = *(const DAN_GLOBAL f32x4 *)(vec + 2 * kC + ro);
+      for (int j = 0; j < 2; ++j) o.kt[mb][j] = ldf(rc, kKtB, 2 * (2 * rb + mb) + j);
+    o.vq = *(const DAN_GLOBAL float *)(vec + 2 * kC + ri);
     o.glast = *(const DAN_GLOBAL float *)(vec + 4 * kC);
   };
   // the 16 bytes of plane column c, rows k0 .. k0 + 7
@@ -807,14 +845,18 @@ void chunk_scan_bf16_kernel(const Params p) {
     return *reinterpret_cast<const u32x4 *>(lds + plane + 2 * (c * stride + k0));
   };
 
-  OpsBf<NC> op;
+  OpsBf<COLS> op;
   int s = r + row0 / kC;
   if (row0 < end) {
     load0(op, row0, s);
     load1(op, s);
     load2(op, s);
   }
-  __syncthreads();
+#pragma unroll
+  for (int mb = 0; mb < 2; ++mb)
+#pragma unroll
+    for (int n = 0; n < NC; ++n) put4_bf(lds + LB::sHi, lds + LB::sLo, 2 * ((16 * n + l16) * kPS + srow(mb)), st[mb][n]);
+  barrier_lds();
   for (int t0 = row0; t0 < end; t0 += kC, ++s) {
     const int L = min(kC, end - t0), jmax = (L - 1) >> 5;
     const int jt = min(rb >> 1, jmax);  // the wave's last 32-row block of T Y and A D
@@ -822,6 +864,13 @@ void chunk_scan_bf16_kernel(const Params p) {
     const int tn = more ? t0 + kC : t0, sn = more ? s + 1 : s;
 
     // phase 0: K S and Q S; Y = diag(beta) V - diag(beta gamma r_k) K S
+    if constexpr (kVec) {  // the wave's 16 rows of v, as they lie (read back below, by this wave only)
+      typedef uint32_t piece __attribute__((ext_vector_type(COLS / 8)));
+      piece x;
+#pragma unroll
+      for (int i = 0; i < COLS / 8; ++i) x[i] = op.v[i];
+      *reinterpret_cast<piece *>(lds + LB::vRows + rb * LB::vWave + lane * (COLS / 2)) = x;
+    }
     f32x4 x[NC], o1[NC];
 #pragma unroll
     for (int n = 0; n < NC; ++n) x[n] = o1[n] = f32x4{};
@@ -832,15 +881,30 @@ void chunk_scan_bf16_kernel(const Params p) {
         const u32x4 bh = rd(LB::sHi, kPS, 16 * n + l16, 32 * j + 8 * g4);
         const u32x4 bl = rd(LB::sLo, kPS, 16 * n + l16, 32 * j + 8 * g4);
         x[n] = mma_bf(op.ka[j], bh, x[n]);
-        o1[n] = mma_bf(op.qa[j], bh, o1[n]);
+        o1[n] = mma_bf(bh, op.qa[j], o1[n]);
         x[n] = mma_bf(op.ka[j], bl, x[n]);
-        o1[n] = mma_bf(op.qa[j], bl, o1[n]);
+        o1[n] = mma_bf(bl, op.qa[j], o1[n]);
       }
 #pragma unroll
     for (int n = 0; n < NC; ++n) {
+      f32x4 v;
+      if constexpr (kVec) {
+        typedef int16_t i16x4 __attribute__((ext_vector_type(4)));
+        // lane i of 16 addresses row 4 g4 + i / 4, columns 16 n + 4 (i % 4) .. + 3
+        uint8_t *at = lds + LB::vRows + rb * LB::vWave + (4 * g4 + (l16 >> 2)) * (COLS * 2) + 2 * (16 * n + 4 * (l16 & 3));
+        const i16x4 t = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) i16x4 *)(__attribute__((address_space(3))) uint8_t *)at);
+#pragma unroll
+        for (int rr = 0; rr < 4; ++rr) {
+          const uint16_t bits = (uint16_t)t[rr];
+          v[rr] = __builtin_bit_cast(float, (uint32_t)bits << 16);
+        }
+      } else {
+#pragma unroll
+        for (int rr = 0; rr < 4; ++rr) v[rr] = op.vv[n][rr];
+      }
       f32x4 y;
 #pragma unroll
-      for (int rr = 0; rr < 4; ++rr) y[rr] = op.vb[rr] * op.vv[n][rr] - op.va[rr] * x[n][rr];
+      for (int rr = 0; rr < 4; ++rr) y[rr] = op.vb[rr] * v[rr] - op.va[rr] * x[n][rr];
       put4_bf(lds + LB::yHi, lds + LB::yLo, 2 * ((16 * n + l16) * kPC + ro), y);
     }
     load0(op, tn, sn);
@@ -887,27 +951,33 @@ void chunk_scan_bf16_kernel(const Params p) {
           for (int n = 0; n < NC; ++n) {
             const u32x4 bh = rd(LB::dHi, kPC, 16 * n + l16, 32 * j + 8 * g4);
             const u32x4 bl = rd(LB::dLo, kPC, 16 * n + l16, 32 * j + 8 * g4);
-            o2[n] = mma_bf(op.ah[j], bh, o2[n]);
-            o2[n] = mma_bf(op.ah[j], bl, o2[n]);
-            o2[n] = mma_bf(op.al[j], bh, o2[n]);
+            o2[n] = mma_bf(bh, op.ah[j], o2[n]);
+            o2[n] = mma_bf(bl, op.ah[j], o2[n]);
+            o2[n] = mma_bf(bh, op.al[j], o2[n]);
           }
         }
+      // row ri, columns 16 n + 4 g4 .. + 3
+      if (ri < L) {
 #pragma unroll
-      for (int rr = 0; rr < 4; ++rr)
-        if (ro + rr < L) {
+        for (int n = 0; n < NC; ++n) {
+          f32x4 y;
 #pragma unroll
-          for (int n = 0; n < NC; ++n)
-            *(DAN_GLOBAL __bf16 *)(oh + (int64_t)(t0 + ro + rr) * p.o_st + 16 * n + l16) = (__bf16)(op.vq[rr] * o1[n][rr] + o2[n][rr]);
+          for (int rr = 0; rr < 4; ++rr) y[rr] = op.vq * o1[n][rr] + o2[n][rr];
+          typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
+          const bf16x4 yb = __builtin_convertvector(y, bf16x4);
+          __bf16 *dst = oh + (int64_t)(t0 + ri) * p.o_st + 16 * n + 4 * g4;
+          if constexpr (kVec) *(DAN_GLOBAL bf16x4 *)dst = yb;
+          else {
+#pragma unroll
+            for (int rr = 0; rr < 4; ++rr) *(DAN_GLOBAL __bf16 *)(dst + rr) = yb[rr];
+          }
         }
+      }
     }
 #pragma unroll
     for (int mb = 0; mb < 2; ++mb) {
-      const int sr = 32 * rb + 16 * mb + 4 * g4;  // the lane's first state row of block mb
-      f32x4 acc[NC];
 #pragma unroll
-      for (int n = 0; n < NC; ++n)
-#pragma unroll
-        for (int rr = 0; rr < 4; ++rr) acc[n][rr] = op.glast * sS[(sr + rr) * kSS + 16 * n + l16];
+      for (int n = 0; n < NC; ++n) st[mb][n] *= op.glast;
 #pragma unroll
       for (int j = 0; j < 2; ++j)
         if (j <= jmax) {
@@ -915,25 +985,23 @@ void chunk_scan_bf16_kernel(const Params p) {
           for (int n = 0; n < NC; ++n) {
             const u32x4 bh = rd(LB::eHi, kPC, 16 * n + l16, 32 * j + 8 * g4);
             const u32x4 bl = rd(LB::eLo, kPC, 16 * n + l16, 32 * j + 8 * g4);
-            acc[n] = mma_bf(op.kt[mb][j], bh, acc[n]);
-            acc[n] = mma_bf(op.kt[mb][j], bl, acc[n]);
+            st[mb][n] = mma_bf(op.kt[mb][j], bh, st[mb][n]);
+            st[mb][n] = mma_bf(op.kt[mb][j], bl, st[mb][n]);
           }
         }
 #pragma unroll
-      for (int n = 0; n < NC; ++n) {
-#pragma unroll
-        for (int rr = 0; rr < 4; ++rr) sS[(sr + rr) * kSS + 16 * n + l16] = acc[n][rr];
-        put4_bf(lds + LB::sHi, lds + LB::sLo, 2 * ((16 * n + l16) * kPS + sr), acc[n]);
-      }
+      for (int n = 0; n < NC; ++n) put4_bf(lds + LB::sHi, lds + LB::sLo, 2 * ((16 * n + l16) * kPS + srow(mb)), st[mb][n]);
     }
     load2(op, sn);
     barrier_lds();  // the new state is whole, and every read of this chunk's Y, D and S is done
   }
 #pragma unroll
-  for (int m = 0; m < kDk * COLS / 256; ++m) {
-    const int x = tid + 256 * m;
-    *(DAN_GLOBAL float *)(p.s_out + sbase + (int64_t)(x / COLS) * p.Dv + x % COLS) = sS[(x / COLS) * kSS + x % COLS];
-  }
+  for (int mb = 0; mb < 2; ++mb)
+#pragma unroll
+    for (int n = 0; n < NC; ++n)
+#pragma unroll
+      for (int rr = 0; rr < 4; ++rr)
+        *(DAN_GLOBAL float *)(p.s_out + sbase + (int64_t)(srow(mb) + rr) * p.Dv + 16 * n + l16) = st[mb][n][rr];
 }
 
 int64_t slots(int32_t num_tokens, int32_t num_runs) { return (int64_t)num_runs + num_tokens / kC; }
@@ -972,7 +1040,17 @@ hipError_t dan_gdn_fwd_chunked(const DanGdnArgs *a, float *records, hipStream_t 
   constexpr int SW = dan_gdnc::kScanShortWaves, SC = dan_gdnc::kShortCols;
   if (a->dtype == DAN_DTYPE_BF16) {
     if (prep) hipLaunchKernelGGL(dan_gdnc::chunk_prep_kernel<__bf16>, dim3((unsigned)prep), block, 0, s, p);
-    scan(dan_gdnc::chunk_scan_bf16_kernel<dan_gdnc::kBfCols>, 4, dan_gdnc::kBfCols);
+    // v in pieces of 16 bytes (a wider column block's), out in pieces of 8
+    const bool vec = !(((uintptr_t)a->v & 15) || a->v_stride_tok % 8 || a->v_stride_head % 8 || ((uintptr_t)a->out & 7) ||
+                       a->o_stride_tok % 4 || a->o_stride_head % 4);
+    using namespace dan_gdnc;
+    if ((int64_t)p.units * (a->v_dim / 16) <= kScan16Groups) {
+      if (vec) scan(chunk_scan_bf16_kernel<16, true>, 4, 16);
+      else scan(chunk_scan_bf16_kernel<16, false>, 4, 16);
+    } else {
+      if (vec) scan(chunk_scan_bf16_kernel<32, true>, 4, 32);
+      else scan(chunk_scan_bf16_kernel<32, false>, 4, 32);
+    }
   } else {
     if (prep) hipLaunchKernelGGL(dan_gdnc::chunk_prep_kernel<_Float16>, dim3((unsigned)prep), block, 0, s, p);
     if (shortrun) scan(dan_gdnc::chunk_scan_kernel<_Float16, SW, SC>, SW, SC);
