@@ -18,11 +18,11 @@
 //                      rows into LDS in coalesced loads, the l2-norm factors
 //                      of the rows, K K^T and Q K^T on v_mfma_f32_32x32x16
 //                      (exact bf16/fp16 products, fp32 sums; the norm factors
-//                      and decays are applied after, in fp32), then T by
-//                      forward substitution, one column per four lanes; T, A
-//                      and the per-row factors (and for bf16 inputs K^T) go
-//                      to the chunk records of the workspace, T and A staged
-//                      in LDS for 16-byte stores.
+//                      and decays are applied after, in fp32), then T block by
+//                      block on v_mfma_f32_16x16x4_f32; T, A and the per-row
+//                      factors (and for bf16 inputs K^T) go to the chunk
+//                      records of the workspace straight from registers, four
+//                      columns a lane.
 //   chunk_scan_bf16_kernel  (bf16 inputs) one work group per (run, value
 //                      head, 32 or 16 state columns), the state slice in the
 //                      waves' registers; the run's chunks in order, each the
@@ -152,6 +152,15 @@ __device__ inline float sumsq8(u32x4 x) {
   return s;
 }
 
+// The sum over each 16 lanes of a wave, in the last of them.
+__device__ inline float sum16(float x) {
+  auto add = [](float x, int y) __attribute__((always_inline)) { return x + __builtin_bit_cast(float, y); };
+  x = add(x, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), 0x111, 0xf, 0xf, true));  // row_shr:1
+  x = add(x, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), 0x112, 0xf, 0xf, true));
+  x = add(x, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), 0x114, 0xf, 0xf, true));
+  return add(x, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), 0x118, 0xf, 0xf, true));
+}
+
 __device__ inline int slot_of(const int32_t *cu, int r) { return r + *(const DAN_GLOBAL int32_t *)(cu + r) / kC; }
 
 // ---------------------------------------------------------------- chunk preparation
@@ -163,37 +172,79 @@ __device__ inline void barrier_lds() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_b
 // The prep's LDS: the chunk's k and q rows, 16 threads per row loading 16
 // bytes each (coalesced; the products then read their operands here). Rows
 // are kTileRow bytes apart: 16 rows reading 16 bytes of one column hit all 64
-// banks. After the products the q tile holds L [64][kC + 4] (the same bytes)
-// and the k tile stages A, then T: 16 KB each, written to the record in
-// coalesced 16-byte stores.
+// banks. After the products the q tile holds L [64][kLRow] (the same bytes)
+// and the k tile the inverses of L's diagonal blocks.
 constexpr int kTileRow = kDk * 2 + 16;
 constexpr int kTileBytes = kC * kTileRow;
-static_assert(kTileBytes == kC * (kC + 4) * 4, "L fits the q tile");
-static_assert(kC * kC * 4 <= kTileBytes, "A or T staging fits the k tile");
+constexpr int kLRow = kC + 4;  // floats
+static_assert(kTileBytes == kC * kLRow * 4, "L fits the q tile");
 
-// Rows 16 W .. kC - 1 of the forward substitution (rows above 16 W are 0 in
-// wave W's columns), as one straight-line block.
-template <int W>
-__device__ inline void tsolve_rows(const float (*sL)[kC + 4], float (&xm)[kC / 4], int j, int part) {
+__device__ inline f32x4 mma(float a, float b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
+// c + a b of 16 x 16 blocks: lane l16 + 16 g4 holds row l16, columns 4 g4 .. + 3
+// of a, and of b and c column l16, rows 4 g4 .. + 3 (so c is a later product's b
+// as it lies).
+__device__ inline f32x4 mma16(f32x4 a, f32x4 b, f32x4 c) {
 #pragma unroll
-  for (int i = 16 * W; i < kC; ++i) {
-    float acc = 0.f;
+  for (int m = 0; m < 4; ++m) c = mma(a[m], b[m], c);
+  return c;
+}
+
+// Column block J of T = (I + L)^-1 in blocks of 16, downwards: T_JJ = D_J, T_iJ =
+// -D_i sum_{J <= k < i} L_ik T_kJ, with D_i the inverse of I + L_ii (sD, row by
+// row; `dj`: D_J's column l16, rows 4 g4 .. + 3). x[i] receives T_iJ transposed: its
+// row l16, columns 4 g4 .. + 3 (the last product of a block is taken both ways).
+// Each block solves its rows of (I + L) T = I, as the substitution row by row
+// does; solving T (I + L) = I blockwise has about three times the error in the
+// updates T Y where keys are much alike.
+template <int J>
+__device__ inline void t_columns(const float *sL, const float *sD, f32x4 dj, f32x4 (&x)[4], int l16, int g4) {
+  auto row4 = [&](const float *m, int stride) __attribute__((always_inline)) {
+    return *reinterpret_cast<const f32x4 *>(m + l16 * stride + 4 * g4);
+  };
+  f32x4 t[4];
+  t[J] = dj;
+  x[J] = row4(sD + J * 256, 16);
 #pragma unroll
-    for (int k = 0; k < (i + 3) / 4; ++k) acc = fmaf(sL[i][4 * k + part], xm[k], acc);
-    acc += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, acc), 0xB1, 0xf, 0xf, false));
-    acc += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, acc), 0x4E, 0xf, 0xf, false));
-    const float xi = (i == j ? 1.f : 0.f) - acc;
-    if (part == (i & 3)) xm[i >> 2] = xi;
+  for (int i = J + 1; i < 4; ++i) {
+    f32x4 y = {};
+#pragma unroll
+    for (int k = J; k < i; ++k) y = mma16(row4(sL + 16 * i * kLRow + 16 * k, kLRow), t[k], y);
+    const f32x4 d = row4(sD + i * 256, 16);
+    if (i < 3) t[i] = -mma16(d, y, f32x4{});
+    x[i] = -mma16(y, d, f32x4{});
   }
 }
 
+// Columns 4 at .. + 3 of a 64 x 64 record matrix's row, at byte `mat` of the
+// record: bf16 pairs in fragment order, the lo plane kC * kC * 2 bytes after
+// the hi plane, or fp32 row-major.
+template <bool kBf>
+__device__ inline void put_row4(uint8_t *mat, int row, int at, f32x4 x) {
+  if constexpr (kBf) {
+    typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
+    const bf16x4 hi = __builtin_convertvector(x, bf16x4);
+    const bf16x4 lo = __builtin_convertvector(x - __builtin_convertvector(hi, f32x4), bf16x4);
+    uint8_t *to = mat + frag_at(row, at >> 1) + 8 * (at & 1);
+    *(DAN_GLOBAL bf16x4 *)to = hi;
+    *(DAN_GLOBAL bf16x4 *)(to + kC * kC * 2) = lo;
+  } else {
+    *(DAN_GLOBAL f32x4 *)(mat + 4 * (row * kC + 4 * at)) = x;
+  }
+}
+
+// Bound by its chain of dependent steps where a phase has few chunks, and by the
+// 49 KiB record a group writes where it has many. Substituting row by row on one
+// lane group per column took 64 serial steps on the slowest wave, and the row
+// factors and the records' staging in LDS three more passes: 15.2 us for one run
+// of 611 tokens (16 heads), now 8.7; the three phases of 9400 tokens 84 us, now 59.
 // Grid: slots x Hv; a slot past its run's last chunk exits at once.
 template <typename T>
 __global__ __launch_bounds__(kThreads) void chunk_prep_kernel(const Params p) {
   __shared__ __attribute__((aligned(16))) uint8_t sKt[kTileBytes];
   __shared__ __attribute__((aligned(16))) uint8_t sQt[kTileBytes];
-  __shared__ float sG[kC], sF[3][kC];  // G; per row beta r_k, r_q Dk^-1/2 and r_k
-  float(*sL)[kC + 4] = reinterpret_cast<float(*)[kC + 4]>(sQt);
+  // G; per row beta r_k, r_q Dk^-1/2 and r_k; the rows' sums of squares (q, k)
+  __shared__ __attribute__((aligned(16))) float sG[kC], sF[3][kC], sSq[2][kC];
+  float *sL = reinterpret_cast<float *>(sQt), *sD = reinterpret_cast<float *>(sKt);
   const int s = blockIdx.x / p.Hv, h = blockIdx.x % p.Hv;
   // The run of slot s: the largest r with slot_of(r) <= s. slot_of increases
   // strictly with r (slot_of(0) = 0), so r + 1 is the number of runs whose
@@ -230,7 +281,14 @@ __global__ __launch_bounds__(kThreads) void chunk_prep_kernel(const Params p) {
   uint8_t *recb = reinterpret_cast<uint8_t *>(rec);
 
   // 1. The k and q rows (rows past the run repeat its last row; the scan
-  //    multiplies padding by zero), and wave 0's gates of row `lane`.
+  //    multiplies padding by zero) and their sums of squares; wave 0's gates of
+  //    row `lane` and their prefix sum G, while the rows are on their way.
+  float G = 0.f, b = 0.f;
+  if (wave == 0) {
+    const int64_t t = t0 + min(lane, L - 1);
+    G = *(const DAN_GLOBAL float *)(p.g + t * p.Hv + h);
+    b = *(const DAN_GLOBAL float *)(p.beta + t * p.Hv + h);
+  }
   {
     const T *kb = static_cast<const T *>(p.k) + (int64_t)hk * p.k_sh + 8 * (tid & 15);
     const T *qb = static_cast<const T *>(p.q) + (int64_t)hk * p.q_sh + 8 * (tid & 15);
@@ -241,41 +299,35 @@ __global__ __launch_bounds__(kThreads) void chunk_prep_kernel(const Params p) {
       kx[m] = *(const DAN_GLOBAL u32x4 *)(kb + t * p.k_st);
       qx[m] = *(const DAN_GLOBAL u32x4 *)(qb + t * p.q_st);
     }
+    if (wave == 0) {
+      if (lane >= L) G = b = 0.f;
+#pragma unroll
+      for (int off = 1; off < 64; off <<= 1) {
+        const float y = __shfl_up(G, off);
+        if (lane >= off) G += y;
+      }
+    }
 #pragma unroll
     for (int m = 0; m < 4; ++m) {
-      const int at = (16 * m + (tid >> 4)) * kTileRow + 16 * (tid & 15);
+      const int row = 16 * m + (tid >> 4), at = row * kTileRow + 16 * (tid & 15);
       *reinterpret_cast<u32x4 *>(sKt + at) = kx[m];
       *reinterpret_cast<u32x4 *>(sQt + at) = qx[m];
+      const float sq = sum16(sumsq8<T>(qx[m])), sk = sum16(sumsq8<T>(kx[m]));
+      if ((tid & 15) == 15) {
+        sSq[0][row] = sq;
+        sSq[1][row] = sk;
+      }
     }
-  }
-  float G = 0.f, b = 0.f;
-  if (wave == 0) {
-    const bool ok = lane < L;
-    const int64_t t = t0 + min(lane, L - 1);
-    G = ok ? *(const DAN_GLOBAL float *)(p.g + t * p.Hv + h) : 0.f;
-    b = ok ? *(const DAN_GLOBAL float *)(p.beta + t * p.Hv + h) : 0.f;
   }
   barrier_lds();
 
   // 2. Wave 0: the row factors of row `lane`: 1 / sqrt(sum x^2 + 1e-6) of its
-  //    q and k rows (dan/models/qwen3_5.py:99-100), G by a prefix sum over the
-  //    lanes, the record's five rows.
+  //    q and k rows (dan/models/qwen3_5.py:99-100), the record's five rows.
   if (wave == 0) {
     const int i = lane;
     const bool ok = i < L;
-    float sq = 0.f, sk = 0.f;
-#pragma unroll
-    for (int j = 0; j < kDk / 8; ++j) {
-      sq += sumsq8<T>(*reinterpret_cast<const u32x4 *>(sQt + i * kTileRow + 16 * j));
-      sk += sumsq8<T>(*reinterpret_cast<const u32x4 *>(sKt + i * kTileRow + 16 * j));
-    }
-    const float rq = ok ? 1.0f / sqrtf(sq + 1e-6f) : 0.f;
-    const float rk = ok ? 1.0f / sqrtf(sk + 1e-6f) : 0.f;
-#pragma unroll
-    for (int off = 1; off < 64; off <<= 1) {
-      const float y = __shfl_up(G, off);
-      if (lane >= off) G += y;
-    }
+    const float rq = ok ? 1.0f / sqrtf(sSq[0][i] + 1e-6f) : 0.f;
+    const float rk = ok ? 1.0f / sqrtf(sSq[1][i] + 1e-6f) : 0.f;
     const float Glast = __shfl(G, 63);  // padding rows add 0: the decay through the run's last row
     const float gam = expf(G);
     sG[i] = G;
@@ -289,8 +341,9 @@ __global__ __launch_bounds__(kThreads) void chunk_prep_kernel(const Params p) {
     sF[2][i] = rk;
   }
 
-  // K K^T and Q K^T, 32 x 32 block (bi, bj) per wave: lane l reads 16 bytes
-  // of row 32 b + l % 32 at element 16 kk + 8 (l / 32).
+  // K K^T and Q K^T, 32 x 32 block (bi, bj) per wave, transposed (a lane holds
+  // row l % 32 of the block, four consecutive columns at a time): lane l reads
+  // 16 bytes of row 32 b + l % 32 at element 16 kk + 8 (l / 32).
   const int bi = wave >> 1, bj = wave & 1;
   const uint8_t *ki = sKt + (32 * bi + (lane & 31)) * kTileRow + 16 * (lane >> 5);
   const uint8_t *kj = sKt + (32 * bj + (lane & 31)) * kTileRow + 16 * (lane >> 5);
@@ -301,8 +354,8 @@ __global__ __launch_bounds__(kThreads) void chunk_prep_kernel(const Params p) {
     const u32x4 a = *reinterpret_cast<const u32x4 *>(ki + 32 * kk);
     const u32x4 bb = *reinterpret_cast<const u32x4 *>(kj + 32 * kk);
     const u32x4 aq = *reinterpret_cast<const u32x4 *>(qi + 32 * kk);
-    P = mfma_in<T>(a, bb, P);
-    QK = mfma_in<T>(aq, bb, QK);
+    P = mfma_in<T>(bb, a, P);
+    QK = mfma_in<T>(bb, aq, QK);
   }
   if constexpr (kBf) {
     // K^T for the bf16 scan: thread t writes d rows 2 dp and 2 dp + 1,
@@ -325,73 +378,63 @@ __global__ __launch_bounds__(kThreads) void chunk_prep_kernel(const Params p) {
   }
   barrier_lds();  // sG, the row factors; every read of the tiles is done
 
-  // 3. L into the q tile's bytes, A staged in the k tile's (the record's A
-  //    block layout: bf16 hi and lo planes, or fp32).
+  // 3. L into the q tile's bytes, A to the record.
+  constexpr int kMatBytes = kC * kC * 4;  // the T block, then the A block, of the record
+  static_assert(kAhiB == kMatBytes && kThiB == 0 && kTloB == kC * kC * 2 && kAloB == kAhiB + kTloB, "record layout");
+  {
+    const int i = 32 * bi + (lane & 31);
+    const float Gi = sG[i], fk = sF[0][i], fq = sF[1][i];
 #pragma unroll
-  for (int rr = 0; rr < 16; ++rr) {  // accumulator: row 8 (rr / 4) + 4 (lane / 32) + rr % 4, column lane % 32
-    const int i = 32 * bi + 8 * (rr >> 2) + 4 * (lane >> 5) + (rr & 3), j = 32 * bj + (lane & 31);
-    const float e = (i >= j && i < L) ? expf(sG[i] - sG[j]) : 0.f;
-    const float rkj = sF[2][j];
-    sL[i][j] = i > j ? sF[0][i] * rkj * P[rr] * e : 0.f;
-    const float av = sF[1][i] * rkj * QK[rr] * e;
-    if constexpr (kBf) {
-      const __bf16 hi = (__bf16)av;
-      *reinterpret_cast<__bf16 *>(sKt + 2 * (i * kC + j)) = hi;
-      *reinterpret_cast<__bf16 *>(sKt + kC * kC * 2 + 2 * (i * kC + j)) = (__bf16)(av - (float)hi);
-    } else {
-      *reinterpret_cast<float *>(sKt + 4 * (i * kC + j)) = av;
+    for (int c = 0; c < 4; ++c) {  // accumulators 4 c .. + 3: columns 8 c + 4 (lane / 32) .. + 3 of the block
+      const int j = 32 * bj + 8 * c + 4 * (lane >> 5);
+      const f32x4 Gj = *reinterpret_cast<const f32x4 *>(sG + j), rkj = *reinterpret_cast<const f32x4 *>(sF[2] + j);
+      f32x4 lv, av;
+#pragma unroll
+      for (int x = 0; x < 4; ++x) {
+        const float e = (i >= j + x && i < L) ? expf(Gi - Gj[x]) : 0.f;
+        lv[x] = i > j + x ? fk * rkj[x] * P[4 * c + x] * e : 0.f;
+        av[x] = fq * rkj[x] * QK[4 * c + x] * e;
+      }
+      *reinterpret_cast<f32x4 *>(sL + i * kLRow + j) = lv;
+      put_row4<kBf>(recb + kMatBytes, i, j >> 2, av);
     }
   }
   barrier_lds();
 
-  // 4. A out (16 KB from the stage), then T = (I + L)^-1 by forward
-  //    substitution, x_i = [i == j] - sum_{m < i} L[i][m] x_m for column j:
-  //    wave w solves columns 16 w .. 16 w + 15, four lanes per column (lane
-  //    4 c + p: column 16 w + c, the terms m = p mod 4), the four partial sums
-  //    added by two quad swaps. Rows above 16 w are 0 in these columns;
-  //    L[i][m] = 0 for m >= i, so whole groups of four are summed.
-  constexpr int kBlockBytes = kC * kC * 4;  // the T block, then the A block, of the record
-  static_assert(kAhiB == kBlockBytes && kThiB == 0, "record layout");
-  // The stage's byte that goes to byte `off` of the record's block: for bf16
-  // the hi and lo planes (row-major in the stage) in fragment order.
-  auto staged = [](int off) __attribute__((always_inline)) {
-    if (!kBf) return off;
-    const int f = off % (kC * kC * 2), lane = f / 16 % 64, fb = f / 1024;  // fragment fb: rows 16 (fb / 2), columns 32 (fb % 2)
-    return off - f + 2 * ((16 * (fb >> 1) + (lane & 15)) * kC + 32 * (fb & 1) + 8 * (lane >> 4));
-  };
+  // 4. T = (I + L)^-1. Wave w: D_w, the inverse of its diagonal block, by forward
+  //    substitution, column l16 in every group of 16 lanes; then column block w of T
+  //    (t_columns) on the matrix cores in fp32.
+  const int l16 = lane & 15, g4 = lane >> 4;
+  f32x4 mine;  // D_w's column l16, rows 4 g4 .. + 3
+  {
+    const float *diag = sL + 16 * wave * (kLRow + 1);
+    float x[16];
 #pragma unroll
-  for (int m = 0; m < kBlockBytes / (16 * kThreads); ++m) {
-    const int off = 16 * (kThreads * m + tid);
-    *(DAN_GLOBAL u32x4 *)(recb + kBlockBytes + off) = *reinterpret_cast<const u32x4 *>(sKt + staged(off));
-  }
-  const int j = 16 * wave + (lane >> 2), part = lane & 3;
-  float xm[kC / 4];  // x_{4 k + part}
+    for (int i = 0; i < 16; ++i) {
+      x[i] = i == l16 ? 1.f : 0.f;
 #pragma unroll
-  for (int k = 0; k < kC / 4; ++k) xm[k] = 0.f;
-  switch (wave) {  // wave-uniform
-    case 0: tsolve_rows<0>(sL, xm, j, part); break;
-    case 1: tsolve_rows<1>(sL, xm, j, part); break;
-    case 2: tsolve_rows<2>(sL, xm, j, part); break;
-    default: tsolve_rows<3>(sL, xm, j, part); break;
-  }
-  barrier_lds();  // every wave's A reads of the stage are done
+      for (int m4 = 0; m4 < i; m4 += 4) {
+        const f32x4 row = *reinterpret_cast<const f32x4 *>(diag + i * kLRow + m4);
 #pragma unroll
-  for (int k = 0; k < kC / 4; ++k) {
-    const int i = 4 * k + part;
-    if constexpr (kBf) {
-      const __bf16 hi = (__bf16)xm[k];
-      *reinterpret_cast<__bf16 *>(sKt + 2 * (i * kC + j)) = hi;
-      *reinterpret_cast<__bf16 *>(sKt + kC * kC * 2 + 2 * (i * kC + j)) = (__bf16)(xm[k] - (float)hi);
-    } else {
-      *reinterpret_cast<float *>(sKt + 4 * (i * kC + j)) = xm[k];
+        for (int m = m4; m < min(m4 + 4, i); ++m) x[i] = fmaf(-row[m - m4], x[m], x[i]);
+      }
+    }
+#pragma unroll
+    for (int m = 0; m < 4; ++m) {
+      mine[m] = g4 < 2 ? (g4 == 0 ? x[m] : x[4 + m]) : (g4 == 2 ? x[8 + m] : x[12 + m]);
+      sD[(16 * wave + 4 * g4 + m) * 16 + l16] = mine[m];
     }
   }
   barrier_lds();
-#pragma unroll
-  for (int m = 0; m < kBlockBytes / (16 * kThreads); ++m) {
-    const int off = 16 * (kThreads * m + tid);
-    *(DAN_GLOBAL u32x4 *)(recb + off) = *reinterpret_cast<const u32x4 *>(sKt + staged(off));
+  f32x4 x[4] = {};
+  switch (wave) {  // wave-uniform
+    case 0: t_columns<0>(sL, sD, mine, x, l16, g4); break;
+    case 1: t_columns<1>(sL, sD, mine, x, l16, g4); break;
+    case 2: t_columns<2>(sL, sD, mine, x, l16, g4); break;
+    default: t_columns<3>(sL, sD, mine, x, l16, g4); break;
   }
+#pragma unroll
+  for (int i = 0; i < 4; ++i) put_row4<kBf>(recb, 16 * i + l16, 4 * wave + g4, x[i]);
 }
 
 // ---------------------------------------------------------------- the scan over chunks
@@ -414,8 +457,6 @@ struct ScanLds {
 // also runs as 8 waves on 32 columns, one tile each, which took 11 % longer on
 // a trunk phase of 5 runs of 286 to 1843 tokens.)
 constexpr int kScanLongWaves = 4, kScanShortWaves = 4;
-
-__device__ inline f32x4 mma(float a, float b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
 
 
 // Contraction orders: the 128-long sums over the state rows take k-index
