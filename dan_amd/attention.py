@@ -159,12 +159,13 @@ def attend(q, k, v, segments, layer, scale=None, *, q_scale=None, k_scale=None, 
 
 
 def _check_inputs(q, k, v):
-    if q.dim() != 3 or k.dim() != 3 or v.dim() != 3:
+    qs, ks, vs = q.shape, k.shape, v.shape
+    if len(qs) != 3 or len(ks) != 3 or len(vs) != 3:
         raise ValueError("q must be [H, N, D] and k, v [Hkv, N, D]")
-    h, n, d = q.shape
-    hkv = k.shape[0]
-    if k.shape != (hkv, n, d) or v.shape != (hkv, n, d):
-        raise ValueError(f"k {tuple(k.shape)} and v {tuple(v.shape)} must be [Hkv, {n}, {d}]")
+    h, n, d = qs
+    hkv = ks[0]
+    if ks != vs or ks[1] != n or ks[2] != d:
+        raise ValueError(f"k {tuple(ks)} and v {tuple(vs)} must be [Hkv, {n}, {d}]")
     if hkv == 0 or h % hkv:
         raise ValueError(f"{h} query heads is not a multiple of {hkv} kv heads")
     if q.dtype not in _DTYPES or k.dtype != q.dtype or v.dtype != q.dtype:
@@ -183,9 +184,8 @@ def _check_scale(t, name, device):
 
 def _aligned(t):
     """16-byte vector loads need 16-byte aligned rows with a unit-stride head_dim."""
-    es = t.element_size()
-    return (t.stride(-1) == 1 and t.data_ptr() % 16 == 0
-            and all((st * es) % 16 == 0 for st in t.stride()[:-1]))
+    es, st = t.element_size(), t.stride()
+    return st[-1] == 1 and t.data_ptr() % 16 == 0 and all((s * es) % 16 == 0 for s in st[:-1])
 
 
 def _kernel_view(t):
@@ -194,8 +194,8 @@ def _kernel_view(t):
     kernel's 32-bit in-tile offsets). The copy is a new allocation, so its
     base is aligned; ``contiguous()`` would return a contiguous but
     misaligned view unchanged."""
-    small = abs(t.stride(-2)) * 64 < 2 ** 31
-    if _aligned(t) and small:
+    es, st = t.element_size(), t.stride()
+    if len(st) == 3 and st[2] == 1 and not ((st[0] | st[1]) * es | t.data_ptr()) & 15 and abs(st[1]) < 2 ** 25:
         return t
     return torch.empty_like(t, memory_format=torch.contiguous_format).copy_(t)
 
@@ -213,7 +213,8 @@ def get_plan(segments, num_tokens, tile_q, device, groups=None, num_cus=None, pl
     if planner not in ("device", "host"):
         raise ValueError(f"planner {planner!r}: 'device' or 'host'")
     plan = getattr(segments, "tile_plan", None)
-    want_device = planner == "device" and groups is not None and torch.device(device).type == "cuda"
+    device = torch.device(device)
+    want_device = planner == "device" and groups is not None and device.type == "cuda"
     stale = plan is None or not plan.matches(num_tokens, tile_q, device)
     if not stale and want_device and plan.cost is None and (groups, num_cus) not in plan.schedules:
         stale = True  # device-built for another head layout
@@ -263,14 +264,14 @@ def _stage_f16(x):
     power of 2 that keeps the copy within fp16's range
     (``dan_tree_attn_stage_f16``, two launches on the current stream)."""
     a, out, scale, _x = _stage_args(x)
-    _native.stage_f16(a, torch.cuda.current_stream(out.device).cuda_stream)
+    _native.stage_f16(a, _native.stream(out.device))
     return out, scale
 
 
 def _stage_f16_pair(q, k):
     """``_stage_f16`` of q and of k through one pair of launches."""
     (a, qo, qs, _q), (b, ko, ks, _k) = _stage_args(q), _stage_args(k)
-    _native.stage_f16_pair(a, b, torch.cuda.current_stream(qo.device).cuda_stream)
+    _native.stage_f16_pair(a, b, _native.stream(qo.device))
     return (qo, qs), (ko, ks)
 
 
@@ -480,38 +481,17 @@ def _launch_tree_attn(q, k, v, tables, scales, meta, scale, workspace, pasts_hos
             ws = workspace if workspace is not None else torch.empty(nbytes, dtype=torch.uint8, device=q.device)
             if ws.dtype != torch.uint8 or ws.device != q.device or not ws.is_contiguous() or ws.numel() < nbytes:
                 raise ValueError(f"workspace: a contiguous uint8 tensor of >= {nbytes} bytes on {q.device}")
-        a = _native.DanTreeAttnArgs()
-        a.abi_version = _native.ABI_VERSION
-        a.in_dtype = _DTYPES[q.dtype]
-        a.v_dtype = _DTYPES[v.dtype]
-        a.out_dtype = _DTYPES[out.dtype]
-        a.num_heads, a.num_kv_heads, a.head_dim, a.num_tokens = h, hkv, d, n
-        a.scale = scale
-        a.q, a.q_stride_tok, a.q_stride_head = q.data_ptr(), q.stride(1), q.stride(0)
-        a.k, a.k_stride_tok, a.k_stride_head = k.data_ptr(), k.stride(1), k.stride(0)
-        a.v, a.v_stride_tok, a.v_stride_head = v.data_ptr(), v.stride(1), v.stride(0)
-        a.out, a.o_stride_tok, a.o_stride_head = out.data_ptr(), out.stride(0), out.stride(1)
-        a.segments, a.num_segments = segs_d.data_ptr(), num_segments
-        a.pasts, a.num_pasts = past_table.data_ptr(), num_pasts
-        if pasts_host is not None:
-            a.pasts_host = pasts_host.data_ptr()
-        a.work, a.num_work = work_d.data_ptr(), num_work
-        a.key_lo = key_lo_d.data_ptr()
-        a.tile_q, a.key_halves = tile_q, _layout(h, hkv, d)[0] // tile_q
-        a.vt_cols = vt_cols
-        a.col_seg = col_seg_d.data_ptr()
-        if ws is not None:
-            a.workspace, a.workspace_bytes = ws.data_ptr(), nbytes
-        if scales:  # e4m3: q, k, v; fp32 staged to fp16: q, k
-            a.q_scale, a.k_scale = scales[0].data_ptr(), scales[1].data_ptr()
-            if len(scales) == 3:
-                a.v_scale = scales[2].data_ptr()
-        a.phases = phases
-        a.units, a.sched_off, a.num_slots = units.data_ptr(), sched_off.data_ptr(), slots
-        if counts is not None:
-            a.counts = counts.data_ptr()
-        launch = _native.forward_noalloc if noalloc else _native.forward
-        launch(a, torch.cuda.current_stream(q.device).cuda_stream, lib)
+        scale_ptrs = [t.data_ptr() for t in scales] + [0] * (3 - len(scales))  # e4m3: q, k, v; fp32 staged to fp16: q, k
+        (q_head, q_tok, _), (k_head, k_tok, _), (v_head, v_tok, _), (o_tok, o_head, _) = q.stride(), k.stride(), v.stride(), out.stride()
+        launch = _native.call_forward_noalloc if noalloc else _native.call_forward
+        launch(_native.stream(q.device),
+               _native.ABI_VERSION, _DTYPES[q.dtype], _DTYPES[out.dtype], _DTYPES[v.dtype], h, hkv, d, n, _native.f32(scale),
+               q.data_ptr(), q_tok, q_head, k.data_ptr(), k_tok, k_head, v.data_ptr(), v_tok, v_head, out.data_ptr(), o_tok, o_head,
+               *scale_ptrs, segs_d.data_ptr(), num_segments, past_table.data_ptr(), num_pasts,
+               work_d.data_ptr(), num_work, key_lo_d.data_ptr(), tile_q, vt_cols, col_seg_d.data_ptr(),
+               0 if ws is None else ws.data_ptr(), 0 if ws is None else nbytes, phases,
+               units.data_ptr(), sched_off.data_ptr(), slots, 0 if counts is None else counts.data_ptr(),
+               0 if pasts_host is None else pasts_host.data_ptr(), _layout(h, hkv, d)[0] // tile_q)
     return out.transpose(0, 1)
 
 

@@ -105,25 +105,16 @@ def _delta_rule(q, k, v, g, beta, lengths, states, cu=None, form=None, state_ind
         raise ValueError(f"out {tuple(out.shape)} {out.dtype} on {out.device}: want [M, {hv}, {dv}] {q.dtype} on {dev}")
     if finals is None:
         finals = torch.empty((r, hv, dk, dv), dtype=torch.float32, device=dev)
-    a = _native.DanGdnArgs()
-    a.abi_version = _native.GDN_ABI_VERSION
-    a.dtype = _DTYPES[q.dtype]
-    a.num_k_heads, a.num_v_heads, a.k_dim, a.v_dim, a.num_runs, a.num_tokens = hk, hv, dk, dv, r, n
-    a.cu = cu_d.data_ptr()
-    a.q, a.q_stride_tok, a.q_stride_head = q.data_ptr(), q.stride(0), q.stride(1)
-    a.k, a.k_stride_tok, a.k_stride_head = k.data_ptr(), k.stride(0), k.stride(1)
-    a.v, a.v_stride_tok, a.v_stride_head = v.data_ptr(), v.stride(0), v.stride(1)
-    a.g, a.beta = g.data_ptr(), beta.data_ptr()
-    a.states_in, a.states_out = s_in.data_ptr(), finals.data_ptr()
-    a.out, a.o_stride_tok, a.o_stride_head = out.data_ptr(), out.stride(0), out.stride(1)
-    nbytes = _native.load().dan_gdn_workspace_size(code, n, r, hk, hv, dv)
+    nbytes = _native.gdn_workspace_size(code, n, r, hk, hv, dv)
     ws = torch.empty(max(nbytes, 16), dtype=torch.uint8, device=dev)
-    a.workspace, a.workspace_bytes, a.form = ws.data_ptr(), nbytes, code
-    if state_index is not None:
-        a.state_index, a.num_states_in = state_index.data_ptr(), s_in.shape[0]
-    if out_start is not None:
-        a.out_start, a.num_out_rows = out_start.data_ptr(), out.shape[0]
-    _native.gdn(a, torch.cuda.current_stream(dev).cuda_stream)
+    (q_tok, q_head, _), (k_tok, k_head, _), (v_tok, v_head, _), (o_tok, o_head, _) = q.stride(), k.stride(), v.stride(), out.stride()
+    _native.call_gdn(
+        _native.stream(dev), _native.GDN_ABI_VERSION, _DTYPES[q.dtype], hk, hv, dk, dv, r, n, cu_d.data_ptr(),
+        q.data_ptr(), q_tok, q_head, k.data_ptr(), k_tok, k_head, v.data_ptr(), v_tok, v_head,
+        g.data_ptr(), beta.data_ptr(), s_in.data_ptr(), finals.data_ptr(), out.data_ptr(), o_tok, o_head,
+        ws.data_ptr(), nbytes, code, 0, 0 if state_index is None else state_index.data_ptr(),
+        0 if state_index is None else s_in.shape[0], 0 if out_start is None else out.shape[0],
+        0 if out_start is None else out_start.data_ptr())
     return out, finals
 
 
@@ -156,13 +147,9 @@ def _gated_norm(out, z, weight, eps):
             or any(t.data_ptr() % 16 for t in (out, z, weight)) or not 0 <= eps < float("inf")):
         return gated_rms_norm(out.reshape(-1, dv), z.reshape(-1, dv), weight, eps).reshape(n, hv * dv)
     y = torch.empty((n, hv * dv), dtype=out.dtype, device=out.device)
-    a = _native.DanGdnNormArgs()
-    a.abi_version = _native.GDN_ABI_VERSION
-    a.dtype = _DTYPES[out.dtype]
-    a.num_tokens, a.num_v_heads, a.v_dim, a.eps = n, hv, dv, eps
-    a.x, a.x_stride, a.gate, a.gate_stride = out.data_ptr(), hv * dv, z.data_ptr(), z.stride(0)
-    a.weight, a.out, a.out_stride = weight.data_ptr(), y.data_ptr(), hv * dv
-    _native.gdn_gated_norm(a, torch.cuda.current_stream(out.device).cuda_stream)
+    _native.call_gdn_gated_norm(
+        _native.stream(out.device), _native.GDN_ABI_VERSION, _DTYPES[out.dtype], n, hv, dv, _native.f32(float(eps)),
+        out.data_ptr(), hv * dv, z.data_ptr(), z.stride(0), weight.data_ptr(), y.data_ptr(), hv * dv)
     return y
 
 
@@ -274,8 +261,8 @@ def conv_phase(qkv, hist, ph, weight, b, a, a_log, dt_bias):
     histories in layout order or None, ``weight`` [C, 1, K], ``b``/``a``
     [N, Hv], ``a_log``/``dt_bias`` [Hv]. Returns (conv [T, C] in qkv's dtype,
     beta [T, Hv] fp32, g [T, Hv] fp32)."""
-    x, outs, _keep = conv_phase_args(qkv, hist, ph, weight, b, a, a_log, dt_bias)
-    _native.gdn_conv(x, torch.cuda.current_stream(qkv.device).cuda_stream)
+    fields, outs, _keep = _conv_fields(qkv, hist, ph, weight, b, a, a_log, dt_bias)
+    _native.call_gdn_conv(_native.stream(qkv.device), *fields)
     return outs
 
 
@@ -283,6 +270,12 @@ def conv_phase_args(qkv, hist, ph, weight, b, a, a_log, dt_bias):
     """``conv_phase``'s ``DanGdnConvArgs``, its outputs (conv, beta, g) and the
     tensors the arguments point at (keep them alive while the call runs), so
     that a caller can launch the same phase again without rebuilding them."""
+    fields, outs, keep = _conv_fields(qkv, hist, ph, weight, b, a, a_log, dt_bias)
+    return _native.DanGdnConvArgs(*fields), outs, keep
+
+
+def _conv_fields(qkv, hist, ph, weight, b, a, a_log, dt_bias):
+    """``conv_phase_args`` with the structure's fields in order."""
     if not qkv.is_cuda:
         raise RuntimeError("dan_amd.deltanet.conv_phase runs on a gfx950 GPU only")
     n, c = qkv.shape
@@ -304,20 +297,11 @@ def conv_phase_args(qkv, hist, ph, weight, b, a, a_log, dt_bias):
     out = torch.empty((t, c), dtype=qkv.dtype, device=dev)
     beta = torch.empty((t, hv), dtype=torch.float32, device=dev)
     g = torch.empty((t, hv), dtype=torch.float32, device=dev)
-    x = _native.DanGdnConvArgs()
-    x.abi_version = _native.GDN_ABI_VERSION
-    x.dtype = _DTYPES[qkv.dtype]
-    x.channels, x.kernel, x.num_rows = c, kk, n
-    x.num_hist_rows = 0 if hist is None else hist.shape[0]
-    x.num_ext, x.num_out = len(ph.ext), t
-    x.src, x.src_stride = qkv.data_ptr(), qkv.stride(0)
-    x.hist = 0 if hist is None else hist.data_ptr()
-    x.ext, x.take, x.weight = ph.ext.data_ptr(), ph.take.data_ptr(), w.data_ptr()
-    x.out, x.out_stride = out.data_ptr(), out.stride(0)
-    x.num_heads, x.gate_dtype, x.rows = hv, int(lp), ph.rows.data_ptr()
-    x.b, x.b_stride, x.a, x.a_stride = b.data_ptr(), b.stride(0), a.data_ptr(), a.stride(0)
-    x.a_log, x.dt_bias, x.beta, x.g = al.data_ptr(), dtb.data_ptr(), beta.data_ptr(), g.data_ptr()
-    return x, (out, beta, g), (qkv, w, hist, b, a, al, dtb, ph)
+    fields = (_native.GDN_ABI_VERSION, _DTYPES[qkv.dtype], c, kk, n, 0 if hist is None else hist.shape[0], len(ph.ext), t,
+              qkv.data_ptr(), qkv.stride(0), 0 if hist is None else hist.data_ptr(), ph.ext.data_ptr(), ph.take.data_ptr(),
+              w.data_ptr(), out.data_ptr(), c, hv, int(lp), ph.rows.data_ptr(), b.data_ptr(), b.stride(0), a.data_ptr(), a.stride(0),
+              al.data_ptr(), dtb.data_ptr(), beta.data_ptr(), g.data_ptr())
+    return fields, (out, beta, g), (qkv, w, hist, b, a, al, dtb, ph)
 
 
 class DeltaNet(nn.Module):
@@ -389,6 +373,8 @@ def _virtual_rows(qkv, hist, idx):
     """Rows ``idx`` of the virtual source (packed rows, the zero row, then the
     cached histories) as a new [len(idx), C] tensor."""
     n = qkv.shape[0]
+    if idx and idx[-1] < n and idx == list(range(idx[0], idx[-1] + 1)):  # consecutive packed rows
+        return qkv[idx[0]:idx[-1] + 1].clone(memory_format=torch.contiguous_format)
     parts = []
     for e in idx:
         if e < n:

@@ -28,8 +28,8 @@ NORMS = {None: _native.FRONT_NORM_NONE, "rms": _native.FRONT_NORM_RMS,
 
 
 def _row_ok(t):
-    es = t.element_size()
-    return t.stride(-1) == 1 and t.data_ptr() % 16 == 0 and all((s * es) % 16 == 0 for s in t.stride()[:-1])
+    es, st = t.element_size(), t.stride()
+    return st[-1] == 1 and t.data_ptr() % 16 == 0 and not any((s * es) % 16 for s in st[:-1])
 
 
 def _view(t):
@@ -104,7 +104,6 @@ def qkv_front(q, k, v, cos, sin, *, q_norm_weight=None, k_norm_weight=None, eps=
             raise ValueError(f"cos and sin must both be [{n}, R]")
         if cos.dtype != q.dtype or sin.dtype != q.dtype:
             raise ValueError("cos and sin must be in the model dtype (the reference casts them, llama.py:158)")
-    lib = _native.load()
     dev = q.device
     q_in, k_in, v_in = _view(q), _view(k), _view(v)
     cs = sn = None
@@ -121,41 +120,28 @@ def qkv_front(q, k, v, cos, sin, *, q_norm_weight=None, k_norm_weight=None, eps=
     q_out = torch.empty((n, h, d), dtype=q.dtype, device=dev)
     k_out = torch.empty((n, hkv, d), dtype=q.dtype, device=dev)
 
-    a = _native.DanQkvFrontArgs()
-    a.abi_version = _native.FRONT_ABI_VERSION
-    a.dtype = _DTYPES[q.dtype]
-    a.num_tokens, a.num_heads, a.num_kv_heads, a.head_dim, a.rotary_dim = n, h, hkv, d, r
-    a.norm, a.eps = NORMS[norm], float(eps)
-    a.q, a.q_stride_tok, a.q_stride_head = q_in.data_ptr(), q_in.stride(0), q_in.stride(1)
-    a.k, a.k_stride_tok, a.k_stride_head = k_in.data_ptr(), k_in.stride(0), k_in.stride(1)
-    a.v, a.v_stride_tok, a.v_stride_head = v_in.data_ptr(), v_in.stride(0), v_in.stride(1)
-    if r:
-        a.cos, a.sin, a.cs_stride_tok = cs.data_ptr(), sn.data_ptr(), cs.stride(0)
-    if weights:
-        a.q_norm_weight, a.k_norm_weight = weights[0].data_ptr(), weights[1].data_ptr()
-    a.q_out, a.qo_stride_tok, a.qo_stride_head = q_out.data_ptr(), q_out.stride(0), q_out.stride(1)
-    a.k_out, a.ko_stride_tok, a.ko_stride_head = k_out.data_ptr(), k_out.stride(0), k_out.stride(1)
-
-    keep = []
+    save_of = table_d = table = None
+    num_saves = 0
     if segments is not None and layer is not None and any(s.save for s in segments):
         save_of, order = save_index(segments, n, dev)
         dst = [(torch.empty((hkv, s.save, d), dtype=q.dtype, device=dev),
                 torch.empty((hkv, s.save, d), dtype=q.dtype, device=dev)) for s in order]
-        table = (_native.DanFrontSave * len(order))()
-        for i, (s, (kd, vd)) in enumerate(zip(order, dst)):
-            table[i].start, table[i].len, table[i].k_dst, table[i].v_dst = s.start, s.save, kd.data_ptr(), vd.data_ptr()
-        a.save_of, a.num_saves = save_of.data_ptr(), len(order)
-        if len(order) <= _native.FRONT_INLINE_SAVES:  # in the launch's arguments
-            a.saves_host = ctypes.addressof(table)
-        else:
-            raw = torch.frombuffer(bytearray(table), dtype=torch.uint8)
-            table_d = raw.pin_memory().to(dev, non_blocking=True)
-            a.saves = table_d.data_ptr()
-            keep = [table_d]
+        num_saves = len(order)
+        table = (_native.DanFrontSave * num_saves)(*((s.start, s.save, kd.data_ptr(), vd.data_ptr())
+                                                    for s, (kd, vd) in zip(order, dst)))
+        if num_saves > _native.FRONT_INLINE_SAVES:  # at most so many: in the launch's arguments
+            table_d = torch.frombuffer(bytearray(table), dtype=torch.uint8).pin_memory().to(dev, non_blocking=True)
         for s, kv in zip(order, dst):
             s.saved[layer] = kv
-    _native.front(a, torch.cuda.current_stream(dev).cuda_stream, lib)
-    if keep:
+    _native.call_front(
+        _native.stream(dev), _native.FRONT_ABI_VERSION, _DTYPES[q.dtype], n, h, hkv, d, r, NORMS[norm], _native.f32(float(eps)),
+        q_in.data_ptr(), *q_in.stride()[:2], k_in.data_ptr(), *k_in.stride()[:2], v_in.data_ptr(), *v_in.stride()[:2],
+        cs.data_ptr() if r else 0, sn.data_ptr() if r else 0, cs.stride(0) if r else 0,
+        weights[0].data_ptr() if weights else 0, weights[1].data_ptr() if weights else 0,
+        q_out.data_ptr(), *q_out.stride()[:2], k_out.data_ptr(), *k_out.stride()[:2],
+        0 if save_of is None else save_of.data_ptr(), 0 if table_d is None else table_d.data_ptr(), num_saves,
+        ctypes.addressof(table) if table is not None and table_d is None else 0)
+    if table_d is not None:
         # the table must outlive the launch: tie its lifetime to the stream's progress
-        keep[0].record_stream(torch.cuda.current_stream(dev))
+        table_d.record_stream(torch.cuda.current_stream(dev))
     return q_out.transpose(0, 1), k_out.transpose(0, 1), v.transpose(0, 1)

@@ -312,7 +312,9 @@ class TilePlan:
     def matches(self, num_tokens, tile_q, device):
         import torch
 
-        return self.num_tokens == num_tokens and self.tile_q == tile_q and self.device == torch.device(device)
+        if not isinstance(device, torch.device):
+            device = torch.device(device)
+        return self.num_tokens == num_tokens and self.tile_q == tile_q and self.device == device
 
     def schedule(self, groups, num_cus):
         """Device copies of the unit records of ``schedule(self.cost, groups,

@@ -88,15 +88,10 @@ def fp8_quantize(x, fp8_max=E4M3_MAX, rowwise=True, tiled=False):
     else:
         xq = torch.empty((m, k), dtype=E4M3, device=x.device)
     scale = torch.empty((m, 1) if rowwise else (1, 1), dtype=torch.float32, device=x.device)
-    a = _native.DanFp8QuantArgs()
-    a.abi_version = _native.FP8_ABI_VERSION
-    a.dtype = _DTYPES[x.dtype]
-    a.rows, a.cols = m, k
-    a.mode = _native.FP8_SCALE_ROW if rowwise else _native.FP8_SCALE_TENSOR
-    a.layout = _native.FP8_LAYOUT_TILED if tiled else _native.FP8_LAYOUT_ROWS
-    a.x, a.x_stride = x.data_ptr(), x.stride(0)
-    a.xq, a.scale = xq.data_ptr(), scale.data_ptr()
-    _native.fp8_quantize(a, torch.cuda.current_stream(x.device).cuda_stream)
+    _native.call_fp8_quantize(
+        _native.stream(x.device), _native.FP8_ABI_VERSION, _DTYPES[x.dtype], m, k,
+        _native.FP8_SCALE_ROW if rowwise else _native.FP8_SCALE_TENSOR,
+        _native.FP8_LAYOUT_TILED if tiled else _native.FP8_LAYOUT_ROWS, x.data_ptr(), x.stride(0), xq.data_ptr(), scale.data_ptr())
     return (TiledE4M3(xq, m, k) if tiled else xq), scale
 
 
@@ -157,15 +152,9 @@ def fp8_gemm(xq, scale_a, wq, scale_b, bias=None, out_dtype=torch.bfloat16):
     xp, xs, xf = operand(xq, _native.FP8_GEMM_X_TILED)
     wp, ws, wf = operand(wq, _native.FP8_GEMM_W_TILED)
     y = torch.empty((m, n), dtype=out_dtype, device=xq.device)
-    a = _native.DanFp8GemmArgs()
-    a.abi_version = _native.FP8_ABI_VERSION
-    a.out_dtype = _DTYPES[out_dtype]
-    a.m, a.n, a.k, a.flags = m, n, k, flags | xf | wf
-    a.xq, a.xq_stride, a.x_scale = xp, xs, sa.data_ptr()
-    a.wq, a.wq_stride, a.w_scale = wp, ws, sb.data_ptr()
-    a.bias = bias.data_ptr() if bias is not None else None
-    a.y, a.y_stride = y.data_ptr(), y.stride(0)
-    _native.fp8_gemm(a, torch.cuda.current_stream(y.device).cuda_stream)
+    _native.call_fp8_gemm(
+        _native.stream(y.device), _native.FP8_ABI_VERSION, _DTYPES[out_dtype], m, n, k, flags | xf | wf,
+        xp, xs, sa.data_ptr(), wp, ws, sb.data_ptr(), bias.data_ptr() if bias is not None else 0, y.data_ptr(), y.stride(0))
     return y
 
 
