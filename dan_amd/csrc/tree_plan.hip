@@ -12,9 +12,9 @@
 //   2. work items; their costs (key tiles) sorted longest first, ties by
 //      creation order (bitonic sort of 64-bit keys in LDS)
 //   3. one wave deals the sorted items to the k slots of a head-group class,
-//      each to the least loaded slot (ties: lowest slot), then repeatedly
-//      moves one item out of the most loaded slot, or swaps one of its items
-//      with a lighter item elsewhere, choosing the option with the lowest
+//      each to the least loaded slot (ties: lowest slot); then all waves
+//      repeatedly move one item out of the most loaded slot, or swap one of its
+//      items with a lighter item elsewhere, choosing the option with the lowest
 //      resulting larger load of the pair, while that is below the maximum
 //   4. a sort by (slot, rank) gives each slot's items longest first; slot s
 //      of the k * G slots runs class s / G for head group s % G
@@ -70,10 +70,11 @@ struct Params {
 struct Smem {
   DanSegmentDesc seg[kMaxSegs];
   int32_t bst[kMaxBranches];
-  uint64_t keys[kMaxWork];  // sort keys
+  uint64_t keys[kMaxWork];  // sort keys; between the sorts the items of the most loaded slot
+  uint64_t best[2];         // the rounds' best options, in turn
   int32_t w[kMaxWork];      // schedule weight of the item at each rank
   int16_t slot[kMaxWork];   // slot of each rank
-  int16_t alist[kMaxWork];  // ranks held by the most loaded slot
+  int32_t held[2];  // items in keys, in turn
   int32_t load[kMaxSlots];
   int32_t start[kMaxSlots + 1];  // first position of each slot's run after the (slot, rank) sort
 };
@@ -245,97 +246,131 @@ __global__ __launch_bounds__(kThreads) void plan_kernel(const Params pg) {
   }
   __syncthreads();
 
-  // ---- 3. one wave: longest-processing-time dealing, then moves and swaps
+  // ---- 3. wave 0: longest-processing-time dealing. A step is one reduction of
+  // load * 256 + slot where loads stay below 2^24, two of the full loads else.
   if (tid < 64) {
     constexpr int kPer = kMaxSlots / 64;  // slots per lane: j = lane + 64 m
-    int32_t lreg[kPer];
+    if ((uint64_t)sm.w[0] * (uint32_t)p.W < (1u << 24)) {  // sm.w[0] is the largest
+      uint32_t key[kPer];
 #pragma unroll
-    for (int m = 0; m < kPer; ++m) lreg[m] = lane + 64 * m < p.k ? sm.load[lane + 64 * m] : 0x7fffffff;
-    for (int q = k0; q < p.W; ++q) {
-      uint32_t bl = 0xffffffffu, bj = 0xffffffffu;  // the lane's least loaded slot (lowest first)
+      for (int m = 0; m < kPer; ++m) {
+        const int j = lane + 64 * m;
+        key[m] = j < p.k ? ((uint32_t)sm.load[j] << 8) | (uint32_t)j : 0xffffffffu;
+      }
+      for (int q0 = k0; q0 < p.W; q0 += 64) {
+        const int cnt = min(64, p.W - q0);
+        const uint32_t wreg = lane < cnt ? (uint32_t)sm.w[q0 + lane] << 8 : 0u;
+        int dealt = 0;
+        for (int i = 0; i < cnt; ++i) {
+          const uint32_t least = wave_min_u32(min(min(key[0], key[1]), min(key[2], key[3])));
+          const uint32_t wq = (uint32_t)__builtin_amdgcn_readlane((int)wreg, i);
+          dealt = lane == i ? (int)(least & 255u) : dealt;
+#pragma unroll
+          for (int m = 0; m < kPer; ++m) key[m] += key[m] == least ? wq : 0u;
+        }
+        if (lane < cnt) sm.slot[q0 + lane] = (int16_t)dealt;
+      }
 #pragma unroll
       for (int m = 0; m < kPer; ++m)
-        if ((uint32_t)lreg[m] < bl) {
-          bl = (uint32_t)lreg[m];
-          bj = (uint32_t)(lane + 64 * m);
-        }
-      const uint32_t gl = wave_min_u32(bl);
-      const int j = (int)wave_min_u32(bl == gl ? bj : 0xffffffffu);
-      const int wq = sm.w[q];
+        if (lane + 64 * m < p.k) sm.load[lane + 64 * m] = (int32_t)(key[m] >> 8);
+    } else {
+      int32_t lreg[kPer];
+#pragma unroll
+      for (int m = 0; m < kPer; ++m) lreg[m] = lane + 64 * m < p.k ? sm.load[lane + 64 * m] : 0x7fffffff;
+      for (int q = k0; q < p.W; ++q) {
+        uint32_t bl = 0xffffffffu, bj = 0xffffffffu;  // the lane's least loaded slot (lowest first)
+#pragma unroll
+        for (int m = 0; m < kPer; ++m)
+          if ((uint32_t)lreg[m] < bl) {
+            bl = (uint32_t)lreg[m];
+            bj = (uint32_t)(lane + 64 * m);
+          }
+        const uint32_t gl = wave_min_u32(bl);
+        const int j = (int)wave_min_u32(bl == gl ? bj : 0xffffffffu);
+        const int wq = sm.w[q];
+#pragma unroll
+        for (int m = 0; m < kPer; ++m)
+          if (lane + 64 * m == j) lreg[m] += wq;
+        if (lane == 0) sm.slot[q] = (int16_t)j;
+      }
 #pragma unroll
       for (int m = 0; m < kPer; ++m)
-        if (lane + 64 * m == j) lreg[m] += wq;
-      if (lane == 0) sm.slot[q] = (int16_t)j;
+        if (lane + 64 * m < p.k) sm.load[lane + 64 * m] = lreg[m];
     }
+  }
+  if (tid < 2) {
+    sm.best[tid] = ~0ull;
+    sm.held[tid] = 0;
+  }
+  __syncthreads();
+
+  // Then moves and swaps, every wave over its part of the items: an option's key
+  // is (the resulting larger load, the rank of a's item, moves before swaps, the
+  // slot or rank of the other side), lowest first, so the choice does not depend
+  // on the order in which a's items are listed. The keys' array holds that list.
+  // A round is a chain of about 500 dependent instructions and three barriers,
+  // 2 us; one wave over all the items took 4 (the whole planner: 250 items in 64
+  // slots, 51 rounds 268 us before, 135 now; 131 in 32, 25 rounds 120, 72). Work
+  // groups of 256 or 512 threads take the same time.
+  for (int round = 0; round < p.max_rounds; ++round) {
+    const int cur = round & 1;
+    uint32_t tl = 0, aj = 0xffffffffu;  // the most loaded slot (lowest first), in every wave
+    for (int j = lane; j < p.k; j += 64) {
+      const uint32_t l = (uint32_t)sm.load[j];
+      if (l > tl) aj = (uint32_t)j;
+      tl = max(tl, l);
+    }
+    const int top = (int)wave_max_u32(tl);
+    const int a = (int)wave_min_u32(tl == (uint32_t)top ? aj : 0xffffffffu);
+    for (int q = tid; q < p.W; q += kThreads)
+      if (sm.slot[q] == a) sm.keys[atomicAdd(&sm.held[cur], 1)] = ((uint64_t)(uint32_t)sm.w[q] << 32) | (uint32_t)q;
+    __syncthreads();
+    const int ma = sm.held[cur];
+    uint64_t best = ~0ull;
+    for (int jq = tid; jq < p.W; jq += kThreads) {
+      const bool move = jq < p.k && jq != a;  // a move to slot jq
+      const int lm = sm.load[min(jq, p.k - 1)];
+      const int b = sm.slot[jq], lb = sm.load[b], wj = sm.w[jq];  // a swap with item jq
+      auto option = [&](uint64_t it) __attribute__((always_inline)) {
+        const int wa = (int)(it >> 32), d = wa - wj;
+        const int nm = max(top - wa, lm + wa), ns = max(top - d, lb + d);
+        if (move && wa > 0 && nm < top) {
+          const uint64_t key = ((uint64_t)(uint32_t)nm << 32) | ((uint32_t)it << 13) | (uint32_t)jq;
+          best = key < best ? key : best;
+        }
+        if (b != a && d > 0 && ns < top) {
+          const uint64_t key = ((uint64_t)(uint32_t)ns << 32) | ((uint32_t)it << 13) | (1u << 12) | (uint32_t)jq;
+          best = key < best ? key : best;
+        }
+      };
+      for (int i0 = 0; i0 < ma; i0 += 8) {  // eight reads in flight, not one after the other
+        uint64_t it[8];
 #pragma unroll
-    for (int m = 0; m < kPer; ++m)
-      if (lane + 64 * m < p.k) sm.load[lane + 64 * m] = lreg[m];
-    __builtin_amdgcn_wave_barrier();
-    for (int round = 0; round < p.max_rounds; ++round) {
-      uint32_t tl = 0;  // the most loaded slot (lowest first)
-      for (int j = lane; j < p.k; j += 64) tl = max(tl, (uint32_t)sm.load[j]);
-      tl = wave_max_u32(tl);
-      uint32_t aj = 0xffffffffu;
-      for (int j = lane; j < p.k; j += 64)
-        if ((uint32_t)sm.load[j] == tl) aj = min(aj, (uint32_t)j);
-      const int a = (int)wave_min_u32(aj);
-      const int top = (int)tl;
-      // ranks held by slot a, in rank order
-      int ma = 0;
-      for (int q0 = 0; q0 < p.W; q0 += 64) {
-        const int q = q0 + lane;
-        const bool in = q < p.W && sm.slot[q] == a;
-        const uint64_t mask = __ballot(in);
-        if (in) sm.alist[ma + __builtin_popcountll(mask & ((1ull << lane) - 1))] = (int16_t)q;
-        ma += __builtin_popcountll(mask);
+        for (int i = 0; i < 8; ++i) it[i] = sm.keys[min(i0 + i, ma - 1)];
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+          if (i0 + i < ma) option(it[i]);
       }
-      __builtin_amdgcn_wave_barrier();
-      // best option: lowest resulting larger load, then lowest position in a's
-      // list, moves before swaps, then lowest slot / rank
-      uint64_t best = ~0ull;
-      for (int pi = 0; pi < ma; ++pi) {
-        const int ia = sm.alist[pi];
-        const int wa = sm.w[ia];
-        for (int b = lane; b < p.k; b += 64) {
-          if (b == a) continue;
-          const int nw = max(top - wa, sm.load[b] + wa);
-          if (wa > 0 && nw < top) {
-            const uint64_t key = ((uint64_t)(uint32_t)nw << 32) | ((uint32_t)pi << 13) | (uint32_t)b;
-            best = key < best ? key : best;
-          }
-        }
-        for (int jq = lane; jq < p.W; jq += 64) {
-          const int b = sm.slot[jq];
-          if (b == a) continue;
-          const int d = wa - sm.w[jq];
-          const int nw = max(top - d, sm.load[b] + d);
-          if (d > 0 && nw < top) {
-            const uint64_t key = ((uint64_t)(uint32_t)nw << 32) | ((uint32_t)pi << 13) | (1u << 12) | (uint32_t)jq;
-            best = key < best ? key : best;
-          }
-        }
-      }
-      const uint32_t bhi = wave_min_u32((uint32_t)(best >> 32));
-      const uint32_t blo = wave_min_u32((uint32_t)(best >> 32) == bhi ? (uint32_t)best : 0xffffffffu);
-      if (bhi == 0xffffffffu && blo == 0xffffffffu) break;
-      best = ((uint64_t)bhi << 32) | blo;
-      const int pi = (int)((best >> 13) & 0x7ffff), kind = (int)((best >> 12) & 1), idx = (int)(best & 0xfff);
-      if (lane == 0) {
-        const int ia = sm.alist[pi];
-        if (kind == 0) {  // move item ia to slot idx
-          sm.load[a] -= sm.w[ia];
-          sm.load[idx] += sm.w[ia];
-          sm.slot[ia] = (int16_t)idx;
-        } else {  // swap item ia with item idx
-          const int b = sm.slot[idx], d = sm.w[ia] - sm.w[idx];
-          sm.load[a] -= d;
-          sm.load[b] += d;
-          sm.slot[ia] = (int16_t)b;
-          sm.slot[idx] = (int16_t)a;
-        }
-      }
-      __builtin_amdgcn_wave_barrier();
     }
+    const uint32_t bhi = wave_min_u32((uint32_t)(best >> 32));
+    const uint32_t blo = wave_min_u32((uint32_t)(best >> 32) == bhi ? (uint32_t)best : 0xffffffffu);
+    if (lane == 0 && bhi != 0xffffffffu)
+      atomicMin(reinterpret_cast<unsigned long long *>(&sm.best[cur]), ((unsigned long long)bhi << 32) | blo);
+    __syncthreads();
+    best = sm.best[cur];
+    if (best == ~0ull) break;  // the same for every thread
+    if (tid == 0) {
+      const int ia = (int)((best >> 13) & 0xfff), idx = (int)(best & 0xfff);
+      const bool swap = (best >> 12) & 1;  // item ia with item idx; else item ia to slot idx
+      const int b = swap ? sm.slot[idx] : idx, d = sm.w[ia] - (swap ? sm.w[idx] : 0);
+      atomicSub(&sm.load[a], d);
+      atomicAdd(&sm.load[b], d);
+      sm.slot[ia] = (int16_t)b;
+      if (swap) sm.slot[idx] = (int16_t)a;
+      sm.best[cur ^ 1] = ~0ull;  // the next round's; this round's were read before the barrier below
+      sm.held[cur ^ 1] = 0;
+    }
+    __syncthreads();
   }
   __syncthreads();
 
