@@ -28,7 +28,7 @@ import sys
 HERE = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(HERE)
 SRCS = [os.path.join(HERE, "csrc", f) for f in ("tree_attn.hip", "qkv_front.hip", "tree_plan.hip", "fp8_quant.hip", "fp8_gemm.hip",
-                                                 "gdn.hip", "gdn_chunk.hip", "gdn_conv.hip", "gdn_norm.hip")]
+                                                 "gdn.hip", "gdn_chunk.hip", "gdn_conv.hip", "gdn_norm.hip", "gdn_proj.hip")]
 # Extra flags per source (file name -> flags).
 SRC_FLAGS = {"tree_attn.hip": ["-fno-honor-nans", "-mno-amdgpu-ieee"]}
 # Matrix-core results in VGPRs, for every source but the GEMM, whose 256

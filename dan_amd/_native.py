@@ -145,7 +145,7 @@ class DanFp8GemmArgs(ctypes.Structure):
                 ("w_scale", _vp), ("bias", _vp), ("y", _vp), ("y_stride", _i64)]
 
 
-GDN_ABI_VERSION = 6
+GDN_ABI_VERSION = 7
 GDN_FORM_TOKEN, GDN_FORM_CHUNK = 0, 1
 GDN_CHUNK = 64
 
@@ -177,11 +177,17 @@ class DanGdnNormArgs(ctypes.Structure):
                 ("out", _vp), ("out_stride", _i64)]
 
 
+class DanGdnProjArgs(ctypes.Structure):
+    _fields_ = [("abi_version", _i32), ("dtype", _i32), ("rows", _i32), ("cols", _i32), ("hidden", _i32), ("reserved", _i32),
+                ("x", _vp), ("x_stride", _i64), ("w0", _vp), ("w0_stride", _i64), ("w1", _vp), ("w1_stride", _i64),
+                ("y0", _vp), ("y0_stride", _i64), ("y1", _vp), ("y1_stride", _i64)]
+
+
 EXPORTS = ("dan_tree_attn_fwd", "dan_tree_attn_fwd_noalloc", "dan_tree_attn_stage_f16", "dan_tree_attn_stage_f16_pair", "dan_tree_attn_tile_q", "dan_tree_attn_head_groups", "dan_tree_attn_workspace_size",
            "dan_tree_attn_last_error", "dan_tree_attn_abi_version", "dan_qkv_front", "dan_qkv_front_abi_version",
            "dan_tree_attn_plan", "dan_tree_attn_plan_slots", "dan_tree_attn_plan_abi_version",
            "dan_fp8_quantize", "dan_fp8_gemm", "dan_fp8_tiled_bytes", "dan_fp8_abi_version", "dan_gdn_fwd", "dan_gdn_workspace_size", "dan_gdn_abi_version",
-           "dan_gdn_conv", "dan_gdn_gated_norm")
+           "dan_gdn_conv", "dan_gdn_gated_norm", "dan_gdn_project")
 
 _lock = threading.Lock()
 _lib = None
@@ -245,6 +251,8 @@ def load(path=LIB_PATH):
         lib.dan_gdn_conv.restype = ctypes.c_int
         lib.dan_gdn_gated_norm.argtypes = [ctypes.POINTER(DanGdnNormArgs), _vp]
         lib.dan_gdn_gated_norm.restype = ctypes.c_int
+        lib.dan_gdn_project.argtypes = [ctypes.POINTER(DanGdnProjArgs), _vp]
+        lib.dan_gdn_project.restype = ctypes.c_int
         lib.dan_gdn_abi_version.argtypes = []
         lib.dan_gdn_abi_version.restype = ctypes.c_int
         got = (lib.dan_tree_attn_abi_version(), lib.dan_qkv_front_abi_version(), lib.dan_tree_attn_plan_abi_version(),
@@ -309,6 +317,7 @@ call_fp8_gemm = Entry("dan_fp8_gemm", DanFp8GemmArgs)
 call_gdn = Entry("dan_gdn_fwd", DanGdnArgs)
 call_gdn_conv = Entry("dan_gdn_conv", DanGdnConvArgs)
 call_gdn_gated_norm = Entry("dan_gdn_gated_norm", DanGdnNormArgs)
+call_gdn_project = Entry("dan_gdn_project", DanGdnProjArgs)
 
 
 def last_error(lib):

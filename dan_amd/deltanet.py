@@ -23,7 +23,7 @@ import torch
 from torch import nn
 
 from . import _native
-from .attention import _DTYPES, Batch
+from .attention import _DTYPES, Batch, _num_cus
 
 
 def _row_ok(t):
@@ -151,6 +151,44 @@ def _gated_norm(out, z, weight, eps):
         _native.stream(out.device), _native.GDN_ABI_VERSION, _DTYPES[out.dtype], n, hv, dv, _native.f32(float(eps)),
         out.data_ptr(), hv * dv, z.data_ptr(), z.stride(0), weight.data_ptr(), y.data_ptr(), hv * dv)
     return y
+
+
+def _narrow_pair(x, first, second):
+    """``first(x), second(x)`` of two linears of the same narrow width on x
+    [N, K]: one ``dan_gdn_project`` launch where both are plain nn.Linear
+    modules without bias, hooks or wanted gradients whose layout and types it
+    takes, else the modules' own calls."""
+    w0, w1 = first.weight, second.weight
+    if (not (_plain(first) and _plain(second)) or type(x) is not torch.Tensor or not x.is_cuda or x.dim() != 2
+            or torch.compiler.is_compiling() or torch.is_autocast_enabled("cuda")
+            or torch.is_grad_enabled() and (x.requires_grad or w0.requires_grad or w1.requires_grad)
+            or x.dtype not in (torch.bfloat16, torch.float16) or not w0.dtype == w1.dtype == x.dtype
+            or not w0.device == w1.device == x.device or w0.shape != w1.shape or w0.shape[1] != x.shape[1]
+            or w0.shape[0] % 4 or not w0.shape[0] or x.shape[1] % 32 or not 0 < x.shape[1] <= NARROW_HIDDEN
+            or -(-x.shape[0] // 32) * -(-w0.shape[0] // 16) > _num_cus(x.device)
+            or not (_row_ok(x) and _row_ok(w0) and _row_ok(w1)) or min(x.stride(0), w0.stride(0), w1.stride(0)) < x.shape[1]):
+        return first(x), second(x)
+    (n, k), cols = x.shape, w0.shape[0]
+    y0, y1 = (torch.empty((n, cols), dtype=x.dtype, device=x.device) for _ in range(2))
+    _native.call_gdn_project(
+        _native.stream(x.device), _native.GDN_ABI_VERSION, _DTYPES[x.dtype], n, cols, k, 0, x.data_ptr(), x.stride(0),
+        w0.data_ptr(), w0.stride(0), w1.data_ptr(), w1.stride(0), y0.data_ptr(), cols, y1.data_ptr(), cols)
+    return y0, y1
+
+
+# Hidden sizes up to which ``_narrow_pair`` launches its own kernel, where 32 rows and
+# 16 columns a work group make at most one group per CU. GPU time of the launch
+# against the two linears', microseconds: hidden 2048, 834 rows x 16 columns 7.2 / 10.5,
+# 834 x 64 7.5 / 10.4, 2779 x 32 9.6 / 11.9, 8192 x 16 9.7 / 16.8; past one group per CU
+# 8192 x 32 17.6 / 17.3; hidden 5120, 834 x 16 15.2 / 12.2.
+NARROW_HIDDEN = 2560
+
+
+def _plain(m):
+    """m is an nn.Linear without bias whose call is F.linear and nothing else."""
+    return (type(m) is nn.Linear and type(m.weight) is nn.Parameter and m.bias is None and "forward" not in m.__dict__
+            and not (m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks)
+            and not torch.nn.modules.module._has_any_global_hook())
 
 
 @dataclass
@@ -335,7 +373,8 @@ class DeltaNet(nn.Module):
 
     def forward(self, x, segments):
         n = x.shape[0]
-        qkv, z, b, a = self.in_proj_qkv(x), self.in_proj_z(x), self.in_proj_b(x), self.in_proj_a(x)
+        qkv, z = self.in_proj_qkv(x), self.in_proj_z(x)
+        b, a = _narrow_pair(x, self.in_proj_b, self.in_proj_a)
         k1 = self.kernel - 1
         lay = getattr(segments, "recurrent", None)
         if lay is None or lay.rows != n:

@@ -29,7 +29,7 @@
 extern "C" {
 #endif
 
-#define DAN_GDN_ABI_VERSION 6
+#define DAN_GDN_ABI_VERSION 7
 
 /* Tokens per chunk of the chunked form. */
 #define DAN_GDN_CHUNK 64
@@ -163,6 +163,26 @@ typedef struct {
 
 /* Replaces dan/fused.py:52-56 as dan/models/qwen3_5.py:226 calls it. */
 int dan_gdn_gated_norm(const DanGdnNormArgs *args, void *stream);
+
+/* The layer's two narrow projections, one value head a column:
+ *   y0 = rnd(x w0^T), y1 = rnd(x w1^T)      (fp32 sums, rounded to dtype once)
+ * (GDN ABI 7) */
+typedef struct {
+  int32_t abi_version;  /* DAN_GDN_ABI_VERSION */
+  int32_t dtype;        /* DanDtype of all five: bf16 or f16 */
+  int32_t rows;         /* of x, y0 and y1 */
+  int32_t cols;         /* of y0 and of y1; a multiple of 4 */
+  int32_t hidden;       /* a multiple of 32 */
+  int32_t reserved;
+  const void *x; int64_t x_stride;    /* [rows, hidden], row strides in elements: multiples of 8, 16-byte aligned rows */
+  const void *w0; int64_t w0_stride;  /* [cols, hidden] */
+  const void *w1; int64_t w1_stride;
+  void *y0; int64_t y0_stride;        /* [rows, cols]: strides multiples of 4, 8-byte aligned rows */
+  void *y1; int64_t y1_stride;
+} DanGdnProjArgs;
+
+/* Replaces in_proj_b and in_proj_a of dan/models/qwen3_5.py:186-189. */
+int dan_gdn_project(const DanGdnProjArgs *args, void *stream);
 
 int dan_gdn_abi_version(void);
 
