@@ -88,7 +88,8 @@ typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
 // The bf16 scan takes 16 state columns per work group while that makes at most
 // one group per CU, else 32. A chunk's step of 16 columns is the shorter, but
 // two groups on a CU take longer than one of twice the columns. The whole rule
-// (16 value heads of 128 columns, microseconds at 16 / 32 columns): 4 runs of
+// (16 value heads of 128 columns), when the choice was measured (every call has
+// become 10 to 25 % faster since), microseconds at 16 / 32 columns: 4 runs of
 // 1000 tokens 82.9 / 71.0, 8 of 800 128.8 / 96.4, 45 branches of 16-96 108.9 /
 // 80.7, 150 of 1-200 499 / 356; with one group per CU 2 runs of 1000 take 53.1 / 61.7.
 constexpr int kScan16Groups = 256;
@@ -726,8 +727,10 @@ struct BfLds {
   static constexpr int yHi = sLo + COLS * kPS * 2, yLo = yHi + COLS * kPC * 2;
   static constexpr int dHi = yLo + COLS * kPC * 2, dLo = dHi + COLS * kPC * 2;
   static constexpr int eHi = dLo + COLS * kPC * 2, eLo = eHi + COLS * kPC * 2;
-  static constexpr int vRows = eLo + COLS * kPC * 2, vWave = 16 * COLS * 2;
-  static constexpr int bytes = vRows + 4 * vWave;
+  static constexpr int vRows = dHi, vWave = 16 * COLS * 2;  // in phase 0, when D's planes hold nothing
+  static constexpr int kqRows = eLo + COLS * kPC * 2, kqWave = 2 * 16 * kDk * 2;  // a wave's 16 rows of k, then of q
+  static_assert(4 * vWave <= COLS * kPC * 2, "v's rows fit D's hi plane");
+  static constexpr int bytes = kqRows + 4 * kqWave;
   static_assert(sHi % 16 == 0 && (kPS * 2) % 16 == 0 && (kPC * 2) % 16 == 0, "16-byte operand reads");
 };
 
@@ -758,7 +761,7 @@ __device__ inline void put4_bf(uint8_t *hi_plane, uint8_t *lo_plane, int off, co
 // after its last use in the chunk before).
 template <int COLS>
 struct OpsBf {
-  u32x4 ka[4], qa[4];   // k, q row 16 rb + l16, d 32 j + 8 g4 .. + 7
+  u32x4 k[4], q[4];     // k, q rows 16 rb + 4 j + lane / 16, d 8 (lane % 16) .. + 7
   f32x4 va, vb, vs;     // the row factors of rows 16 rb + 4 g4 .. + 3
   float vq;             // r_q Dk^-1/2 gamma of row 16 rb + l16
   uint32_t v[COLS / 8]; // row 16 rb + lane / 4 of v, columns COLS / 4 (lane % 4) .. (kVec)
@@ -786,14 +789,19 @@ struct OpsBf {
 // 16 receives element p of the pieces that lanes c, c + 4, c + 8 and c + 12
 // address). kVec: v's and out's rows allow these accesses; else one element at
 // a time, as any alignment does.
-// A chain of chunk steps, bound by each step's issue and its three barriers,
-// not by memory. The step before had 32 more LDS accesses (the fp32 master lay
-// there), read the record in 16-byte pieces of different rows, stored 2 bytes
-// at a time and split one value at a time. The whole rule with its preparation
-// (16 value heads of 128 columns), before and now, microseconds: 1 run of 1462
-// tokens 98.1, 64.5; 5 of 286-1843 165.7, 130.8; 45 branches of 16-96 105.3,
-// 80.7. The state's products on four waves and the output's on four others: 73.0,
-// 125.0, 103.8, not taken.
+// k and q come as whole rows (a load of 64 lanes: 4 rows) and are turned into
+// operands through the wave's own LDS as well, a chunk ahead.
+// A chain of chunk steps, bound by each step's issue, its three barriers and the
+// loads' way through the CU's address unit (without any load 1 run of 1462 tokens
+// takes 41 us), not by memory. The step before had 32 more LDS accesses (the fp32
+// master lay there), read the record, k and q in 16-byte pieces of 16 rows, stored
+// 2 bytes at a time, split one value at a time and loaded the last chunk twice. The
+// whole rule (16 value heads of 128 columns) with the preparation as it is now,
+// microseconds: with all of that and the slower preparation 1 run of 1462 tokens
+// took 98.1, 5 of 286-1843 165.7, 45 branches of 16-96 105.3; with pieces of 16 rows
+// and the double load of the last chunk 59.2, 120.4 and 69.9; now 55.7, 107.9, 61.0.
+// The state's products on four waves and the output's on four others took 8 to
+// 30 % longer, two accumulators a chain 1 to 8 %.
 template <int COLS, bool kVec>
 __global__ __attribute__((amdgpu_flat_work_group_size(256, 256), amdgpu_waves_per_eu(2)))
 void chunk_scan_bf16_kernel(const Params p) {
@@ -836,12 +844,13 @@ void chunk_scan_bf16_kernel(const Params p) {
   };
   auto load0 = [&](OpsBf<COLS> &o, int t0, int s) __attribute__((always_inline)) {
     const int L = min(kC, end - t0);
-    const int64_t tr = t0 + min(ri, L - 1);
     const float *vec = reinterpret_cast<const float *>(recb(s)) + kVecBf;
 #pragma unroll
-    for (int j = 0; j < 4; ++j) o.ka[j] = *(const DAN_GLOBAL u32x4 *)(kh + tr * p.k_st + 32 * j + 8 * g4);
-#pragma unroll
-    for (int j = 0; j < 4; ++j) o.qa[j] = *(const DAN_GLOBAL u32x4 *)(qh + tr * p.q_st + 32 * j + 8 * g4);
+    for (int j = 0; j < 4; ++j) {
+      const int64_t t = t0 + min(16 * rb + 4 * j + g4, L - 1);
+      o.k[j] = *(const DAN_GLOBAL u32x4 *)(kh + t * p.k_st + 8 * l16);
+      o.q[j] = *(const DAN_GLOBAL u32x4 *)(qh + t * p.q_st + 8 * l16);
+    }
     o.va = *(const DAN_GLOBAL f32x4 *)(vec + 0 * kC + ro);
     o.vb = *(const DAN_GLOBAL f32x4 *)(vec + 1 * kC + ro);
     if constexpr (kVec) {
@@ -886,12 +895,28 @@ void chunk_scan_bf16_kernel(const Params p) {
     return *reinterpret_cast<const u32x4 *>(lds + plane + 2 * (c * stride + k0));
   };
 
+  // The wave's k and q rows to its own LDS, 16-byte piece c of row x at piece
+  // c ^ x, and its operands of them: row l16, d 32 j + 8 g4 .. + 7.
+  uint8_t *kq = lds + LB::kqRows + rb * LB::kqWave;
+  auto put_kq = [&](const OpsBf<COLS> &o) __attribute__((always_inline)) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int row = 4 * j + g4, at = row * kDk * 2 + 16 * (l16 ^ row);
+      *reinterpret_cast<u32x4 *>(kq + at) = o.k[j];
+      *reinterpret_cast<u32x4 *>(kq + LB::kqWave / 2 + at) = o.q[j];
+    }
+  };
+  auto get_kq = [&](int q, int j) __attribute__((always_inline)) {
+    return *reinterpret_cast<const u32x4 *>(kq + q * (LB::kqWave / 2) + l16 * kDk * 2 + 16 * ((4 * j + g4) ^ l16));
+  };
+
   OpsBf<COLS> op;
   int s = r + row0 / kC;
   if (row0 < end) {
     load0(op, row0, s);
     load1(op, s);
     load2(op, s);
+    put_kq(op);
   }
 #pragma unroll
   for (int mb = 0; mb < 2; ++mb)
@@ -901,8 +926,8 @@ void chunk_scan_bf16_kernel(const Params p) {
   for (int t0 = row0; t0 < end; t0 += kC, ++s) {
     const int L = min(kC, end - t0), jmax = (L - 1) >> 5;
     const int jt = min(rb >> 1, jmax);  // the wave's last 32-row block of T Y and A D
-    const bool more = t0 + kC < end;    // the next chunk (this one again after the last: the loads stay in bounds)
-    const int tn = more ? t0 + kC : t0, sn = more ? s + 1 : s;
+    const bool more = t0 + kC < end;    // after the last chunk nothing is loaded
+    const int tn = t0 + kC, sn = s + 1;
 
     // phase 0: K S and Q S; Y = diag(beta) V - diag(beta gamma r_k) K S
     if constexpr (kVec) {  // the wave's 16 rows of v, as they lie (read back below, by this wave only)
@@ -916,16 +941,18 @@ void chunk_scan_bf16_kernel(const Params p) {
 #pragma unroll
     for (int n = 0; n < NC; ++n) x[n] = o1[n] = f32x4{};
 #pragma unroll
-    for (int j = 0; j < 4; ++j)
+    for (int j = 0; j < 4; ++j) {
+      const u32x4 ka = get_kq(0, j), qa = get_kq(1, j);
 #pragma unroll
       for (int n = 0; n < NC; ++n) {
         const u32x4 bh = rd(LB::sHi, kPS, 16 * n + l16, 32 * j + 8 * g4);
         const u32x4 bl = rd(LB::sLo, kPS, 16 * n + l16, 32 * j + 8 * g4);
-        x[n] = mma_bf(op.ka[j], bh, x[n]);
-        o1[n] = mma_bf(bh, op.qa[j], o1[n]);
-        x[n] = mma_bf(op.ka[j], bl, x[n]);
-        o1[n] = mma_bf(bl, op.qa[j], o1[n]);
+        x[n] = mma_bf(ka, bh, x[n]);
+        o1[n] = mma_bf(bh, qa, o1[n]);
+        x[n] = mma_bf(ka, bl, x[n]);
+        o1[n] = mma_bf(bl, qa, o1[n]);
       }
+    }
 #pragma unroll
     for (int n = 0; n < NC; ++n) {
       f32x4 v;
@@ -948,7 +975,7 @@ void chunk_scan_bf16_kernel(const Params p) {
       for (int rr = 0; rr < 4; ++rr) y[rr] = op.vb[rr] * v[rr] - op.va[rr] * x[n][rr];
       put4_bf(lds + LB::yHi, lds + LB::yLo, 2 * ((16 * n + l16) * kPC + ro), y);
     }
-    load0(op, tn, sn);
+    if (more) load0(op, tn, sn);
     barrier_lds();
 
     // phase 1: D = T Y
@@ -977,7 +1004,7 @@ void chunk_scan_bf16_kernel(const Params p) {
         put4_bf(lds + LB::eHi, lds + LB::eLo, 2 * ((16 * n + l16) * kPC + ro), e);
       }
     }
-    load1(op, sn);
+    if (more) load1(op, sn);
     barrier_lds();
 
     // phase 2: O = diag(r_q Dk^-1/2 gamma) Q S + A D; S <- gamma_63 S + K^T Ds
@@ -1033,7 +1060,10 @@ void chunk_scan_bf16_kernel(const Params p) {
 #pragma unroll
       for (int n = 0; n < NC; ++n) put4_bf(lds + LB::sHi, lds + LB::sLo, 2 * ((16 * n + l16) * kPS + srow(mb)), st[mb][n]);
     }
-    load2(op, sn);
+    if (more) {
+      load2(op, sn);
+      put_kq(op);
+    }
     barrier_lds();  // the new state is whole, and every read of this chunk's Y, D and S is done
   }
 #pragma unroll
