@@ -85,14 +85,15 @@ typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
 
-// The bf16 scan takes 16 state columns per work group while that makes at most
-// one group per CU, else 32. A chunk's step of 16 columns is the shorter, but
-// two groups on a CU take longer than one of twice the columns. The whole rule
-// (16 value heads of 128 columns), when the choice was measured (every call has
-// become 10 to 25 % faster since), microseconds at 16 / 32 columns: 4 runs of
-// 1000 tokens 82.9 / 71.0, 8 of 800 128.8 / 96.4, 45 branches of 16-96 108.9 /
-// 80.7, 150 of 1-200 499 / 356; with one group per CU 2 runs of 1000 take 53.1 / 61.7.
-constexpr int kScan16Groups = 256;
+// The bf16 scan takes 16 state columns per work group while all groups are
+// resident at once, two per CU, else 32: a chunk's step of 16 columns is the
+// shorter, so the longest run ends sooner, but the groups' total work is more.
+// The whole rule (16 value heads of 128 columns), microseconds at 16 / 32 columns:
+// 1 run of 1462 tokens (128 groups) 55.4 / 71.4, 2000 + 300 + 900 (384) 82.9 / 99.8,
+// 3 of 1500 87.8 / 87.0, 4 of 1000 (512) 63.6 / 63.1; past that it depends on how
+// unequal the runs are: 5 of 286-1843 (640) 92 / 108, but 5 of 1000 91 / 80, 6 of
+// 400-1900 116 / 111, 8 of 800 95 / 79, 45 branches of 16-96 77 / 62.
+constexpr int kScan16Groups = 512;
 
 struct Params {
   const int32_t *cu;

@@ -48,7 +48,7 @@ def test_misaligned_v_and_out(gpu, lengths, dv):
 
 def test_column_widths_agree(gpu):
     """One run alone (few work groups, 16 columns each) and among many (32): the same bits."""
-    lengths = [130, 1, 64] * 13  # 39 runs x 4 heads x 8 column blocks of 16: over one group per CU
+    lengths = [130, 1, 64] * 13  # 39 runs x 4 heads x 8 column blocks of 16: more groups than two per CU hold
     args = _inputs(gpu, lengths, 4, 4, 128)
     o, f = delta_rule(*args, form="chunk")
     for i in (0, 1, 2, 38):
