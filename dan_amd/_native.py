@@ -24,7 +24,7 @@ LIB_DIR = os.path.join(HERE, "_lib")
 LIB_NAME = "libdan_tree_attn.so"
 LIB_PATH = os.path.join(LIB_DIR, LIB_NAME)
 
-ABI_VERSION = 9
+ABI_VERSION = 10
 KEY_TILE = 64
 SCRATCH_BYTES = 32 << 20  # DAN_TREE_ATTN_SCRATCH_BYTES: dan_tree_attn_fwd_noalloc's V^T scratch per GPU
 
@@ -77,10 +77,15 @@ class DanTreeAttnArgs(ctypes.Structure):
                 ("col_seg", _vp),
                 ("workspace", _vp), ("workspace_bytes", _i64), ("phases", _i32),
                 ("units", _vp), ("sched_off", _vp), ("num_slots", _i32), ("counts", _vp),
-                ("pasts_host", _vp), ("key_halves", _i32)]
+                ("pasts_host", _vp), ("key_halves", _i32), ("num_saves", _i32), ("save_layout", _i32), ("saves", _vp)]
 
 
 INLINE_PASTS = 8  # DAN_TREE_ATTN_INLINE_PASTS
+INLINE_SAVES = 8  # DAN_TREE_ATTN_INLINE_SAVES
+
+
+class DanTreeAttnSave(ctypes.Structure):
+    _fields_ = [("start", _i32), ("len", _i32), ("k_dst", _vp), ("v_dst", _vp)]
 
 
 STAGE_PARTIALS = 1024  # DAN_TREE_ATTN_STAGE_PARTIALS

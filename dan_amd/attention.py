@@ -151,11 +151,53 @@ def attend(q, k, v, segments, layer, scale=None, *, q_scale=None, k_scale=None, 
     ``save=False`` skips the clones, for a caller whose front end already
     filled ``saved[layer]`` (``dan_amd.front.qkv_front``)."""
     fp8 = q.dtype == E4M3
+    if save and (todo := _launch_saves(k, v, segments)):  # the launch writes these
+        kvs, table = _save_table(k, v, todo)
+        out = _attend_fused(q, k, v, segments, layer, scale, saves=table)
+        for s, kv in zip(todo, kvs):
+            s.saved[layer] = kv
+        return out
     for s in segments if save else ():
         if s.save:
             kv = (k[:, s.start:s.start + s.save].clone(), v[:, s.start:s.start + s.save].clone())
             s.saved[layer] = kv + (k_scale.clone(), v_scale.clone()) if fp8 and k_scale is not None else kv
     return _attend_fused(q, k, v, segments, layer, scale, (q_scale, k_scale, v_scale) if fp8 else None)
+
+
+def _launch_saves(k, v, segments):
+    """The saving segments whose rows ``attend``'s launch copies; none of them
+    where it clones instead: more than INLINE_SAVES, other types than bf16 and
+    fp16, a single row or kv head, rows past the packed ones or the segment's
+    own, tracing, gradients, or a k or v whose heads overlap its tokens."""
+    todo = [s for s in segments if s.save]
+    if (not 0 < len(todo) <= _native.INLINE_SAVES or type(k) is not torch.Tensor or type(v) is not torch.Tensor
+            or k.dtype not in (torch.bfloat16, torch.float16) or v.dtype != k.dtype or k.dim() != 3 or v.shape != k.shape
+            or not k.is_cuda or k.device != v.device or torch.compiler.is_compiling()
+            or torch.is_grad_enabled() and (k.requires_grad or v.requires_grad)):
+        return []
+    hkv, n, d = k.shape
+    if hkv < 2 or any(not (0 <= s.start and 1 < s.save <= min(n, s.end) - s.start) for s in todo):
+        return []  # (a clone keeps the stride of a dimension of one, too)
+    if k.stride(0) == k.stride(1) or v.stride(0) == v.stride(1):
+        return []
+    return todo
+
+
+def _save_table(k, v, todo):
+    """New (k, v) tensors for the saves ``todo``, in the order of dimensions
+    that a clone keeps, and the ``DanTreeAttnSave`` entries that name them
+    with their layout bits."""
+    hkv, _, d = k.shape
+    by_token = [t.stride(0) < t.stride(1) for t in (k, v)]
+
+    def new(rows, by_token):
+        if by_token:
+            return torch.empty((rows, hkv, d), dtype=k.dtype, device=k.device).transpose(0, 1)
+        return torch.empty((hkv, rows, d), dtype=k.dtype, device=k.device)
+
+    kvs = [(new(s.save, by_token[0]), new(s.save, by_token[1])) for s in todo]
+    table = (_native.DanTreeAttnSave * len(todo))(*((s.start, s.save, kd.data_ptr(), vd.data_ptr()) for s, (kd, vd) in zip(todo, kvs)))
+    return kvs, (table, by_token[0] + 2 * by_token[1])
 
 
 def _check_inputs(q, k, v):
@@ -339,8 +381,9 @@ def _num_cus(device):
 
 
 def _attend_fused(q, k, v, segments, layer, scale, fp8_scales=None, phases=_native.PHASES_ALL, noalloc=False,
-                  workspace=None):
-    """The kernel call behind ``attend`` (no save side effect). ``phases``
+                  workspace=None, saves=None):
+    """The kernel call behind ``attend`` (no save side effect but the entries
+    of ``saves``, which the launch fills). ``phases``
     selects the launches (the C ABI's ``phases``); a split call passes its own
     ``workspace`` (``workspace_bytes`` bytes of uint8 on the device) so that
     the attention-only launch reads the V^T copy an earlier PHASE_PACK or full
@@ -361,7 +404,7 @@ def _attend_fused(q, k, v, segments, layer, scale, fp8_scales=None, phases=_nati
     # an attention-only launch has no copy before it that would fill the prefix table
     args, pasts_host = _call_args(q, k, v, segments, layer, scale, fp8_scales, phases, noalloc,
                                   upload=phases == _native.PHASE_ATTEND)
-    return _launch_tree_attn(*args, workspace, pasts_host)
+    return _launch_tree_attn(*args, workspace, pasts_host, saves)
 
 
 @functools.lru_cache(maxsize=None)
@@ -464,9 +507,10 @@ def tree_attn(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, tables: List[to
     return _launch_tree_attn(q, k, v, tables, scales, meta, scale, workspace)
 
 
-def _launch_tree_attn(q, k, v, tables, scales, meta, scale, workspace, pasts_host=None):
+def _launch_tree_attn(q, k, v, tables, scales, meta, scale, workspace, pasts_host=None, saves=None):
     """The body of ``tree_attn``; ``pasts_host`` (uint8, on the host): the
-    prefix-cache table's entries, which the launch writes to the table."""
+    prefix-cache table's entries, which the launch writes to the table;
+    ``saves``: ``DanTreeAttnSave`` entries it fills, and their layout bits."""
     lib = _native.load()
     h, n, d = q.shape
     hkv = k.shape[0]
@@ -491,7 +535,8 @@ def _launch_tree_attn(q, k, v, tables, scales, meta, scale, workspace, pasts_hos
                work_d.data_ptr(), num_work, key_lo_d.data_ptr(), tile_q, vt_cols, col_seg_d.data_ptr(),
                0 if ws is None else ws.data_ptr(), 0 if ws is None else nbytes, phases,
                units.data_ptr(), sched_off.data_ptr(), slots, 0 if counts is None else counts.data_ptr(),
-               0 if pasts_host is None else pasts_host.data_ptr(), _layout(h, hkv, d)[0] // tile_q)
+               0 if pasts_host is None else pasts_host.data_ptr(), _layout(h, hkv, d)[0] // tile_q,
+               *((0, 0, 0) if saves is None else (len(saves[0]), saves[1], ctypes.addressof(saves[0]))))
     return out.transpose(0, 1)
 
 

@@ -169,7 +169,19 @@ struct PackParams {
   DanPastDesc *pasts_out;
   int32_t num_inline;
   DanPastDesc inl[DAN_TREE_ATTN_INLINE_PASTS];
+  // Prefix saves (16-bit k and v): work groups from `pack_blocks` on copy rows
+  // of k and v. As two clones of the saving segment a call of 834 tokens took
+  // 31.6 us, now 26.7 (16 KB of rows a work group).
+  const void *k;
+  int64_t k_st, k_sh;
+  int32_t pack_blocks, num_saves, save_layout;
+  DanTreeAttnSave saves[DAN_TREE_ATTN_INLINE_SAVES];
 };
+constexpr int kSavePieces = 4;  // 16-byte pieces a thread of a save's work groups copies
+// Work groups of a save of `len` tokens.
+__host__ __device__ inline int64_t save_blocks(int64_t len, int num_kv_heads, int head_dim) {
+  return (2 * len * num_kv_heads * (head_dim / 8) + 256 * kSavePieces - 1) / (256 * kSavePieces);
+}
 
 // ---------------------------------------------------------------- element I/O
 // Kernel pointers arrive inside a struct, so the compiler cannot prove they are
@@ -608,8 +620,45 @@ __host__ __device__ inline int vt_exponent(float amax) {
 // 2^e as an fp32 (exact for e in [-126, 127]).
 __device__ inline float exp2i(int e) { return __builtin_bit_cast(float, (uint32_t)(e + 127) << 23); }
 
+// Work group `block` of the saves' copy.
+template <int D>
+__device__ inline void copy_saves(const PackParams &p, int64_t block) {
+  const __attribute__((address_space(4))) uint8_t *args = (const __attribute__((address_space(4))) uint8_t *)__builtin_amdgcn_kernarg_segment_ptr();
+  const DanTreeAttnSave *saves = (const DanTreeAttnSave *)(args + __builtin_offsetof(PackParams, saves));
+  int i = 0;
+  for (; i < p.num_saves - 1; ++i) {
+    const int64_t n = save_blocks(saves[i].len, p.num_kv_heads, D);
+    if (block < n) break;
+    block -= n;
+  }
+  const int start = saves[i].start, len = saves[i].len;
+  void *dst[2] = {saves[i].k_dst, saves[i].v_dst};
+  const int64_t half = (int64_t)len * p.num_kv_heads * (D / 8);
+  u32x4 x[kSavePieces];
+  int64_t at[kSavePieces];
+#pragma unroll
+  for (int m = 0; m < kSavePieces; ++m) {
+    at[m] = (block * kSavePieces + m) * 256 + threadIdx.x;
+    const int64_t c = min(at[m], 2 * half - 1), o = c < half ? c : c - half, row = o / (D / 8);
+    const bool by_token = p.save_layout >> (c < half ? 0 : 1) & 1;
+    const int inner = by_token ? p.num_kv_heads : len, hi = (int)(row / inner), lo = (int)(row % inner);
+    const int head = by_token ? lo : hi, tok = start + (by_token ? hi : lo);
+    const uint16_t *src = c < half ? static_cast<const uint16_t *>(p.k) + head * p.k_sh + tok * p.k_st
+                                   : static_cast<const uint16_t *>(p.v) + head * p.v_sh + tok * p.v_st;
+    x[m] = *gbl(reinterpret_cast<const u32x4 *>(src + 8 * (o % (D / 8))));
+  }
+#pragma unroll
+  for (int m = 0; m < kSavePieces; ++m)
+    if (at[m] < 2 * half) {
+      const int64_t o = at[m] < half ? at[m] : at[m] - half;
+      *gbl_mut(static_cast<u32x4 *>(at[m] < half ? dst[0] : dst[1]) + o) = x[m];
+    }
+}
+
 template <typename TV, int D>
 __global__ __launch_bounds__(256) void vt_pack_kernel(const PackParams p) {
+  if constexpr (sizeof(TV) == 2)
+    if (p.num_saves > 0 && (int)blockIdx.x >= p.pack_blocks) return copy_saves<D>(p, (int)blockIdx.x - p.pack_blocks);
   constexpr bool kF8 = std::is_same<TV, E4M3>::value;
   constexpr int kPasses = D / 64;  // (8-value d chunk, key pair) items per thread
   // tile: row d = 32 dwords, dword kp holding keys 2 kp and 2 kp + 1 (fp16) at
@@ -1775,6 +1824,18 @@ int dan_tree_attn_fwd(const DanTreeAttnArgs *a, void *stream) {
   if (!f8 && (!a->q_scale != !a->k_scale || (a->q_scale && !f32)))
     return fail(DAN_ERR_INVALID_ARGUMENT, "q_scale and k_scale go together, and only with e4m3 or fp32-staged inputs");
   if (!finite_positive(a->scale)) return fail(DAN_ERR_INVALID_ARGUMENT, "scale must be finite and > 0");
+  if (a->save_layout < 0 || a->save_layout > 3) return fail(DAN_ERR_INVALID_ARGUMENT, "save_layout %d: bits 0 and 1", a->save_layout);
+  if (a->num_saves < 0 || a->num_saves > DAN_TREE_ATTN_INLINE_SAVES || (a->num_saves && (!a->saves || !(bf16 || f16))))
+    return fail(DAN_ERR_INVALID_ARGUMENT, "num_saves %d: 0 to %d host entries, with bf16 or f16 inputs", a->num_saves, DAN_TREE_ATTN_INLINE_SAVES);
+  int64_t save_grid = 0;
+  for (int i = 0; i < a->num_saves; ++i) {
+    const DanTreeAttnSave &sv = a->saves[i];
+    if (sv.start < 0 || sv.len <= 0 || sv.len > a->num_tokens - sv.start)
+      return fail(DAN_ERR_INVALID_ARGUMENT, "save %d: tokens %d + %d of %d", i, sv.start, sv.len, a->num_tokens);
+    if (!sv.k_dst || !sv.v_dst || (((uintptr_t)sv.k_dst | (uintptr_t)sv.v_dst) & 15))
+      return fail(DAN_ERR_INVALID_ARGUMENT, "save %d: destinations must be 16-byte aligned", i);
+    save_grid += save_blocks(sv.len, Hkv, D);
+  }
   if (a->phases < DAN_TREE_ATTN_PHASES_ALL || a->phases > DAN_TREE_ATTN_PHASE_ATTEND)
     return fail(DAN_ERR_INVALID_ARGUMENT, "phases %d: 0 (all), 1 (pack) or 2 (attend)", a->phases);
   const int64_t need = dan_tree_attn_workspace_size(Hkv, D, a->vt_cols);
@@ -1802,7 +1863,7 @@ int dan_tree_attn_fwd(const DanTreeAttnArgs *a, void *stream) {
   const int chunks = (rep + hpw - 1) / hpw;
   const int64_t units = (int64_t)a->num_work * Hkv * chunks;
   const int64_t pack_grid = (int64_t)(a->vt_cols / kKeyTile) * Hkv;
-  if (units > 0x7fffffff || pack_grid > 0x7fffffff) return fail(DAN_ERR_INVALID_ARGUMENT, "grid is too large");
+  if (units > 0x7fffffff || pack_grid + save_grid > 0x7fffffff) return fail(DAN_ERR_INVALID_ARGUMENT, "grid is too large");
   if (a->phases != DAN_TREE_ATTN_PHASE_PACK && (!a->units || !a->sched_off || a->num_slots <= 0 || a->num_slots > units))
     return fail(DAN_ERR_INVALID_ARGUMENT, "schedule: need units, sched_off and 1 <= num_slots <= %lld units",
                 (long long)units);
@@ -1818,6 +1879,9 @@ int dan_tree_attn_fwd(const DanTreeAttnArgs *a, void *stream) {
   pp.pasts_out = const_cast<DanPastDesc *>(a->pasts);
   pp.num_inline = a->pasts_host ? a->num_pasts : 0;
   for (int i = 0; i < pp.num_inline; ++i) pp.inl[i] = a->pasts_host[i];
+  pp.k = a->k; pp.k_st = a->k_stride_tok; pp.k_sh = a->k_stride_head;
+  pp.pack_blocks = (int)pack_grid; pp.num_saves = a->num_saves; pp.save_layout = a->save_layout;
+  for (int i = 0; i < a->num_saves; ++i) pp.saves[i] = a->saves[i];
 
   KParams kp;
   kp.q = a->q; kp.k = a->k; kp.o = a->out; kp.vt = pp.vt; kp.vexp = pp.vexp;
@@ -1834,9 +1898,9 @@ int dan_tree_attn_fwd(const DanTreeAttnArgs *a, void *stream) {
   hipStream_t s = static_cast<hipStream_t>(stream);
   // One instantiation per (input types, head_dim).
   auto by_d = [&](auto f64, auto f128, auto f256) { return D == 64 ? f64() : D == 128 ? f128() : f256(); };
-#define DAN_PACK(TV) by_d([&] { return launch_pack<TV, 64>(pp, (int)pack_grid, s); }, \
-                          [&] { return launch_pack<TV, 128>(pp, (int)pack_grid, s); }, \
-                          [&] { return launch_pack<TV, 256>(pp, (int)pack_grid, s); })
+#define DAN_PACK(TV) by_d([&] { return launch_pack<TV, 64>(pp, (int)(pack_grid + save_grid), s); }, \
+                          [&] { return launch_pack<TV, 128>(pp, (int)(pack_grid + save_grid), s); }, \
+                          [&] { return launch_pack<TV, 256>(pp, (int)(pack_grid + save_grid), s); })
 #define DAN_ATTN(TQK, TO) by_d([&] { return launch_attn<TQK, TO, 64>(kp, grid, halves, s); }, \
                                [&] { return launch_attn<TQK, TO, 128>(kp, grid, halves, s); }, \
                                [&] { return launch_attn<TQK, TO, 256>(kp, grid, halves, s); })

@@ -42,7 +42,7 @@
 extern "C" {
 #endif
 
-#define DAN_TREE_ATTN_ABI_VERSION 9
+#define DAN_TREE_ATTN_ABI_VERSION 10
 
 /* Keys per key tile; the work list's key-tile indices count in these. */
 #define DAN_TREE_ATTN_KEY_TILE 64
@@ -131,6 +131,13 @@ typedef struct {
 } DanUnit;
 
 typedef struct {
+  int32_t start; /* packed token */
+  int32_t len;   /* tokens, > 0 */
+  void *k_dst;
+  void *v_dst;
+} DanTreeAttnSave;
+
+typedef struct {
   int32_t abi_version; /* DAN_TREE_ATTN_ABI_VERSION */
   int32_t in_dtype;    /* DanDtype of q, k and the pasts' k: bf16, f16 or e4m3 */
   int32_t out_dtype;   /* DanDtype of out: bf16, f16 or f32 (bf16 for e4m3) */
@@ -210,9 +217,18 @@ typedef struct {
    * queries, whose key tiles the two halves of a work group's waves split --
    * the faster form for a batch of at most half as many units as CUs. */
   int32_t key_halves;
+  /* (ABI 10) Prefix saves of bf16 and f16 inputs: num_saves host entries, at
+   * most DAN_TREE_ATTN_INLINE_SAVES, read during the call only; the V^T copy's
+   * launch writes rows [start, start + len) of k and of v to each entry's
+   * k_dst and v_dst, contiguous and 16-byte aligned: [Hkv][len][D], or
+   * [len][Hkv][D] for k with bit 0 of save_layout and for v with bit 1. */
+  int32_t num_saves;
+  int32_t save_layout;
+  const DanTreeAttnSave *saves;
 } DanTreeAttnArgs;
 
 #define DAN_TREE_ATTN_INLINE_PASTS 8
+#define DAN_TREE_ATTN_INLINE_SAVES 8
 
 #define DAN_TREE_ATTN_PHASES_ALL 0
 #define DAN_TREE_ATTN_PHASE_PACK 1
