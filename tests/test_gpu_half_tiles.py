@@ -1,8 +1,8 @@
 """Half tiles (each key tile split between the two halves of a work group's
 waves) against the oracle and against whole tiles, at the sizes where the
 split can go wrong: segments shorter than a wave, trunks that end inside the
-first 32 keys (a half that sees no key of its first tile runs again with the
-running-max check), tiles that hold past and new keys, ragged last tiles, GQA
+first 32 keys (a half that sees no key of its first tile starts from its
+partner's running max), tiles that hold past and new keys, ragged last tiles, GQA
 ratios with 4, 2 and 1 heads per work group and with a second head chunk.
 
 Bars: 2e-2 against the oracle as in tests/test_gpu_parity.py; against whole
@@ -78,6 +78,34 @@ def test_half_tiles_overflowing_units(gpu, monkeypatch):
     for out in (whole, half):
         assert torch.isfinite(out).all()
         assert (out.float().cpu() - ref).abs().max().item() <= 2e-2
+
+
+@pytest.mark.parametrize("trunk,past", [(20, 0), (32, 0), (1, 31), (0, 8)])
+@pytest.mark.parametrize("heads,d,dtype", [((32, 8), 128, torch.bfloat16), ((4, 4), 64, torch.bfloat16), ((8, 2), 128, "e4m3")])
+def test_short_trunks_start_from_the_whole_first_tile(gpu, monkeypatch, trunk, past, heads, d, dtype):
+    """Past and trunk within the first 32 keys: a branch whose keys begin in a
+    later tile sees none of keys 32-63 of the first one. Both halves start from
+    the tile's maximum (past and trunk score 30 powers of 2 above the branches, and
+    their values are 0), so a branch key's p rounds to 0 in both, as in whole
+    tiles. A half that ran again from its own keys' maximum would leave 2^-30."""
+    print(f"[gpu-case] half tiles, past {past} trunk {trunk}, heads {heads} x {d} {dtype}", flush=True)
+    rng = np.random.default_rng(trunk)
+    w = build("short", [(trunk, [70, 60, 90])], heads[0], heads[1], d, torch.bfloat16, gpu, rng, per_segment_past=[past])
+    for t in (w.q, w.k, w.v):
+        t.zero_()
+    top = 30 * 0.6931471805599453 * d ** 0.5 / 8
+    w.q[..., 0] = 8
+    w.k[:, :trunk, 0] = top
+    w.v[:, trunk:] = 1
+    if past:
+        pk, pv = w.segments[0].past[0]
+        pk.zero_()
+        pk[..., 0] = top
+        pv.zero_()
+    w = to_e4m3(w) if dtype == "e4m3" else w
+    whole, half = both(w, monkeypatch)
+    branches = slice(trunk + 70, None)  # those whose keys begin past the first tile
+    assert not whole[:, branches].any() and not half[:, branches].any()
 
 
 def test_rule_depends_on_the_length_alone(gpu):
