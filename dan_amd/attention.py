@@ -275,10 +275,12 @@ def get_plan(segments, num_tokens, tile_q, device, groups=None, num_cus=None, pl
     return plan
 
 
-# Half tiles (``_tile_q``) where the whole ones, this many times over, fit the
-# CUs. Attention launch on 256 CUs, whole / half time: 1.0 to 1.5 at up to 128
-# units (834 tokens on 32/8 heads 1.35), 0.92 to 1.36 at 192, 0.84 to 1.22 at 256
-# (more than one request: 0.84 to 1.0), 0.82 to 0.97 from 352 on.
+# Half tiles (``_tile_q``) where the packed tokens' whole tiles, this many times
+# over, fit the CUs. Attention launch on 256 CUs, whole / half time, 32/8 and
+# 32/32 heads x 128 and 8/2 x 64, no prefix to 1024 tokens of it: 1.0 to 1.6 while
+# the halves' units, counted over the segments, fit the CUs. Where they do not,
+# about 1000 tokens: 25 segments of 40 (200 whole, 400 half units) 0.70 to 0.81,
+# 12 of 65 0.76 to 0.85, but 50 of 20 (400 of both) 0.99 to 1.40.
 HALF_TILE_UNITS = 2
 
 
@@ -414,16 +416,28 @@ def _layout(h, hkv, d):
     return _native.tile_q(h, hkv, d, lib=lib), _native.head_groups(h, hkv, lib)
 
 
-def _tile_q(h, hkv, d, n, device):
+def _tile_q(h, hkv, d, n, device, items=None):
     """Queries per work item of a batch of ``n`` packed tokens: the kernel's
     tile, or half of it where whole tiles would leave at least half of the
-    CUs without one (the kernel then splits each key tile between its waves).
-    It depends on the packed length alone, so a BudgetPlan and a batch's own
-    plan agree. 0: unsupported head layout."""
+    CUs without one (the kernel then splits each key tile between its waves)
+    and the halves' units, of which every segment has its own, fit the CUs or
+    are no more than the whole tiles'. ``items``: tile -> the batch's work
+    items of that many queries (default: those of one segment). 0:
+    unsupported head layout."""
     tile_q, groups = _layout(h, hkv, d)
-    if tile_q > 0 and d <= 128 and -(-n // tile_q) * groups * HALF_TILE_UNITS <= _num_cus(device):
-        return tile_q // 2
+    cus = _num_cus(device)
+    if tile_q > 0 and d <= 128 and -(-n // tile_q) * groups * HALF_TILE_UNITS <= cus:
+        if items is None or (half := items(tile_q // 2)) * groups <= cus or half <= items(tile_q):
+            return tile_q // 2
     return tile_q
+
+
+def _work_items(segments, n):
+    """Tile -> work items of ``segments``, over ``n`` packed tokens."""
+    plan = getattr(segments, "tile_plan", None)
+    if plan is not None and plan.num_tokens == n:
+        return plan.items
+    return lambda tile: sum(-(-(s.end - s.start) // tile) for s in segments)
 
 
 def workspace_bytes(q, k, segments):
@@ -431,7 +445,7 @@ def workspace_bytes(q, k, segments):
     batch (the plan is built or found as for the call itself)."""
     h, n, d = q.shape
     hkv = k.shape[0]
-    tile_q, groups = _tile_q(h, hkv, d, n, q.device), _layout(h, hkv, d)[1]
+    tile_q, groups = _tile_q(h, hkv, d, n, q.device, _work_items(segments, n)), _layout(h, hkv, d)[1]
     plan = get_plan(segments, n, tile_q, q.device, groups=groups, num_cus=_num_cus(q.device))
     return _native.workspace_size(hkv, d, plan.vt_cols)
 
@@ -455,7 +469,7 @@ def _call_args(q, k, v, segments, layer, scale, fp8_scales, phases, noalloc, upl
         raise ValueError(f"scale {scale}: the kernel needs a finite positive softmax scale")
     h, n, d = q.shape
     hkv = k.shape[0]
-    tile_q = _tile_q(h, hkv, d, n, q.device)
+    tile_q = _tile_q(h, hkv, d, n, q.device, _work_items(segments, n))
     if tile_q <= 0:
         raise ValueError(f"unsupported head layout H={h}, Hkv={hkv}")
     groups = _layout(h, hkv, d)[1]
@@ -564,13 +578,15 @@ class BudgetPlan:
                         max_branches=256, max_past_tokens=16 * 1024)
         bp.load(batch)                    # per batch, outside the graph: one upload, one
                                           # planner launch, each layer's prefix table
-        out = bp.attend(q, k, v, layer)   # capturable; equals attend(q, k, v, batch, layer)
+        out = bp.attend(q, k, v, layer)   # capturable; attend(q, k, v, batch, layer)
 
     q, k, v keep their addresses between replays (copy each batch's values
     into the captured tensors); prefix-cache entries may change freely (they
     are reached through the prefix tables ``load`` rewrites). Rows beyond the
-    batch's segments are left as they are. ``load`` waits for its previous
-    upload to finish before reusing the host staging buffer."""
+    batch's segments are left as they are. The plan takes whole or half tiles
+    for the most work items its capacities allow; a batch's own plan may take
+    the other form, whose results differ by the rounding of P. ``load`` waits
+    for its previous upload to finish before reusing the host staging buffer."""
 
     def __init__(self, num_tokens, num_heads, num_kv_heads, head_dim, dtype, device, max_segments, max_branches,
                  max_past_tokens=0):
@@ -579,7 +595,9 @@ class BudgetPlan:
             raise RuntimeError("BudgetPlan runs on a gfx950 GPU only")
         lib = _native.load()
         self.n, self.h, self.hkv, self.d, self.dtype, self.device = num_tokens, num_heads, num_kv_heads, head_dim, dtype, device
-        self.tile_q = _tile_q(num_heads, num_kv_heads, head_dim, num_tokens, device)
+        # the most work items that num_tokens in max_segments can make
+        self.tile_q = _tile_q(num_heads, num_kv_heads, head_dim, num_tokens, device,
+                              lambda tile: (num_tokens - max_segments) // tile + max_segments if num_tokens > max_segments else num_tokens)
         self.groups = _layout(num_heads, num_kv_heads, head_dim)[1]
         if self.tile_q <= 0 or head_dim not in (64, 128, 256) or dtype not in _DTYPES:
             raise ValueError(f"unsupported layout {num_heads}/{num_kv_heads} x {head_dim}, {dtype}")

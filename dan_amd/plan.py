@@ -250,6 +250,7 @@ class TilePlan:
     past_hosts: dict = field(default_factory=dict)  # layer -> the table's host bytes (None: too long to ride in a launch)
     past_uploaded: set = field(default_factory=set)  # the layers whose device table was filled by an upload
     schedules: dict = field(default_factory=dict)  # (groups, CUs) -> (units_d, sched_off_d, slots)
+    item_counts: dict = field(default_factory=dict)  # tile -> work items of so many queries
 
     @classmethod
     def build(cls, segments, num_tokens, tile_q, device):
@@ -304,6 +305,12 @@ class TilePlan:
             _native.plan(a, torch.cuda.current_stream(dev).cuda_stream, lib)
         plan.schedules[(groups, num_cus)] = (units, off, slots)
         return plan
+
+    def items(self, tile):
+        """Work items that the segments make with ``tile`` queries each."""
+        if tile not in self.item_counts:
+            self.item_counts[tile] = int((-(-self.segs[:, 1] // tile)).sum())
+        return self.item_counts[tile]
 
     @property
     def vt_cols(self):

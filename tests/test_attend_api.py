@@ -60,3 +60,20 @@ def test_custom_op_fake_output(qdt, vdt, want):
         o = torch.ops.dan_amd.tree_attn(q, k, v, tables, scales, [1, 0, 1, 64, 128, 1, 0, 0], 0.1, None)
         assert o.shape == (h, n, d) and o.dtype == want and o.device.type == "cuda"
         assert o.stride() == (d, h * d, 1)
+
+
+@pytest.mark.parametrize("lens,want", [([1024], 32), ([1025], 64), ([40] * 25, 64), ([70] * 10, 32), ([20] * 50, 32), ([33] * 15 + [505], 64), ([32] * 64, 64)])
+def test_half_tiles_count_every_segments_units(monkeypatch, lens, want):
+    """32/8 heads x 128 on 256 CUs: half tiles while their units, counted over
+    the segments, fit the CUs or are no more than the whole tiles' (segments of
+    at most half a tile), from the segments and from a cached plan alike."""
+    from dan_amd.plan import TilePlan
+
+    monkeypatch.setattr(A, "_num_cus", lambda device: 256)
+    n, segs = sum(lens), A.Batch()
+    for x in lens:
+        segs.append(A.segment(segs[-1].end if segs else 0, [0] * x))
+    tile = lambda: A._tile_q(32, 8, 128, n, "cuda", A._work_items(segs, n))  # noqa: E731
+    assert tile() == want
+    segs.tile_plan = TilePlan.build(segs, n, 64, "cpu")
+    assert tile() == want

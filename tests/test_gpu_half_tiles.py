@@ -108,7 +108,7 @@ def test_short_trunks_start_from_the_whole_first_tile(gpu, monkeypatch, trunk, p
     assert not whole[:, branches].any() and not half[:, branches].any()
 
 
-def test_rule_depends_on_the_length_alone(gpu):
+def test_rule_of_one_segment(gpu):
     lib = _native.load()
     cus = A._num_cus(torch.device(gpu))
     tile = lambda h, hkv, d, n: A._tile_q(h, hkv, d, n, torch.device(gpu))  # noqa: E731
@@ -117,6 +117,32 @@ def test_rule_depends_on_the_length_alone(gpu):
         assert tile(8, 2, 64, 4096) == 32 and tile(8, 2, 64, 4097) == 64
     assert tile(16, 2, 256, 16) == _native.tile_q(16, 2, 256, lib=lib)
     assert tile(12, 8, 128, 16) == 0
+
+
+@pytest.mark.parametrize("lens,want", [([40] * 25, 64), ([70] * 10, 32), ([20] * 50, 32)])
+def test_segments_make_their_own_units(gpu, lens, want):
+    """About 1000 tokens in many segments: half tiles only while all their units are resident at once."""
+    w = build("many", [(x, []) for x in lens], 32, 8, 128, torch.bfloat16, gpu, np.random.default_rng(1))
+    for _ in range(2):  # the second call finds the plan
+        out = A.attend(w.q, w.k, w.v, w.segments, w.layer)
+        if A._num_cus(torch.device(gpu)) == 256:
+            assert w.segments.tile_plan.tile_q == want
+    ref = oracle.attend_dense(w.q, w.k, w.v, w.segments, w.layer)
+    assert (out.float().cpu() - ref).abs().max().item() <= 2e-2
+
+
+@pytest.mark.parametrize("segments,want", [(1, 32), (4, 32), (16, 64)])
+def test_budget_plan_counts_its_capacity(gpu, segments, want):
+    """A BudgetPlan takes the form for the most units its capacities allow; its
+    results are attend's, up to the rounding of P where that takes the other form."""
+    w = build("budget", [(700, [60, 74])], 32, 8, 128, torch.bfloat16, gpu, np.random.default_rng(2))
+    bp = A.BudgetPlan(w.num_tokens, 32, 8, 128, torch.bfloat16, gpu, max_segments=segments, max_branches=8)
+    if A._num_cus(torch.device(gpu)) == 256:
+        assert bp.tile_q == want
+    bp.load(w.segments)
+    got, out = bp.attend(w.q, w.k, w.v, w.layer).float(), A.attend(w.q, w.k, w.v, w.segments, w.layer).float()
+    bar = 2.0 ** -9 * w.v.float().abs().max().item() + 2.0 ** -7 * out.abs().max().item() if want == 64 else 0.0
+    assert (got - out).abs().max().item() <= bar
 
 
 def test_half_tiles_need_their_flag():
