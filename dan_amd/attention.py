@@ -404,9 +404,12 @@ def _attend_fused(q, k, v, segments, layer, scale, fp8_scales=None, phases=_nati
     if torch.compiler.is_compiling():
         return torch.ops.dan_amd.tree_attn(*_op_args(q, k, v, segments, layer, scale, fp8_scales, phases, noalloc), workspace)
     # an attention-only launch has no copy before it that would fill the prefix table
-    args, pasts_host = _call_args(q, k, v, segments, layer, scale, fp8_scales, phases, noalloc,
-                                  upload=phases == _native.PHASE_ATTEND)
-    return _launch_tree_attn(*args, workspace, pasts_host, saves)
+    args, pasts_host, plan = _call_args(q, k, v, segments, layer, scale, fp8_scales, phases, noalloc,
+                                        upload=None if phases == _native.PHASE_ATTEND else False)
+    out = _launch_tree_attn(*args, workspace, pasts_host, saves)
+    if workspace is not None and pasts_host is not None and not torch.cuda.is_current_stream_capturing():
+        plan.past_filled[layer] = (_native.stream(q.device), args[3][4])  # for attention-only launches behind this one
+    return out
 
 
 @functools.lru_cache(maxsize=None)
@@ -457,8 +460,9 @@ def _op_args(q, k, v, segments, layer, scale, fp8_scales=None, phases=_native.PH
 
 
 def _call_args(q, k, v, segments, layer, scale, fp8_scales, phases, noalloc, upload=True):
-    """``_op_args``, and the host bytes of the prefix-cache table that the
-    launch fills it from (None: the table is uploaded, or empty)."""
+    """``_op_args``, the host bytes of the prefix-cache table that the launch
+    fills it from (None: the table is uploaded, filled or empty) and the
+    plan. ``upload`` None: unless a launch on this stream has filled the table."""
     if not q.is_cuda:
         raise RuntimeError("dan_amd.attend runs on a gfx950 GPU only; got tensors on "
                            f"{q.device} (the masked CPU path is the test oracle, not a backend)")
@@ -474,6 +478,11 @@ def _call_args(q, k, v, segments, layer, scale, fp8_scales, phases, noalloc, upl
         raise ValueError(f"unsupported head layout H={h}, Hkv={hkv}")
     groups = _layout(h, hkv, d)[1]
     plan = get_plan(segments, n, tile_q, q.device, groups=groups, num_cus=_num_cus(q.device))
+    filled = False
+    if upload is None:
+        stream, table = plan.past_filled.get(layer, (None, None))
+        filled = stream == _native.stream(q.device) and plan.past_tables[layer][0] is table
+        upload = not filled
     table, _refs = _past_table(plan, layer, hkv, d, q.dtype, q.device, upload)
     if q.dtype == E4M3:
         q_scale, k_scale, v_scale = (_check_scale(t, nm, q.device) for t, nm in zip(fp8_scales, ("q_scale", "k_scale", "v_scale")))
@@ -488,8 +497,8 @@ def _call_args(q, k, v, segments, layer, scale, fp8_scales, phases, noalloc, upl
         tables += [units, sched_off]
     meta = [len(plan.segs), len(plan.past_dicts), plan.num_work, tile_q, plan.vt_cols, slots, phases, int(noalloc)]
     softmax_scale = (1.0 / math.sqrt(d)) if scale is None else float(scale)
-    pasts_host = None if upload or not plan.past_dicts or layer in plan.past_uploaded else plan.past_hosts[layer]
-    return (q, k, v, tables, scales, meta, softmax_scale), pasts_host
+    pasts_host = None if upload or filled or not plan.past_dicts or layer in plan.past_uploaded else plan.past_hosts[layer]
+    return (q, k, v, tables, scales, meta, softmax_scale), pasts_host, plan
 
 
 def _out_dtype(q, v):

@@ -249,6 +249,7 @@ class TilePlan:
     past_tables: dict = field(default_factory=dict)  # layer -> (device bytes, keep-alive refs)
     past_hosts: dict = field(default_factory=dict)  # layer -> the table's host bytes (None: too long to ride in a launch)
     past_uploaded: set = field(default_factory=set)  # the layers whose device table was filled by an upload
+    past_filled: dict = field(default_factory=dict)  # layer -> (stream, table) of a launch with a caller's workspace that filled it
     schedules: dict = field(default_factory=dict)  # (groups, CUs) -> (units_d, sched_off_d, slots)
     item_counts: dict = field(default_factory=dict)  # tile -> work items of so many queries
 

@@ -62,6 +62,35 @@ def test_attention_only_launch_finds_its_table(gpu):
     assert torch.equal(out, want)
 
 
+@pytest.mark.parametrize("first", [_native.PHASE_PACK, _native.PHASES_ALL])
+def test_attention_only_launch_uses_the_filled_table(gpu, monkeypatch, first):
+    """Behind a launch that filled the table (on its stream) an attention-only
+    one uploads nothing; on another stream, or behind a captured launch that
+    has not run, it does."""
+    say(f"attention-only launches behind phases {first}")
+    q, k, v, segs = case(gpu, 3, 6)
+    want = attend(q, k, v, Batch(segs), 0)
+    ws = torch.empty(workspace_bytes(q, k, segs), dtype=torch.uint8, device=gpu)
+    pinned, pin = [], torch.Tensor.pin_memory
+    monkeypatch.setattr(torch.Tensor, "pin_memory", lambda t, *a: (pinned.append(t.numel()), pin(t, *a))[1])
+    only = lambda: _attend_fused(q, k, v, segs, 0, None, phases=_native.PHASE_ATTEND, workspace=ws)  # noqa: E731
+    _attend_fused(q, k, v, segs, 0, None, phases=first, workspace=ws)
+    outs = [only(), only()]
+    torch.cuda.synchronize()
+    assert not pinned and all(torch.equal(o, want) for o in outs)
+    side = torch.cuda.Stream(gpu)
+    with torch.cuda.stream(side):
+        out = only()
+    torch.cuda.synchronize()
+    assert len(pinned) == 1 and torch.equal(out, want)
+    fresh = Batch(segs)
+    workspace_bytes(q, k, fresh)  # plans outside the capture
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        _attend_fused(q, k, v, fresh, 0, None, phases=first, workspace=ws)
+    assert not fresh.tile_plan.past_filled
+
+
 @pytest.mark.parametrize("saves", [1, 16, 17])
 def test_inline_saves(gpu, saves):
     say(f"{saves} saves")
