@@ -29,6 +29,7 @@ from dataclasses import dataclass, field
 from typing import List, Optional
 
 import torch
+from torch.autograd import forward_ad
 
 from . import _native
 from .plan import TilePlan
@@ -164,16 +165,23 @@ def attend(q, k, v, segments, layer, scale=None, *, q_scale=None, k_scale=None, 
     return _attend_fused(q, k, v, segments, layer, scale, (q_scale, k_scale, v_scale) if fp8 else None)
 
 
+def has_tangent(*tensors):
+    """Whether one of the tensors carries a forward-mode tangent, which torch's
+    operators pass on and a kernel that writes in their place would drop
+    (``requires_grad`` does not show it, and no_grad does not stop it)."""
+    return any(forward_ad.unpack_dual(t).tangent is not None for t in tensors)
+
+
 def _launch_saves(k, v, segments):
     """The saving segments whose rows ``attend``'s launch copies; none of them
     where it clones instead: more than INLINE_SAVES, other types than bf16 and
     fp16, a single row or kv head, rows past the packed ones or the segment's
-    own, tracing, gradients, or a k or v whose heads overlap its tokens."""
+    own, tracing, gradients, tangents, or a k or v whose heads overlap its tokens."""
     todo = [s for s in segments if s.save]
     if (not 0 < len(todo) <= _native.INLINE_SAVES or type(k) is not torch.Tensor or type(v) is not torch.Tensor
             or k.dtype not in (torch.bfloat16, torch.float16) or v.dtype != k.dtype or k.dim() != 3 or v.shape != k.shape
             or not k.is_cuda or k.device != v.device or torch.compiler.is_compiling()
-            or torch.is_grad_enabled() and (k.requires_grad or v.requires_grad)):
+            or torch.is_grad_enabled() and (k.requires_grad or v.requires_grad) or has_tangent(k, v)):
         return []
     hkv, n, d = k.shape
     if hkv < 2 or any(not (0 <= s.start and 1 < s.save <= min(n, s.end) - s.start) for s in todo):

@@ -23,7 +23,7 @@ import torch
 from torch import nn
 
 from . import _native
-from .attention import _DTYPES, Batch, _num_cus
+from .attention import _DTYPES, Batch, _num_cus, has_tangent
 
 
 def _row_ok(t):
@@ -137,10 +137,10 @@ def gated_rms_norm(x, gate, weight, eps):
 def _gated_norm(out, z, weight, eps):
     """``gated_rms_norm`` of every (token, head) row of out [N, Hv, Dv] with
     the gate z [N, Hv * Dv], as [N, Hv * Dv]: one ``dan_gdn_gated_norm``
-    launch where its layout and types allow and no gradient is wanted, else
+    launch where its layout and types allow and no derivative is wanted, else
     the eager ops (both round at the same places)."""
     n, hv, dv = out.shape
-    grad = torch.is_grad_enabled() and any(t.requires_grad for t in (out, z, weight))
+    grad = torch.is_grad_enabled() and any(t.requires_grad for t in (out, z, weight)) or has_tangent(out, z, weight)
     if (grad or torch.compiler.is_compiling() or dv not in (32, 64, 128, 256) or out.dtype not in (torch.bfloat16, torch.float16)
             or not (z.dtype == weight.dtype == out.dtype) or not out.is_contiguous() or z.stride(1) != 1
             or z.stride(0) % 8 or z.stride(0) < hv * dv or not weight.is_contiguous()
@@ -156,12 +156,13 @@ def _gated_norm(out, z, weight, eps):
 def _narrow_pair(x, first, second):
     """``first(x), second(x)`` of two linears of the same narrow width on x
     [N, K]: one ``dan_gdn_project`` launch where both are plain nn.Linear
-    modules without bias, hooks or wanted gradients whose layout and types it
+    modules without bias, hooks or wanted derivatives whose layout and types it
     takes, else the modules' own calls."""
     w0, w1 = first.weight, second.weight
     if (not (_plain(first) and _plain(second)) or type(x) is not torch.Tensor or not x.is_cuda or x.dim() != 2
             or torch.compiler.is_compiling() or torch.is_autocast_enabled("cuda")
             or torch.is_grad_enabled() and (x.requires_grad or w0.requires_grad or w1.requires_grad)
+            or has_tangent(x)  # (a parameter carries none: make_dual gives a plain tensor, which _plain refuses)
             or x.dtype not in (torch.bfloat16, torch.float16) or not w0.dtype == w1.dtype == x.dtype
             or not w0.device == w1.device == x.device or w0.shape != w1.shape or w0.shape[1] != x.shape[1]
             or w0.shape[0] % 4 or not w0.shape[0] or x.shape[1] % 32 or not 0 < x.shape[1] <= NARROW_HIDDEN
