@@ -176,7 +176,9 @@ def _launch_saves(k, v, segments):
     """The saving segments whose rows ``attend``'s launch copies; none of them
     where it clones instead: more than INLINE_SAVES, other types than bf16 and
     fp16, a single row or kv head, rows past the packed ones or the segment's
-    own, tracing, gradients, tangents, or a k or v whose heads overlap its tokens."""
+    own, tracing, gradients, tangents, or a k or v (expanded, or of another order
+    of dimensions) whose clone would lie neither [Hkv][rows][D] nor [rows][Hkv][D]
+    by the order of its strides."""
     todo = [s for s in segments if s.save]
     if (not 0 < len(todo) <= _native.INLINE_SAVES or type(k) is not torch.Tensor or type(v) is not torch.Tensor
             or k.dtype not in (torch.bfloat16, torch.float16) or v.dtype != k.dtype or k.dim() != 3 or v.shape != k.shape
@@ -186,7 +188,7 @@ def _launch_saves(k, v, segments):
     hkv, n, d = k.shape
     if hkv < 2 or any(not (0 <= s.start and 1 < s.save <= min(n, s.end) - s.start) for s in todo):
         return []  # (a clone keeps the stride of a dimension of one, too)
-    if k.stride(0) == k.stride(1) or v.stride(0) == v.stride(1):
+    if any(not 0 < t.stride(2) < min(t.stride(0), t.stride(1)) or t.stride(0) == t.stride(1) for t in (k, v)):
         return []
     return todo
 

@@ -60,6 +60,36 @@ def test_saves_equal_clones(gpu, layout, lengths, saves, d, dtype):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("layout", ["heads expanded", "one expanded", "tokens expanded", "columns outermost", "columns strided", "heads innermost"])
+def test_saves_of_other_layouts_equal_clones(gpu, layout):
+    """Values and strides of the clones where a stride is 0 or head_dim is not the innermost dimension."""
+    print(f"[gpu-case] saves, {layout}", flush=True)
+    segs, n = _batch([40, 30], [17, 9])
+    q, k, v = _qkv("heads", 4, 2, n, 64, torch.bfloat16, gpu)
+    if layout == "heads expanded":
+        k, v = k[:1].expand(2, n, 64), v[:1].expand(2, n, 64)
+    elif layout == "one expanded":
+        v = v[:1].expand(2, n, 64)
+    elif layout == "tokens expanded":
+        k = k[:, :1].expand(2, n, 64)
+    elif layout == "columns outermost":
+        k, v = (t.permute(2, 0, 1).contiguous().permute(1, 2, 0) for t in (k, v))
+    elif layout == "columns strided":
+        k, v = (torch.zeros(2, n, 128, dtype=t.dtype, device=gpu)[:, :, ::2].copy_(t) for t in (k, v))
+    else:
+        k, v = (t.permute(1, 2, 0).contiguous().permute(2, 0, 1) for t in (k, v))
+    with torch.no_grad():
+        out = attend(q, k, v, segs, 3)
+        plain = attend(q, k.contiguous(), v.contiguous(), segs, 3, save=False)
+    torch.cuda.synchronize()
+    assert torch.equal(out, plain)
+    for s in segs:
+        for got, t in zip(s.saved[3], (k, v)):
+            want = t[:, s.start:s.start + s.save].clone()
+            assert torch.equal(got, want) and got.stride() == want.stride()
+
+
+@pytest.mark.gpu
 def test_rows_past_the_segment_are_cloned(gpu):
     segs, n = _batch([20, 30], [0, 0])
     segs[0].save = 25  # into the next segment, as a clone allows
