@@ -174,7 +174,8 @@ def has_tangent(*tensors):
 
 def _launch_saves(k, v, segments):
     """The saving segments whose rows ``attend``'s launch copies; none of them
-    where it clones instead: more than INLINE_SAVES, other types than bf16 and
+    where it clones instead: an entry that this very batch reads as a prefix (it
+    has to be there before the plan and the launch), more than INLINE_SAVES, other types than bf16 and
     fp16, a single row or kv head, rows past the packed ones or the segment's
     own, tracing, gradients, tangents, or a k or v (expanded, or of another order
     of dimensions) whose clone would lie neither [Hkv][rows][D] nor [rows][Hkv][D]
@@ -184,6 +185,9 @@ def _launch_saves(k, v, segments):
             or k.dtype not in (torch.bfloat16, torch.float16) or v.dtype != k.dtype or k.dim() != 3 or v.shape != k.shape
             or not k.is_cuda or k.device != v.device or torch.compiler.is_compiling()
             or torch.is_grad_enabled() and (k.requires_grad or v.requires_grad) or has_tangent(k, v)):
+        return []
+    written = {id(s.saved) for s in todo}
+    if any(id(s.past) in written for s in segments):
         return []
     hkv, n, d = k.shape
     if hkv < 2 or any(not (0 <= s.start and 1 < s.save <= min(n, s.end) - s.start) for s in todo):

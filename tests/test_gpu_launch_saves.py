@@ -7,7 +7,7 @@ import pytest
 import torch
 
 from dan_amd import _native
-from dan_amd.attention import Batch, _launch_saves, attend, segment
+from dan_amd.attention import Batch, Segment, _launch_saves, attend, segment
 
 
 def _batch(lengths, saves):
@@ -87,6 +87,25 @@ def test_saves_of_other_layouts_equal_clones(gpu, layout):
         for got, t in zip(s.saved[3], (k, v)):
             want = t[:, s.start:s.start + s.save].clone()
             assert torch.equal(got, want) and got.stride() == want.stride()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_a_batch_reads_what_it_saves(gpu, dtype):
+    """A request whose prefix is the rows that another of its batch saves: each
+    layer's entry is there before the plan and the launch read it."""
+    print(f"[gpu-case] a save read in its own batch, {dtype}", flush=True)
+    first = segment(0, [0] * 50 + [1] * 7, None, 31, 0, "cuda")
+    second = Segment(57, 80, 13, [(70, 80)], first.saved, past_len=31, branch_ids=[0] * 13 + [1] * 10, device="cuda")
+    segs = Batch([first, second])
+    with torch.no_grad():
+        for layer in (0, 1):
+            q, k, v = (t + layer for t in _qkv("fused", 4, 2, 80, 64, dtype, gpu))
+            out = attend(q, k, v, segs, layer)
+            entry = {layer: (k[:, :31].clone(), v[:, :31].clone())}
+            apart = Batch([segment(0, first.branch_ids, None, 0, 0, "cuda"), segment(57, second.branch_ids, entry, 0, 31, "cuda")])
+            assert torch.equal(out, attend(q, k, v, apart, layer))
+            assert all(torch.equal(a, b) for a, b in zip(first.saved[layer], entry[layer]))
 
 
 @pytest.mark.gpu
