@@ -52,3 +52,21 @@ def test_gated_norm_special_values(gpu):
     assert torch.equal(y.isinf(), ref.isinf())
     fine = ref.isfinite()
     assert ((y - ref)[fine].abs() <= 3 * 2.0 ** -7 * ref[fine].abs()).all()
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_silu_of_every_gate(gpu, dtype):
+    """Rows that normalize to 1 leave rnd(silu(gate)): every finite gate of the
+    type down to -88.5 (where exp still fits fp32), within half a spacing of the value
+    in 64 bits and 2^-20 of that value, which is what fp32 operations leave."""
+    print(f"[gpu-case] silu of every gate, {dtype}", flush=True)
+    z = torch.arange(-2 ** 15, 2 ** 15, dtype=torch.int32).to(torch.int16).view(dtype)
+    z = z[z.isfinite() & (z >= -88.5)]
+    z = torch.cat([z, z.new_zeros(-z.numel() % 64)]).view(-1, 64)
+    x = torch.full((z.shape[0], 1, 64), 1024.0, dtype=dtype) if dtype == torch.bfloat16 else torch.full((z.shape[0], 1, 64), 64.0, dtype=dtype)
+    with torch.no_grad():
+        y = _gated_norm(x.to(gpu), z.to(gpu), torch.ones(64, dtype=dtype, device=gpu), 1e-6).cpu().double()
+    ref = z.double() * torch.sigmoid(z.double())
+    digits, least = (8, 2.0 ** -133) if dtype == torch.bfloat16 else (11, 2.0 ** -24)  # significant bits; the smallest value
+    spacing = torch.ldexp(torch.ones_like(ref), torch.frexp(ref).exponent - digits).clamp(min=least)
+    assert ((y - ref).abs() <= 0.5 * spacing + 2.0 ** -20 * ref.abs()).all()
