@@ -49,11 +49,24 @@
 
 #include <type_traits>
 
+#include "cus.h"
 #include "dan_fp8.h"
 
 namespace dan {
 int fail(int status, const char *fmt, ...);  // tree_attn.hip: sets the thread's last-error message
 extern thread_local char g_err[512];
+
+int num_cus() {  // cached per device
+  static int cached[64] = {};
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 0;
+  if (!cached[dev]) {
+    int n = 0;
+    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) return 0;
+    cached[dev] = n;
+  }
+  return cached[dev];
+}
 }  // namespace dan
 
 namespace dan_gemm {
@@ -1031,18 +1044,6 @@ hipError_t launch_persistent(const Params &p, int grid, hipStream_t s) {
   return hipGetLastError();
 }
 
-int num_cus() {  // of the current device, cached per device
-  static int cached[64] = {};
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 0;
-  if (!cached[dev]) {
-    int n = 0;
-    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) return 0;
-    cached[dev] = n;
-  }
-  return cached[dev];
-}
-
 template <typename TOut, int TM, int TN, int KS, int NST, int GM>
 hipError_t launch_small(Params p, hipStream_t s) {
   p.tiles_m = (p.m + TM - 1) / TM;
@@ -1058,7 +1059,7 @@ hipError_t launch_small(Params p, hipStream_t s) {
 
 template <typename TOut>
 hipError_t launch(const Params &p, hipStream_t s) {
-  const int kt = (p.k + kBK - 1) / kBK, tiles = p.tiles_m * p.tiles_n, cus = num_cus();
+  const int kt = (p.k + kBK - 1) / kBK, tiles = p.tiles_m * p.tiles_n, cus = dan::num_cus();
   // The smallest of these tiles that gives every CU at most one; 256 x 256
   // tiles where even 256 x 128 ones are more than the CUs. A CU's time grows
   // with its tile, and a second round doubles it. Over 190 sizes (m 1 to 8192;

@@ -44,6 +44,7 @@
 
 #include <type_traits>
 
+#include "cus.h"
 #include "dan_gdn.h"
 
 namespace dan_gdnc {
@@ -84,16 +85,6 @@ typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
-
-// The bf16 scan takes 16 state columns per work group while all groups are
-// resident at once, two per CU, else 32: a chunk's step of 16 columns is the
-// shorter, so the longest run ends sooner, but the groups' total work is more.
-// The whole rule (16 value heads of 128 columns), microseconds at 16 / 32 columns:
-// 1 run of 1462 tokens (128 groups) 55.4 / 71.4, 2000 + 300 + 900 (384) 82.9 / 99.8,
-// 3 of 1500 87.8 / 87.0, 4 of 1000 (512) 63.6 / 63.1; past that it depends on how
-// unequal the runs are: 5 of 286-1843 (640) 92 / 108, but 5 of 1000 91 / 80, 6 of
-// 400-1900 116 / 111, 8 of 800 95 / 79, 45 branches of 16-96 77 / 62.
-constexpr int kScan16Groups = 512;
 
 struct Params {
   const int32_t *cu;
@@ -1116,7 +1107,7 @@ hipError_t dan_gdn_fwd_chunked(const DanGdnArgs *a, float *records, hipStream_t 
     const bool vec = !(((uintptr_t)a->v & 15) || a->v_stride_tok % 8 || a->v_stride_head % 8 || ((uintptr_t)a->out & 7) ||
                        a->o_stride_tok % 4 || a->o_stride_head % 4);
     using namespace dan_gdnc;
-    if ((int64_t)p.units * (a->v_dim / 16) <= kScan16Groups) {
+    if (dan::scan_columns(a->num_runs, a->num_v_heads, a->v_dim, dan::num_cus()) == 16) {
       if (vec) scan(chunk_scan_bf16_kernel<16, true>, 4, 16);
       else scan(chunk_scan_bf16_kernel<16, false>, 4, 16);
     } else {

@@ -14,6 +14,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "cus.h"
 #include "dan_gdn.h"
 
 namespace dan {
@@ -121,12 +122,9 @@ void launch(const Params &p, hipStream_t s) {
   hipLaunchKernelGGL((proj_kernel<T, RB>), grid, dim3(64 * kWaves), 0, s, p);
 }
 
-// 16 rows a work group while that is at most one group per CU, else 32. 2048
-// hidden values, 16 / 32 rows, microseconds: 834 x 16 7.2 / 9.0 and 2779 x 16 7.4 /
-// 9.1, but 8192 x 16 12.8 / 9.7 and 2779 x 32 12.7 / 9.6.
 template <typename T>
 void run(const Params &p, hipStream_t s) {
-  if (((int64_t)p.M + 15) / 16 * ((p.N + 15) / 16) <= 256) launch<T, 1>(p, s);
+  if (dan::project_rows(p.M, p.N, dan::num_cus()) == 16) launch<T, 1>(p, s);
   else launch<T, 2>(p, s);
 }
 
