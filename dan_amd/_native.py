@@ -362,31 +362,6 @@ def stage_f16_pair(first, second, stream, lib=None):
         raise RuntimeError(f"dan_tree_attn_stage_f16_pair failed (status {rc}): {last_error(lib)}")
 
 
-def forward(args, stream, lib=None):
-    """Launch; raises RuntimeError with the library's message on failure."""
-    lib = lib or load()
-    rc = lib.dan_tree_attn_fwd(ctypes.byref(args), _vp(stream))
-    if rc != OK:
-        raise RuntimeError(f"dan_tree_attn_fwd failed (status {rc}): {last_error(lib)}")
-
-
-def forward_noalloc(args, stream, lib=None):
-    """Launch through dan_tree_attn_fwd_noalloc (the V^T copy in the library's
-    own scratch, nothing allocated); raises RuntimeError on failure."""
-    lib = lib or load()
-    rc = lib.dan_tree_attn_fwd_noalloc(ctypes.byref(args), _vp(stream))
-    if rc != OK:
-        raise RuntimeError(f"dan_tree_attn_fwd_noalloc failed (status {rc}): {last_error(lib)}")
-
-
-def front(args, stream, lib=None):
-    """Launch the attention front end; raises RuntimeError with the library's message on failure."""
-    lib = lib or load()
-    rc = lib.dan_qkv_front(ctypes.byref(args), _vp(stream))
-    if rc != OK:
-        raise RuntimeError(f"dan_qkv_front failed ({rc}): {last_error(lib)}")
-
-
 def plan_slots(num_work, groups, num_cus, lib=None):
     """Slots of the device planner's schedule (0: invalid arguments)."""
     return (lib or load()).dan_tree_attn_plan_slots(num_work, groups, num_cus)
@@ -400,14 +375,6 @@ def plan(args, stream, lib=None):
         raise RuntimeError(f"dan_tree_attn_plan failed ({rc}): {last_error(lib)}")
 
 
-def fp8_quantize(args, stream, lib=None):
-    """Launch the e4m3 quantizer; raises RuntimeError with the library's message on failure."""
-    lib = lib or load()
-    rc = lib.dan_fp8_quantize(ctypes.byref(args), _vp(stream))
-    if rc != OK:
-        raise RuntimeError(f"dan_fp8_quantize failed ({rc}): {last_error(lib)}")
-
-
 @functools.lru_cache(maxsize=256)
 def gdn_workspace_size(form, num_tokens, num_runs, num_k_heads, num_v_heads, v_dim):
     """Bytes of workspace one delta rule call needs (0: invalid arguments)."""
@@ -419,33 +386,9 @@ def fp8_tiled_bytes(rows, cols, lib=None):
     return (lib or load()).dan_fp8_tiled_bytes(rows, cols)
 
 
-def fp8_gemm(args, stream, lib=None):
-    """Launch the e4m3 GEMM; raises RuntimeError with the library's message on failure."""
-    lib = lib or load()
-    rc = lib.dan_fp8_gemm(ctypes.byref(args), _vp(stream))
-    if rc != OK:
-        raise RuntimeError(f"dan_fp8_gemm failed ({rc}): {last_error(lib)}")
-
-
-def gdn(args, stream, lib=None):
-    """Launch the gated delta rule; raises RuntimeError with the library's message on failure."""
-    lib = lib or load()
-    rc = lib.dan_gdn_fwd(ctypes.byref(args), _vp(stream))
-    if rc != OK:
-        raise RuntimeError(f"dan_gdn_fwd failed ({rc}): {last_error(lib)}")
-
-
 def gdn_conv(args, stream, lib=None):
     """Launch the conv and gates of one DeltaNet phase; raises RuntimeError with the library's message on failure."""
     lib = lib or load()
     rc = lib.dan_gdn_conv(ctypes.byref(args), _vp(stream))
     if rc != OK:
         raise RuntimeError(f"dan_gdn_conv failed ({rc}): {last_error(lib)}")
-
-
-def gdn_gated_norm(args, stream, lib=None):
-    """Launch the gated RMS norm of a DeltaNet layer; raises RuntimeError with the library's message on failure."""
-    lib = lib or load()
-    rc = lib.dan_gdn_gated_norm(ctypes.byref(args), _vp(stream))
-    if rc != OK:
-        raise RuntimeError(f"dan_gdn_gated_norm failed ({rc}): {last_error(lib)}")

@@ -446,11 +446,9 @@ struct ScanLds {
 // Long runs, where a chunk step's latency sets the pace: 4 waves on 16 state
 // columns (one 16 x 16 tile each), so a (run, head) spreads over 8 work groups.
 // Many short runs, where the per-group fixed cost does: 4 waves on 32 columns
-// (16 x 32 each). Both leave room for two work groups per CU. (The kernel
-// also runs as 8 waves on 32 columns, one tile each, which took 11 % longer on
-// a trunk phase of 5 runs of 286 to 1843 tokens.)
-constexpr int kScanLongWaves = 4, kScanShortWaves = 4;
-
+// (16 x 32 each). Both leave room for two work groups per CU. (Eight waves on
+// 32 columns, one tile each, took 11 % longer on a trunk phase of 5 runs of
+// 286 to 1843 tokens.)
 
 // Contraction orders: the 128-long sums over the state rows take k-index
 // 32 (kk / 8) + 8 q + kk % 8 at step kk in lane group q = lane / 16 (a lane's
@@ -473,24 +471,20 @@ struct Ops {
   float glast;
 };
 
-// Work group: one (run, value head, 32 state columns). Wave w computes rows
+// Work group: one (run, value head, COLS state columns). Wave rb computes rows
 // 16 rb .. 16 rb + 15 of Y, D and O in its NC column halves, and state rows
-// 32 rb .. 32 rb + 31 of those columns: with 8 waves, half nb = w / 4 and
-// rb = w % 4 or 3 - w % 4 (waves w and w + 4 share a SIMD, so every SIMD
-// carries the same share of the triangular products); with 4 waves, rb = w
-// and both halves. Per chunk, with jmax = (L - 1) / 16 the last row block
-// holding run tokens:
+// 32 rb .. 32 rb + 31 of those columns. Per chunk, with jmax = (L - 1) / 16 the
+// last row block holding run tokens:
 //   phase 0  K S and Q S together (one read of S), Y to LDS        barrier
 //   phase 1  D = T Y over row blocks j <= min(rb, jmax) (T is lower
 //            triangular, blocks past jmax are padding), D and Ds to LDS  barrier
 //   phase 2  O = (Q S) + A D (blocks j <= min(rb, jmax)), S <- gamma S + K^T Ds
 //            (blocks j <= jmax) into the other state buffer        barrier
 // A wave whose rows are all padding skips phases 0-1 and the O products.
-template <typename T, int W, int COLS>
-__global__ __launch_bounds__(64 * W) void chunk_scan_kernel(const Params p) {
-  // 16-column halves per wave: 8 waves x 1 (32 columns), 4 x 2 (32), 4 x 1 (16)
-  constexpr int NC = COLS / 16 * 4 / W;
-  static_assert(NC >= 1 && (W == 4 || (W == 8 && COLS == 32)), "scan shapes");
+template <typename T, int COLS>
+__global__ __launch_bounds__(kThreads) void chunk_scan_kernel(const Params p) {
+  constexpr int NC = COLS / 16;  // 16-column halves per wave
+  static_assert(kThreads == 256, "four waves, 16 of a chunk's 64 rows each");
   constexpr int kCols = COLS, kSS = ScanLds<COLS>::kSS, kSB = ScanLds<COLS>::kSB;
   __shared__ __attribute__((aligned(16))) float smem[ScanLds<COLS>::floats];
   // work group b -> (unit u = r Hv + h, column block cb); the ncb groups of a
@@ -500,26 +494,25 @@ __global__ __launch_bounds__(64 * W) void chunk_scan_kernel(const Params p) {
   if (u >= p.units) return;  // the whole group, before any barrier
   const int r = u / p.Hv, h = u % p.Hv, hk = h / (p.Hv / p.Hk);
   const int tid = threadIdx.x, lane = tid & 63, l16 = lane & 15, q4 = lane >> 4;
-  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int nb0 = W == 8 ? w >> 2 : 0, rb = W == 8 ? (nb0 ? 3 - (w & 3) : (w & 3)) : w;
+  const int rb = __builtin_amdgcn_readfirstlane(tid >> 6);
   float *sY = smem + 2 * kDk * kSS, *sD = sY + kC * kSB, *sDs = sD + kC * kSB;
   const int col0 = kCols * cb;
   int col[NC];
 #pragma unroll
-  for (int n = 0; n < NC; ++n) col[n] = 16 * (nb0 + n) + l16;
+  for (int n = 0; n < NC; ++n) col[n] = 16 * n + l16;
   const int64_t sbase = ((int64_t)r * p.Hv + h) * kDk * p.Dv + col0;
   const int64_t sbase_in = ((int64_t)state_in_of(p, r) * p.Hv + h) * kDk * p.Dv + col0;
   {  // the state slice: every load in flight before the first LDS write
-    constexpr int kSt = kDk * kCols / (64 * W);
+    constexpr int kSt = kDk * kCols / kThreads;
     float sv[kSt];
 #pragma unroll
     for (int m = 0; m < kSt; ++m) {
-      const int x = tid + 64 * W * m;
+      const int x = tid + kThreads * m;
       sv[m] = *(const DAN_GLOBAL float *)(p.s_in + sbase_in + (int64_t)(x / kCols) * p.Dv + x % kCols);
     }
 #pragma unroll
     for (int m = 0; m < kSt; ++m) {
-      const int x = tid + 64 * W * m;
+      const int x = tid + kThreads * m;
       smem[(x / kCols) * kSS + x % kCols] = sv[m];
     }
   }
@@ -691,8 +684,8 @@ __global__ __launch_bounds__(64 * W) void chunk_scan_kernel(const Params p) {
   }
   const float *sS = smem + cur * kDk * kSS;
 #pragma unroll
-  for (int m = 0; m < kDk * kCols / (64 * W); ++m) {
-    const int x = tid + 64 * W * m;
+  for (int m = 0; m < kDk * kCols / kThreads; ++m) {
+    const int x = tid + kThreads * m;
     *(DAN_GLOBAL float *)(p.s_out + sbase + (int64_t)(x / kCols) * p.Dv + x % kCols) = sS[(x / kCols) * kSS + x % kCols];
   }
 }
@@ -1094,13 +1087,12 @@ hipError_t dan_gdn_fwd_chunked(const DanGdnArgs *a, float *records, hipStream_t 
   // longer: the long-run scan.
   const bool shortrun = (int64_t)a->num_tokens <= (int64_t)DAN_GDN_SHORT_RUN * a->num_runs;
   const dim3 block(dan_gdnc::kThreads);
-  auto scan = [&](auto kernel, int waves, int cols) {
+  auto scan = [&](auto kernel, int cols) {
     p.ncb = a->v_dim / cols;
     const int64_t groups = ((int64_t)p.units + 7) / 8 * 8 * p.ncb;
-    hipLaunchKernelGGL(kernel, dim3((unsigned)groups), dim3(64 * waves), 0, s, p);
+    hipLaunchKernelGGL(kernel, dim3((unsigned)groups), block, 0, s, p);
   };
-  constexpr int LW = dan_gdnc::kScanLongWaves, LC = dan_gdnc::kLongCols;
-  constexpr int SW = dan_gdnc::kScanShortWaves, SC = dan_gdnc::kShortCols;
+  constexpr int LC = dan_gdnc::kLongCols, SC = dan_gdnc::kShortCols;
   if (a->dtype == DAN_DTYPE_BF16) {
     if (prep) hipLaunchKernelGGL(dan_gdnc::chunk_prep_kernel<__bf16>, dim3((unsigned)prep), block, 0, s, p);
     // v in pieces of 16 bytes (a wider column block's), out in pieces of 8
@@ -1108,16 +1100,16 @@ hipError_t dan_gdn_fwd_chunked(const DanGdnArgs *a, float *records, hipStream_t 
                        a->o_stride_tok % 4 || a->o_stride_head % 4);
     using namespace dan_gdnc;
     if (dan::scan_columns(a->num_runs, a->num_v_heads, a->v_dim, dan::num_cus()) == 16) {
-      if (vec) scan(chunk_scan_bf16_kernel<16, true>, 4, 16);
-      else scan(chunk_scan_bf16_kernel<16, false>, 4, 16);
+      if (vec) scan(chunk_scan_bf16_kernel<16, true>, 16);
+      else scan(chunk_scan_bf16_kernel<16, false>, 16);
     } else {
-      if (vec) scan(chunk_scan_bf16_kernel<32, true>, 4, 32);
-      else scan(chunk_scan_bf16_kernel<32, false>, 4, 32);
+      if (vec) scan(chunk_scan_bf16_kernel<32, true>, 32);
+      else scan(chunk_scan_bf16_kernel<32, false>, 32);
     }
   } else {
     if (prep) hipLaunchKernelGGL(dan_gdnc::chunk_prep_kernel<_Float16>, dim3((unsigned)prep), block, 0, s, p);
-    if (shortrun) scan(dan_gdnc::chunk_scan_kernel<_Float16, SW, SC>, SW, SC);
-    else scan(dan_gdnc::chunk_scan_kernel<_Float16, LW, LC>, LW, LC);
+    if (shortrun) scan(dan_gdnc::chunk_scan_kernel<_Float16, SC>, SC);
+    else scan(dan_gdnc::chunk_scan_kernel<_Float16, LC>, LC);
   }
   return hipGetLastError();
 }
