@@ -56,6 +56,10 @@ STRUCTS = {
     "DanFp8GemmArgs": _native.DanFp8GemmArgs,
     "DanGdnArgs": _native.DanGdnArgs,
     "DanGdnConvArgs": _native.DanGdnConvArgs,
+    "DanGdnNormArgs": _native.DanGdnNormArgs,
+    "DanGdnProjArgs": _native.DanGdnProjArgs,
+    "DanTreeAttnSave": _native.DanTreeAttnSave,
+    "DanStageF16Args": _native.DanStageF16Args,
 }
 
 
@@ -78,6 +82,8 @@ def test_ctypes_layout_matches_header(tmp_path):
                  'DAN_FP8_GEMM_X_SCALE_TENSOR, DAN_FP8_GEMM_W_SCALE_TENSOR, DAN_FP8_GEMM_X_TILED, DAN_FP8_GEMM_W_TILED, '
                  'DAN_FP8_LAYOUT_ROWS, DAN_FP8_LAYOUT_TILED);')
     lines.append('printf("GDN %d\\n", DAN_GDN_ABI_VERSION);')
+    lines.append('printf("INLINE %d,%d,%d,%d\\n", DAN_TREE_ATTN_INLINE_PASTS, DAN_TREE_ATTN_INLINE_SAVES, '
+                 'DAN_QKV_FRONT_INLINE_SAVES, DAN_TREE_ATTN_STAGE_PARTIALS);')
     lines.append("return 0; }")
     src = tmp_path / "probe.c"
     src.write_text("\n".join(lines))
@@ -92,6 +98,8 @@ def test_ctypes_layout_matches_header(tmp_path):
             assert int(got[f"{cname}.{fname}"]) == getattr(cls, fname).offset, f"{cname}.{fname}"
     assert int(got["ABI"]) == _native.ABI_VERSION
     assert int(got["KEY_TILE"]) == _native.KEY_TILE
+    assert got["INLINE"] == f"{_native.INLINE_PASTS},{_native.INLINE_SAVES},{_native.FRONT_INLINE_SAVES},{_native.STAGE_PARTIALS}"
+    assert set(STRUCTS) == {n for n, c in vars(_native).items() if isinstance(c, type) and issubclass(c, ctypes.Structure)}
     assert int(got["SCRATCH"]) == _native.SCRATCH_BYTES
     assert got["PHASES"] == f"{_native.PHASES_ALL},{_native.PHASE_PACK},{_native.PHASE_ATTEND}"
     assert got["FRONT"] == (f"{_native.FRONT_ABI_VERSION},{_native.FRONT_NORM_NONE},{_native.FRONT_NORM_RMS},"

@@ -9,7 +9,12 @@ from dan_amd import _native
 ENTRIES = [(_native.call_forward, _native.DanTreeAttnArgs), (_native.call_forward_noalloc, _native.DanTreeAttnArgs),
            (_native.call_front, _native.DanQkvFrontArgs), (_native.call_fp8_quantize, _native.DanFp8QuantArgs),
            (_native.call_fp8_gemm, _native.DanFp8GemmArgs), (_native.call_gdn, _native.DanGdnArgs),
-           (_native.call_gdn_conv, _native.DanGdnConvArgs), (_native.call_gdn_gated_norm, _native.DanGdnNormArgs)]
+           (_native.call_gdn_conv, _native.DanGdnConvArgs), (_native.call_gdn_gated_norm, _native.DanGdnNormArgs),
+           (_native.call_gdn_project, _native.DanGdnProjArgs)]
+
+
+def test_every_entry_is_listed():
+    assert {e.name for e, _ in ENTRIES} == {e.name for e in vars(_native).values() if isinstance(e, _native.Entry)}
 
 
 @pytest.mark.parametrize("entry,args", ENTRIES, ids=[e.name for e, _ in ENTRIES])
