@@ -1834,6 +1834,8 @@ int dan_tree_attn_fwd(const DanTreeAttnArgs *a, void *stream) {
     return fail(DAN_ERR_UNSUPPORTED, "dtype combination q/k=%d v=%d out=%d is not built", in, vd, out);
   if (a->num_work < 0 || a->num_segments < 0 || a->num_pasts < 0 || a->num_tokens < 0 || a->vt_cols < 0)
     return fail(DAN_ERR_INVALID_ARGUMENT, "negative count");
+  if (a->num_work == 0 && a->num_saves)  // nothing would be launched that writes them
+    return fail(DAN_ERR_INVALID_ARGUMENT, "num_saves %d without work items", a->num_saves);
   if (a->num_work == 0) return DAN_OK;
   if (!a->q || !a->k || !a->v || !a->out || !a->segments || !a->work || !a->key_lo || !a->col_seg)
     return fail(DAN_ERR_INVALID_ARGUMENT, "NULL tensor or table pointer");
@@ -2001,6 +2003,7 @@ int dan_tree_attn_fwd_noalloc(const DanTreeAttnArgs *a, void *stream) {
   if (!a) return fail(DAN_ERR_INVALID_ARGUMENT, "args is NULL");
   if (a->abi_version != DAN_TREE_ATTN_ABI_VERSION)
     return fail(DAN_ERR_VERSION, "abi_version %d, library speaks %d", a->abi_version, DAN_TREE_ATTN_ABI_VERSION);
+  if (a->num_work == 0 && a->num_saves) return fail(DAN_ERR_INVALID_ARGUMENT, "num_saves %d without work items", a->num_saves);
   if (a->num_work == 0) return DAN_OK;
   const int64_t need = dan_tree_attn_workspace_size(a->num_kv_heads, a->head_dim, a->vt_cols);
   if (need > DAN_TREE_ATTN_SCRATCH_BYTES)

@@ -221,7 +221,8 @@ typedef struct {
    * most DAN_TREE_ATTN_INLINE_SAVES, read during the call only; the V^T copy's
    * launch writes rows [start, start + len) of k and of v to each entry's
    * k_dst and v_dst, contiguous and 16-byte aligned: [Hkv][len][D], or
-   * [len][Hkv][D] for k with bit 0 of save_layout and for v with bit 1. */
+   * [len][Hkv][D] for k with bit 0 of save_layout and for v with bit 1.
+   * Without work items (num_work 0) nothing is launched: saves are refused. */
   int32_t num_saves;
   int32_t save_layout;
   const DanTreeAttnSave *saves;

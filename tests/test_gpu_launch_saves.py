@@ -116,7 +116,7 @@ def test_rows_past_the_segment_are_cloned(gpu):
     assert not _launch_saves(k, v, segs)
 
 
-@pytest.mark.parametrize("kw,needle", [(dict(num_saves=9), "num_saves"), (dict(num_saves=-1), "num_saves"), (dict(save_layout=4), "save_layout"), (dict(saves=None), "num_saves"),
+@pytest.mark.parametrize("kw,needle", [(dict(num_saves=9), "num_saves"), (dict(num_saves=-1), "num_saves"), (dict(save_layout=4), "save_layout"), (dict(saves=None), "num_saves"), (dict(num_work=0), "num_saves"),
                                        (dict(in_dtype=_native.DTYPE_E4M3, v_dtype=_native.DTYPE_E4M3, q_scale=4096, k_scale=4096, v_scale=4096), "num_saves"),
                                        (dict(start=90), "save 0"), (dict(len=0), "save 0"), (dict(k_dst=4104), "aligned")])
 def test_argument_errors(kw, needle):
@@ -131,3 +131,5 @@ def test_argument_errors(kw, needle):
     a = _native.DanTreeAttnArgs(**{**base, **{k: x for k, x in kw.items() if k not in entry}})
     assert lib.dan_tree_attn_fwd(ctypes.byref(a), None) == _native.ERR_INVALID_ARGUMENT
     assert needle in _native.last_error(lib)
+    if "num_work" in kw:
+        assert lib.dan_tree_attn_fwd_noalloc(ctypes.byref(a), None) == _native.ERR_INVALID_ARGUMENT
