@@ -457,12 +457,22 @@ def _work_items(segments, n):
     return lambda tile: sum(-(-(s.end - s.start) // tile) for s in segments)
 
 
+def _batch_tile_q(h, hkv, d, n, device, segments):
+    """``_tile_q`` of a batch; a plan of whole tiles that is on it already (made
+    ahead with ``get_plan``) is kept."""
+    plan = getattr(segments, "tile_plan", None)
+    tile_q = _layout(h, hkv, d)[0]
+    if plan is not None and plan.matches(n, tile_q, device):
+        return tile_q
+    return _tile_q(h, hkv, d, n, device, _work_items(segments, n))
+
+
 def workspace_bytes(q, k, segments):
     """Bytes of the V^T workspace of a split ``_attend_fused`` call on this
     batch (the plan is built or found as for the call itself)."""
     h, n, d = q.shape
     hkv = k.shape[0]
-    tile_q, groups = _tile_q(h, hkv, d, n, q.device, _work_items(segments, n)), _layout(h, hkv, d)[1]
+    tile_q, groups = _batch_tile_q(h, hkv, d, n, q.device, segments), _layout(h, hkv, d)[1]
     plan = get_plan(segments, n, tile_q, q.device, groups=groups, num_cus=_num_cus(q.device))
     return _native.workspace_size(hkv, d, plan.vt_cols)
 
@@ -487,7 +497,7 @@ def _call_args(q, k, v, segments, layer, scale, fp8_scales, phases, noalloc, upl
         raise ValueError(f"scale {scale}: the kernel needs a finite positive softmax scale")
     h, n, d = q.shape
     hkv = k.shape[0]
-    tile_q = _tile_q(h, hkv, d, n, q.device, _work_items(segments, n))
+    tile_q = _batch_tile_q(h, hkv, d, n, q.device, segments)
     if tile_q <= 0:
         raise ValueError(f"unsupported head layout H={h}, Hkv={hkv}")
     groups = _layout(h, hkv, d)[1]

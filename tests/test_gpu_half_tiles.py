@@ -131,6 +131,19 @@ def test_segments_make_their_own_units(gpu, lens, want):
     assert (out.float().cpu() - ref).abs().max().item() <= 2e-2
 
 
+@pytest.mark.parametrize("planner", ["host", "device"])
+def test_a_plan_made_ahead_is_kept(gpu, planner):
+    """A small batch planned with whole tiles before layer 0 (get_plan) runs on that plan."""
+    w = build("ahead", [(300, [20, 40])], 32, 8, 128, torch.bfloat16, gpu, np.random.default_rng(3))
+    ref = A.attend(w.q, w.k, w.v, list(w.segments), w.layer)  # a plan of its own: half tiles
+    plan = A.get_plan(w.segments, w.num_tokens, _native.tile_q(32, 8), gpu, planner=planner,
+                      **(dict(groups=8, num_cus=A._num_cus(torch.device(gpu))) if planner == "device" else {}))
+    out = A.attend(w.q, w.k, w.v, w.segments, w.layer)
+    torch.cuda.synchronize()
+    assert w.segments.tile_plan is plan
+    assert (out.float() - ref.float()).abs().max().item() <= 2.0 ** -9 * w.v.float().abs().max().item() + 2.0 ** -7 * ref.float().abs().max().item()
+
+
 @pytest.mark.parametrize("segments,want", [(1, 32), (4, 32), (16, 64)])
 def test_budget_plan_counts_its_capacity(gpu, segments, want):
     """A BudgetPlan takes the form for the most units its capacities allow; its
