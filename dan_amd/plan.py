@@ -251,7 +251,7 @@ class TilePlan:
     past_uploaded: set = field(default_factory=set)  # the layers whose device table was filled by an upload
     past_filled: dict = field(default_factory=dict)  # layer -> (stream, table) of a launch with a caller's workspace that filled it
     schedules: dict = field(default_factory=dict)  # (groups, CUs) -> (units_d, sched_off_d, slots)
-    item_counts: dict = field(default_factory=dict)  # tile -> work items of so many queries
+    tiles: dict = field(default_factory=dict)  # (heads, kv heads, head_dim) -> queries per work item that a call of this layout takes
 
     @classmethod
     def build(cls, segments, num_tokens, tile_q, device):
@@ -309,9 +309,7 @@ class TilePlan:
 
     def items(self, tile):
         """Work items that the segments make with ``tile`` queries each."""
-        if tile not in self.item_counts:
-            self.item_counts[tile] = int((-(-self.segs[:, 1] // tile)).sum())
-        return self.item_counts[tile]
+        return int((-(-self.segs[:, 1] // tile)).sum())
 
     @property
     def vt_cols(self):

@@ -73,7 +73,9 @@ def test_half_tiles_count_every_segments_units(monkeypatch, lens, want):
     n, segs = sum(lens), A.Batch()
     for x in lens:
         segs.append(A.segment(segs[-1].end if segs else 0, [0] * x))
-    tile = lambda: A._tile_q(32, 8, 128, n, "cuda", A._work_items(segs, n))  # noqa: E731
+    tile = lambda: A._batch_tile_q(32, 8, 128, n, "cuda", segs)  # noqa: E731
     assert tile() == want
-    segs.tile_plan = TilePlan.build(segs, n, 64, "cpu")
-    assert tile() == want
+    segs.tile_plan = TilePlan.build(segs, n, 32, "cpu")
+    assert tile() == want and tile() == want
+    segs.tile_plan = TilePlan.build(segs, n, 64, "cpu")  # a plan of whole tiles is kept
+    assert tile() == 64
