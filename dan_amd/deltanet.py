@@ -32,8 +32,10 @@ def _row_ok(t):
 
 # Calls whose longest run has at least this many tokens go through the chunked
 # form (when Dv is a multiple of 32). Measured on gfx950 with 16/16 heads of
-# 128, 45 or 200 runs of L tokens: the token form is faster up to L = 24, the
-# chunked form from L = 32 on (1.1x at 32, 1.6x at 64, 2.3x at 256).
+# 128, 45 or 200 runs of L tokens, token / chunked time: bf16 0.8 at L = 4, 1.05 at 8,
+# 1.5 at 16, 2.4 at 32, 4 to 5 at 64 and 256; fp16 0.95 at 16, 1.1 at 24, 1.4 at 32, 1.9
+# at 64, 2.3 at 256. One line for both types, where the slower scan gains clearly;
+# bf16 phases whose longest run has 16 to 31 tokens would gain, too.
 CHUNK_MIN_RUN = 32
 
 
@@ -180,8 +182,11 @@ def _narrow_pair(x, first, second):
 # Hidden sizes up to which ``_narrow_pair`` launches its own kernel, where 32 rows and
 # 16 columns a work group make at most one group per CU. GPU time of the launch
 # against the two linears', microseconds: hidden 2048, 834 rows x 16 columns 7.2 / 10.5,
-# 834 x 64 7.5 / 10.4, 2779 x 32 9.6 / 11.9, 8192 x 16 9.7 / 16.8; past one group per CU
-# 8192 x 32 17.6 / 17.3; hidden 5120, 834 x 16 15.2 / 12.2.
+# 834 x 64 7.5 / 10.3, 2779 x 32 9.6 / 11.8, 8192 x 16 9.6 / 16.7; past one group per CU
+# 8192 x 32 17.6 / 17.3. bf16, 1 to 8192 rows x 4 to 64 columns (and fp16 at 77, 834 and 8192
+# x 16 and 32): 0.2 to 0.82 of the linears' time at hidden 512 to 2048, 0.4 to 1.0 at 2560,
+# up to 1.06 at 3072 (2779 x 32 13.5 / 12.7), 1.22 at 4096 (17.8 / 14.6), 1.26 at 5120 (834 x 16
+# 15.3 / 12.2).
 NARROW_HIDDEN = 2560
 
 
